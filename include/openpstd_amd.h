@@ -282,15 +282,12 @@ int pstd_ctx_set_stage_overlap(pstd_ctx *ctx, int on);
  * every choice.
  *  - tile order: 1 gives every XCD a contiguous run of tiles (neighbouring
  *    lines share its L2), 0 the plain round-robin order;
- *  - kernel flavour: 0 loads every descriptor-dependent operand (filter,
- *    twiddles, t_n) before the transforms (most registers), 1 loads them
- *    where they are used (fewest registers, most resident waves), 2 loads
- *    filter and twiddles up front and t_n where used;
- *  - tile threads: block size of the kernel for lines of FFT length <= 2048,
- *    128, 256 or 512 (512 puts twice the lines of 256 in a tile: for columns,
- *    twice the contiguous bytes of each row per wave access; 128 spreads a
- *    small scene over more CUs and needs every such line to have F <= 1024,
- *    else PSTD_ERR_INVALID).
+ *  - kernel flavour: 0, 1 or 2, kept for callers of earlier versions and
+ *    reported back: one stage kernel serves all three;
+ *  - tile threads: block size of the stage kernel, 128, 256 or 512 (128 spreads
+ *    a small scene over more CUs and needs every line of the F <= 2048 class to
+ *    have F <= 1024, else PSTD_ERR_INVALID); lines of FFT length 4096 and 8192
+ *    take blocks of at least 256 and 512 whatever is set.
  * The choice is kept per (device, plan signature: form, scenes, every tile's
  * line class, line count and direction): a later upload of a plan with the
  * same signature on the same device takes it without trials.

@@ -5,15 +5,20 @@
 // kernel/Solver.cpp:153-160).
 //
 // State per domain lives in four arenas with identical layout (fields vx, vy,
-// px, py row-major at per-domain offsets):
+// px, py at per-domain offsets):
 //   TN  - values at t_n after PML attenuation (openPSTD's previous_values)
 //   S0, S1 - raw outputs of the RK stages (ping-pong)
-//   P0I - an explicit p0 (initial state / host-written p0)
-// p0 is never stored between stages: openPSTD recomputes p0 = px0 + py0 after
-// every stage (kernel/Solver.cpp:114-116), so the derivative kernels form it on
-// the fly from the stage outputs.  The first stage of a step reads p0 from the
-// raw stage-5 outputs of the previous step, which is openPSTD's p0 left stale
-// by the PML attenuation (kernel/Solver.cpp:85).
+//   P0I - p0 (px slot) and its transpose (py slot): an explicit p0 (initial
+//         state / host-written p0), and with `p0_pass` every stage's p0
+// vx and px, which only X lines derive and update, are stored row-major; vy and
+// py, which only Y lines do, column-major (transposed).  Every line of both
+// directions is then contiguous in the field it derives, in t_n and in its
+// output; only p0 = px + py (kernel/Solver.cpp:114-116) brings the two layouts
+// together.  Large scenes form it in a pass of its own after every stage
+// (p0_pass_kernel, both layouts); small ones, where a further launch costs more
+// than it saves, add the other layout's field on the fly, strided.  The first
+// stage of a step reads p0 from the raw stage-5 outputs of the previous step,
+// which is openPSTD's p0 left stale by the PML attenuation (kernel/Solver.cpp:85).
 //
 // One RK stage = one launch of the fused line kernel: for each line of each
 // segment it gathers the windowed line (spatderp3, kernel/core/
@@ -43,19 +48,18 @@
 using namespace pstdamd::dev;
 
 // Scratch of the allocation-free advance (pstd_ctx_advance_static): the
-// GEMM form's per-scene maxima, 3 slots x 2 classes x kStaticScenes scenes
-// (24 KiB), one copy per device (each device has its own address, resolved
+// GEMM form's per-scene maxima, 2 classes x kStaticScenes scenes (8 KiB), one copy per device (each device has its own address, resolved
 // with hipGetSymbolAddress), shared by every call on that device.
 constexpr int kStaticScenes = 1024;
-static __device__ __align__(256) unsigned scratch[3 * 2 * kStaticScenes];
+static __device__ __align__(256) unsigned scratch[2 * kStaticScenes];
 
 namespace {
 
 constexpr int kPassChunk = 2048;    // elements per passthrough tile
 constexpr int kMaxDomainFloats = 1 << 29;  // one domain block (4 fields) per buffer resource
 
-// A domain's four fields (vx, vy, px, py, row-major) form one block at the same
-// offset of every arena (TN, S0, S1, P0I and the PML factors).
+// A domain's four fields (vx, px row-major, vy, py column-major) form one block
+// at the same offset of every arena (TN, S0, S1, P0I and the PML factors).
 struct DomainDev {
     int nx, ny;
     long long base;                 // element offset of the block in an arena
@@ -65,36 +69,45 @@ struct DomainDev {
     int is_pml;
 };
 
-// One work item of a stage launch; everything a workgroup needs in one
-// scalar-loadable record.
-//  kind 0: derivative tile — `count` lines of a segment (Domain::calc,
-//          kernel/core/Domain.cpp:149-370): gather, derivative, update.
-//  kind 1: passthrough — elements [line0, line0+count) of one field that no
-//          segment updates (rigid domains, directions openPSTD skips).
+// A line segment of a domain (Domain::calc, kernel/core/Domain.cpp:149-370) with
+// everything a workgroup needs in one scalar-loadable record, shared by all of
+// the segment's tiles.
+//  kind 0: derivative lines: gather, derivative, update.
+//  kind 1: passthrough: a field that no segment updates (rigid domains,
+//          directions openPSTD skips); lines are elements.
 //  kind 2: receiver sampling (first stage of a step).
 //  kind 3: the segment addressing of a GEMM-form tile (GemmTile::t).
 // Memory is addressed through buffer resources over one domain block (base
 // `*_dom`, `*_size` elements): value (line, pos) of a source field is element
-// a + line*ls + pos*ps of the block (+ element b of the second array for
-// p0 = px0 + py0).  Offsets past the block read 0 and drop stores, which is how
-// absent neighbours, the zero padding and partial tiles are expressed.
+// a + line*ls + pos of the block; where p0 = px + py is formed on the fly, plus
+// element b + line + pos*bp (the field of the other layout).  Offsets past the
+// block read 0 and drop stores, which is how absent neighbours, the zero padding
+// and partial tiles are expressed.
 struct TileDesc {
     int kind;
     int F;
     int line0, count;
     int wlen, wlog, n_main, n_out, vel, dir;  // wlog: log2 of the halo slot (2^wlog >= wlen)
     int h_off, tw_off, win_off;
-    int tw2_off;  // F = 8192: the 4096-point twiddle table (its two halves run as 4096-point transforms)
     long long m_dom, s1_dom, s2_dom;
     int m_size, s1_size, s2_size;
-    int m_a, m_b, m_ls, m_ps;
-    int s1_a, s1_b, s1_ls, s1_ps, s1_line, s1_len;  // s1_len < 0: no neighbour (zeros)
-    int s2_a, s2_b, s2_ls, s2_ps, s2_line, s2_len;
+    int m_a, m_b, m_ls, m_bp;
+    int s1_a, s1_b, s1_ls, s1_bp, s1_line, s1_len;  // s1_len < 0: no neighbour (zeros)
+    int s2_a, s2_b, s2_ls, s2_bp, s2_line, s2_len;
     float c_s1, c_m1, c_s2, c_m2;
-    int o_f, o_ls, o_ps;  // output field (vx, px, vy or py) within the main block
+    int o_f, o_ls;        // output field (vx, px, vy or py) within the main block
     float coef;           // 1/rho (velocity update) or rho*c1^2 (pressure update)
     int is_pml;
     int scene;            // scene of the batch (per-scene maxima of the GEMM form's scaling)
+};
+
+// One workgroup of a stage launch: `count` lines of a segment from line0 on.  16
+// bytes: neighbouring workgroups share a cache line, and the segments they name
+// stay in the caches (a whole descriptor per workgroup came from memory before
+// anything else could start).
+struct TileRef {
+    int seg, line0, count;
+    int slot;  // GEMM form: of the first wavefront's maximum
 };
 
 struct ReceiverCell {
@@ -102,11 +115,12 @@ struct ReceiverCell {
 };
 
 struct StageArgs {
-    const TileDesc *__restrict__ tiles;
+    const TileRef *tiles;
+    const TileDesc *segs;
     const float2 *ctab;
     const float *ftab;
-    const float *p0a;  // p0 = p0a[...] + (p0b ? p0b[...] : 0)
-    const float *p0b;
+    const float *p0;   // p0 arena: P0I, or (p0_two) a stage arena whose px + py it is
+    int p0_two;
     const float *vsrc; // current vx / vy
     float *tn;
     float *out;
@@ -120,10 +134,10 @@ struct StageArgs {
     float *samples;    // samples[slot * nrec + r], slot < 0: no sampling in this launch
     int slot;
     int remap;         // XCD-contiguous tile order (tile_index)
-    // GEMM form (umax == nullptr otherwise): per-scene maxima of the written
-    // values in three rotating slots (write slot_w, read slot_r, clear slot_z)
-    unsigned *umax;
-    int slot_w, slot_r, slot_z, n_scenes;
+    // GEMM form (wmax == nullptr otherwise): the largest |value| each wavefront
+    // wrote, and what the previous stage's came to per scene (max_reduce)
+    float *wmax;
+    const unsigned *umax;
     const void *dmat;  // derivative matrices (2-byte elements)
 };
 
@@ -136,710 +150,348 @@ __device__ __forceinline__ Rsrc block_rsrc(const float *arena, long long dom, in
     // raw buffer (stride 0) over `size` floats; word 3 as for every gfx9 raw buffer
     return __builtin_amdgcn_make_buffer_rsrc((void *)(arena + dom), (short)0, size * 4, 0x00020000);
 }
-__device__ __forceinline__ float bload(Rsrc r, int off_bytes) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off_bytes, 0, 0));
+// per-lane byte offset, and a uniform one that the block's bounds need not know
+// (kLead floats of padding cover what it adds)
+__device__ __forceinline__ float bload(Rsrc r, int off_bytes, int uniform = 0) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off_bytes, uniform, 0));
 }
-__device__ __forceinline__ void bstore(Rsrc r, int off_bytes, float v) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off_bytes, 0, 0);
+__device__ __forceinline__ void bstore(Rsrc r, int off_bytes, int uniform, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off_bytes, uniform, 0);
+}
+// A block with the 32 floats before it: positions a halo length before a line's
+// first value have non-negative offsets (they read the values before the line,
+// which every user replaces).  kLead floats precede the first block of an arena and
+// follow the last one: a row of threads that begins inside a line may end up to
+// 512 floats past it.
+constexpr int kLead = 576, kShift = 32;
+__device__ __forceinline__ Rsrc lead_rsrc(const float *arena, long long dom, int size) {
+    return block_rsrc(arena, dom - kShift, size + kShift);
+}
+// A uniform value anew: what is computed or loaded from it is computed again
+// rather than kept in registers.
+__device__ __forceinline__ int again(int x) {
+    asm volatile("" : "+v"(x));
+    return __builtin_amdgcn_readfirstlane(x);
 }
 // two adjacent floats (4-byte aligned suffices for buffer accesses)
 __device__ __forceinline__ float2 bload2(Rsrc r, int off_bytes) {
     return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, off_bytes, 0, 0));
 }
-__device__ __forceinline__ void bstore2(Rsrc r, int off_bytes, float x, float y) {
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, make_float2(x, y)), r, off_bytes, 0, 0);
+
+// The GEMM form scales its operands by the largest |value| of a scene's pressure
+// (class 0) and velocity fields (class 1) after a stage.  Every wavefront stores
+// the largest value it wrote into a slot of its own, and max_reduce brings the
+// slots of a scene and class, which lie together, to umax[scene * 2 + class]
+// (float bits).  (With atomic maxima into the scene's word the strips' tiles of 16
+// scenes took 200 us in the GEMM form, against 100 without them.)
+__device__ __forceinline__ void track_max(const StageArgs &a, int slot, float m) {
+    if (!a.wmax) return;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) a.wmax[slot + (threadIdx.x >> 6)] = m;
 }
 
-// Geometry of a derivative tile: F-point lines (run time), NT threads,
-// T = F/8 threads per line pair, P = NT/T pairs; LAYOUT (compile time) 0: X
-// lines (rows; lanes walk positions), 1: Y lines (columns; lanes walk the
-// pairs).  The gather and update code is shared by all F (one copy per
-// layout keeps the kernel small enough for the instruction cache); only the
-// transforms are specialised per F.
-template <int LAYOUT>
-struct TileGeo {
-    int F, T, P, logT, logP;
-    __device__ TileGeo(int F_, int NT) : F(F_), T(F_ >> 3), P(NT / (F_ >> 3)) {
-        logT = __ffs(T) - 1;
-        logP = __ffs(P) - 1;
-    }
-    __device__ int pair(int tid) const { return LAYOUT == 0 ? tid >> logT : tid & (P - 1); }
-    __device__ int lane_t(int tid) const { return LAYOUT == 0 ? tid & (T - 1) : tid >> logP; }
-    // raw staging of the 2P lines in LDS (float): line-major for rows,
-    // position-major for columns, so that the wavefront's lanes stay contiguous.
-    // Rows use a pitch of 9F/8 floats: the two lines of pair p then fill exactly
-    // the slots pair p's transform uses in the second buffer (its own, so the
-    // transforms of rows need no workgroup barrier after the staging)
-    __device__ int line_base(int ll) const { return LAYOUT == 0 ? (ll << (logT + 3)) + (ll << logT) : ll; }
-    __device__ int pos_step() const { return LAYOUT == 0 ? 1 : 2 * P; }
-    __device__ int stage_at(int ll, int pos) const { return line_base(ll) + pos * pos_step(); }
+// The derivative's input arena.  (Chosen between values: a conditional of two
+// struct members is one of their addresses, and keeps the struct in memory.)
+__device__ __forceinline__ const float *pick(bool c, const float *x, const float *y) { return c ? x : y; }
+__device__ __forceinline__ const float *source(const StageArgs &a, int vel) { return pick(vel != 0, a.vsrc, a.p0); }
+
+// Descriptors are read through the constant address space: by scalar loads,
+// wherever they are needed, also after stores.
+typedef const __attribute__((address_space(4))) TileDesc *Seg;
+typedef const __attribute__((address_space(4))) TileRef *Ref;
+
+// A derivative tile: F-point lines, T = F/V threads per line pair; thread (p, t)
+// holds the values at positions t + m*T (m = 0..V-1) of lines 2p and 2p+1 as one
+// complex sequence (V: fft_line.h).  The code before and after the transforms is
+// shared by all F of one V (few copies keep the kernel inside the instruction
+// cache), the transforms are specialised.
+//
+// gather: the windowed lines (spatderp3, kernel/core/kernel_functions.cpp:210-216
+// pressure, :263-269 velocity) [dom1 | main | dom3 | 0], where dom1[j] =
+// (side1[tail + j] * c_s1 + main[reflected] * c_m1) * window[j] and dom3 likewise.
+// Main values are loaded where they are transformed, a wavefront along the line;
+// positions outside the main piece read whatever lies beside the line and are
+// replaced.  The 2w halo values are formed where they are transformed too: each
+// of T >= 32 threads holds at most one of a side's w <= 32 positions (the 16
+// threads of a 128-point pair, SHORT: two), and loads its side value, its
+// reflected main value (the line itself, a cache hit) and its window coefficient
+// directly.  All loads are issued before the first
+// wait, and no LDS staging or barrier precedes the transform.
+//
+// With p0_two, p0 = px + py is formed on the fly.  Across the other layout a line
+// is strided and the tile's lines are adjacent: the workgroup reads position
+// after position, all of the tile's lines at once (32 bytes of 8 lines; a thread
+// reading its own pair touches 8 bytes per cache sector, which made up a quarter
+// of the time of a 333 000-cell scene), and turns them through the pairs' LDS
+// buffers.
+struct Tile {
+    int T, logT, p, t;  // threads per pair; this thread's pair and position
+    int pitch;          // of the pairs' LDS buffers
+    int line, count;    // first line of the pair; lines of the pair inside the tile (0, 1, 2 or more)
+    // thread rows that positions [0, n) reach into
+    __device__ __forceinline__ int rows(int n) const { return (n + T - 1) >> logT; }
 };
 
-// The windowed lines of one tile (spatderp3, kernel/core/kernel_functions.cpp:
-// 210-216 pressure, :263-269 velocity):  [dom1 | main | dom3 | 0], where
-// dom1[j] = (side1[tail + j] * c_s1 + main[reflected] * c_m1) * window[j] and
-// dom3 likewise.  Thread (p, t) loads the main values it will transform
-// (positions t + m*T of lines 2p and 2p+1); the 2 x w halo values of every
-// line are loaded by the tile's threads in turn; both go to LDS so that halo
-// positions can combine them with the reflected main values.  All loads are
-// issued before the first wait.
-struct GatherRegs {
-    float ra[8][2], rb[8][2];
-    float h1a[4], h1b[4], h2a[4], h2b[4];
-    int hpos1[4], hpos2[4];
-    float win;  // window coefficient threadIdx.x (threads 0..2w)
-};
+// A line fills more than half of its F points (F is the next power of two), less
+// 32 of the halo: rows of threads that lie inside it for sure.
+template <int V, bool SHORT>
+constexpr int kFull = SHORT ? 2 : V / 2 - 1;
 
-template <int NT, int LAYOUT>
-__device__ __forceinline__ void gather_issue(const StageArgs &a, const TileDesc &td, const TileGeo<LAYOUT> &g, int p,
-                                             int t, GatherRegs &R) {
-    const int w = td.wlen, nm = td.n_main, vel = td.vel, count = td.count;
+template <int V, int NT, bool SHORT>
+__device__ __forceinline__ void gather(const StageArgs &a, Seg td, const Tile &x, float2 *lds, float2 (&v)[V]) {
+    constexpr int NI = SHORT ? 2 : 1, FULL = kFull<V, SHORT>;
+    const int w = td->wlen, nm = td->n_main, vel = td->vel, end = w + nm, T = x.T, t = x.t, T4 = T * 4;
     __builtin_assume(w > 0 && w <= 32);
-    // the window, with the lines (not after them: one memory latency less)
-    R.win = (int)threadIdx.x <= 2 * w ? a.ftab[td.win_off + threadIdx.x] : 0.f;
-    const float *A = vel ? a.vsrc : a.p0a;
-    const bool hasB = !vel && a.p0b != nullptr;
-    const float *B = hasB ? a.p0b : A;
-    // resources: main, side1, side2 blocks; B shifted so that A's offsets address it
-    const Rsrc rmA = block_rsrc(A, td.m_dom, td.m_size);
-    const Rsrc rmB = block_rsrc(B, td.m_dom + (td.m_b - td.m_a), td.m_size - (td.m_b - td.m_a));
-    const int la = td.line0 + 2 * p;
-    const int pstep = td.m_ps * 4;
-    const int lbase = (td.m_a + la * td.m_ls) * 4 + (t - w) * pstep, lstep = td.m_ls * 4, mstep = g.T * pstep;
-    int off[8][2];
+    const int rows = x.rows(end);
+    const float *A = source(a, vel);
+    const Rsrc rm = lead_rsrc(A, td->m_dom, td->m_size);
+    const bool ok0 = x.count > 0, ok1 = x.count > 1;
+    const int ls4 = td->m_ls * 4;
+    const int row = (td->m_a + x.line * td->m_ls + kShift) * 4;  // the line's first main value
+    const int off0 = ok0 ? row + (t - w) * 4 : kOOB, off1 = ok1 ? row + ls4 + (t - w) * 4 : kOOB;
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const int e = t + m * g.T - w;
-        const bool ok = e >= 0 && e < nm;
-        off[m][0] = ok && 2 * p < count ? lbase + m * mstep : kOOB;
-        off[m][1] = ok && 2 * p + 1 < count ? lbase + lstep + m * mstep : kOOB;
+    for (int m = 0; m < V; ++m) {
+        v[m] = make_float2(0.f, 0.f);
+        if (m < FULL || m < rows) v[m] = make_float2(bload(rm, off0, m * T4), bload(rm, off1, m * T4));
     }
-    if constexpr (LAYOUT == 1) {
-        // Columns: lines 2p and 2p+1 are adjacent floats (line stride 1), one
-        // 8-byte load fetches both.  An odd last line of a tile reads the float
-        // after its partner (inside the block: every domain block ends with a
-        // spare float); gather_finish drops it.
+    // halo item c of this thread: left position t + cT, right offset j0 + cT
+    const int col = end & (T - 1), j0 = (t - col) & (T - 1);
+    const Rsrc r1 = block_rsrc(A, td->s1_dom, td->s1_size), r2 = block_rsrc(A, td->s2_dom, td->s2_size);
+    const int s1 = td->s1_len - w - vel, l1 = x.line + td->s1_line, l2 = x.line + td->s2_line;
+    const bool has1 = ok0 && td->s1_len >= 0, has2 = ok0 && td->s2_len >= 0;
+    float2 ls[NI], rs[NI], lr[NI], rr[NI];
+    float lw[NI], rw[NI];
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            const float2 x = bload2(rmA, off[m][0]);
-            R.ra[m][0] = x.x;
-            R.ra[m][1] = x.y;
-            const float2 y = hasB ? bload2(rmB, off[m][0]) : make_float2(0.f, 0.f);
-            R.rb[m][0] = y.x;
-            R.rb[m][1] = y.y;
-        }
-    } else if (hasB) {
-#pragma unroll
-        for (int m = 0; m < 8; ++m)
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                R.ra[m][q] = bload(rmA, off[m][q]);
-                R.rb[m][q] = bload(rmB, off[m][q]);
-            }
-    } else {
-#pragma unroll
-        for (int m = 0; m < 8; ++m)
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                R.ra[m][q] = bload(rmA, off[m][q]);
-                R.rb[m][q] = 0.f;
-            }
+    for (int c = 0; c < NI; ++c) {
+        const int i = t + c * T, j = j0 + c * T;
+        const bool li = i < w, ri = j < w;
+        lw[c] = a.ftab[td->win_off + (li ? i : 0)];
+        rw[c] = a.ftab[td->win_off + w + 1 + (ri ? j : 0)];
+        const int o1 = li && has1 ? (td->s1_a + l1 * td->s1_ls + s1 + i) * 4 : kOOB;
+        const int o2 = ri && has2 ? (td->s2_a + l2 * td->s2_ls + j + vel) * 4 : kOOB;
+        const int ol = li && ok0 ? row + (w - 1 + vel - i) * 4 : kOOB, orr = ri && ok0 ? row + (nm - 1 - vel - j) * 4 : kOOB;
+        ls[c] = make_float2(bload(r1, o1), bload(r1, ok1 ? o1 + td->s1_ls * 4 : kOOB));
+        rs[c] = make_float2(bload(r2, o2), bload(r2, ok1 ? o2 + td->s2_ls * 4 : kOOB));
+        lr[c] = make_float2(bload(rm, ol), bload(rm, ok1 ? ol + ls4 : kOOB));
+        rr[c] = make_float2(bload(rm, orr), bload(rm, ok1 ? orr + ls4 : kOOB));
     }
-    // halos: item i of a side is (line ll, offset j), j in slots of 2^wlog >= w;
-    // rows: j fastest, columns: ll fastest (coalesced either way)
-    const Rsrc r1A = block_rsrc(A, td.s1_dom, td.s1_size);
-    const Rsrc r1B = block_rsrc(B, td.s1_dom + (td.s1_b - td.s1_a), td.s1_size - (td.s1_b - td.s1_a));
-    const Rsrc r2A = block_rsrc(A, td.s2_dom, td.s2_size);
-    const Rsrc r2B = block_rsrc(B, td.s2_dom + (td.s2_b - td.s2_a), td.s2_size - (td.s2_b - td.s2_a));
-    if constexpr (LAYOUT == 1) {
-        // columns: item i is (pair pp, offset j), both lines of the pair (adjacent
-        // floats) in one 8-byte load into registers 2k, 2k+1 (at most 2 items per
-        // thread: P 2^wlog <= 2 NT); gather_finish drops a lone last line's value
-        const int n_items = g.P << td.wlog;
-        const int nk = (n_items + NT - 1) / NT;
+    if (!vel && a.p0_two) {
+        const unsigned keep = ok1 ? ~0u : 0u;  // a lone last line's partner stays zero
+        auto add = [&](float2 &u, float2 y) __attribute__((always_inline)) {
+            u.x += y.x;
+            u.y += __uint_as_float(__float_as_uint(y.y) & keep);
+        };
+        const int logP = __builtin_ctz(NT) - x.logT, P = 1 << logP, bp4 = td->m_bp * 4;
+        // item (pair, position) = (i mod P, i / P), i = thread + k NT
+        const int pair = threadIdx.x & (P - 1), pos = threadIdx.x >> logP, step = NT >> logP;
+        const int lines = x.count + 2 * x.p - 2 * pair, b0 = (td->m_b + x.line - 2 * x.p + 2 * pair + kShift) * 4;
+        float2 b[V];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            R.hpos1[k] = R.hpos2[k] = -1;
-            R.h1a[k] = R.h1b[k] = R.h2a[k] = R.h2b[k] = 0.f;
+        for (int k = 0; k < V; ++k)
+            if (k == 0 || k * step < nm)
+                b[k] = bload2(rm, lines > 0 && pos + k * step < nm ? b0 + (pos + k * step) * bp4 : kOOB);
+        float2 y1[NI], y2[NI];
+#pragma unroll
+        for (int c = 0; c < NI; ++c) {
+            y1[c] = bload2(r1, t + c * T < w && has1 ? (td->s1_b + l1 + (s1 + t + c * T) * td->s1_bp) * 4 : kOOB);
+            y2[c] = bload2(r2, j0 + c * T < w && has2 ? (td->s2_b + l2 + (j0 + c * T) * td->s2_bp) * 4 : kOOB);
         }
+        float2 *to = lds + pair * x.pitch;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if (k < nk) {
-                const int i = threadIdx.x + k * NT;
-                const int pp = i & (g.P - 1), j = i >> g.logP;
-                const bool item = i < n_items && j < w;
-                const bool ok = item && 2 * pp < count;
-                const int line = td.line0 + 2 * pp;
-                const int o1 = ok && td.s1_len >= 0
-                                   ? (td.s1_a + (line + td.s1_line) * td.s1_ls + (td.s1_len - w - vel + j) * td.s1_ps) * 4
-                                   : kOOB;
-                const int o2 = ok && td.s2_len >= 0 ? (td.s2_a + (line + td.s2_line) * td.s2_ls + (j + vel) * td.s2_ps) * 4
-                                                    : kOOB;
-                const float2 x1 = bload2(r1A, o1), x2 = bload2(r2A, o2);
-                R.h1a[2 * k] = x1.x;
-                R.h1a[2 * k + 1] = x1.y;
-                R.h2a[2 * k] = x2.x;
-                R.h2a[2 * k + 1] = x2.y;
-                if (hasB) {
-                    const float2 y1 = bload2(r1B, o1), y2 = bload2(r2B, o2);
-                    R.h1b[2 * k] = y1.x;
-                    R.h1b[2 * k + 1] = y1.y;
-                    R.h2b[2 * k] = y2.x;
-                    R.h2b[2 * k + 1] = y2.y;
-                }
-                R.hpos1[k] = item ? g.stage_at(2 * pp, j) : -1;
-                R.hpos2[k] = item ? g.stage_at(2 * pp, w + nm + j) : -1;
-            }
-        }
-    } else {
-        const int n_items = (2 * g.P) << td.wlog;
-        const int nk = (n_items + NT - 1) / NT;
+        for (int k = 0; k < V; ++k)
+            if ((k == 0 || k * step < nm) && pos + k * step < nm) to[lds_slot(w + pos + k * step)] = b[k];
+        __syncthreads();
+        const float2 *buf = lds + x.p * x.pitch;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            R.hpos1[k] = R.hpos2[k] = -1;
-            R.h1a[k] = R.h1b[k] = R.h2a[k] = R.h2b[k] = 0.f;
-            if (k < nk) {
-                const int i = threadIdx.x + k * NT;
-                const int ll = i >> td.wlog;
-                const int j = i & ((1 << td.wlog) - 1);
-                const bool item = i < n_items && j < w;
-                const bool ok = item && ll < count;
-                const int line = td.line0 + ll;
-                const int o1 = ok && td.s1_len >= 0
-                                   ? (td.s1_a + (line + td.s1_line) * td.s1_ls + (td.s1_len - w - vel + j) * td.s1_ps) * 4
-                                   : kOOB;
-                const int o2 = ok && td.s2_len >= 0 ? (td.s2_a + (line + td.s2_line) * td.s2_ls + (j + vel) * td.s2_ps) * 4
-                                                    : kOOB;
-                R.h1a[k] = bload(r1A, o1);
-                R.h2a[k] = bload(r2A, o2);
-                if (hasB) {
-                    R.h1b[k] = bload(r1B, o1);
-                    R.h2b[k] = bload(r2B, o2);
-                }
-                R.hpos1[k] = item ? g.stage_at(ll, j) : -1;
-                R.hpos2[k] = item ? g.stage_at(ll, w + nm + j) : -1;
-            }
+        for (int m = 0; m < V; ++m)
+            if (m < FULL || m < rows) add(v[m], buf[lds_slot(t + m * T)]);
+#pragma unroll
+        for (int c = 0; c < NI; ++c) {
+            const int i = t + c * T, j = j0 + c * T;
+            add(ls[c], y1[c]);
+            add(rs[c], y2[c]);
+            if (i < w) add(lr[c], buf[lds_slot(2 * w - 1 - i)]);
+            if (j < w) add(rr[c], buf[lds_slot(end - 1 - j)]);
         }
     }
+    float2 hr[NI];
+#pragma unroll
+    for (int c = 0; c < NI; ++c) {
+        const float2 hl = make_float2(__builtin_fmaf(ls[c].x, td->c_s1, lr[c].x * td->c_m1) * lw[c],
+                                      __builtin_fmaf(ls[c].y, td->c_s1, lr[c].y * td->c_m1) * lw[c]);
+        hr[c] = make_float2(__builtin_fmaf(rs[c].x, td->c_s2, rr[c].x * td->c_m2) * rw[c],
+                            __builtin_fmaf(rs[c].y, td->c_s2, rr[c].y * td->c_m2) * rw[c]);
+        if (j0 + c * T >= w) hr[c] = make_float2(0.f, 0.f);
+        if (t + c * T < w) v[c] = hl;
+    }
+    // thread row lo + c holds right item c from column `col` on, item c - 1 before it
+    const int lo = end >> x.logT;
+    const bool at_end = t >= col;
+#pragma unroll
+    for (int m = FULL; m < V; ++m)
+#pragma unroll
+        for (int c = 0; c <= NI; ++c)
+            if (m == lo + c) {
+                const float2 from = c < NI ? hr[c < NI ? c : 0] : make_float2(0.f, 0.f);
+                v[m] = at_end ? from : c == 0 ? v[m] : hr[c > 0 ? c - 1 : 0];
+            }
 }
-
-// Stages the raw values, then builds the windowed complex pairs.
-template <int LAYOUT>
-__device__ __forceinline__ void gather_finish(const StageArgs &a, const TileDesc &td, const TileGeo<LAYOUT> &g, int p,
-                                              int t, const GatherRegs &R, float *stage, float *win, float2 (&v)[8]) {
-    const int w = td.wlen, nm = td.n_main, vel = td.vel;
-    __builtin_assume(w > 0 && w <= 32);
-    const float c_s1 = td.c_s1, c_m1 = td.c_m1, c_s2 = td.c_s2, c_m2 = td.c_m2;
-    // LDS addresses: line q of the pair at position pos = lb[q] + pos * ps
-    const int ps = g.pos_step(), lb[2] = {g.line_base(2 * p), g.line_base(2 * p + 1)};
-    const int tps = t * ps, mps = g.T * ps;
-    const bool ok1 = LAYOUT == 0 || 2 * p + 1 < td.count;
-    float raw[8][2];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const int pos = t + m * g.T;
-        const bool mid = pos >= w && pos < w + nm;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            raw[m][q] = q == 0 || ok1 ? R.ra[m][q] + R.rb[m][q] : 0.f;
-            if (mid) stage[lb[q] + tps + m * mps] = raw[m][q];
-        }
-    }
-    if constexpr (LAYOUT == 1) {
-        // a pair's two halo values are adjacent in the staging (stage_at(2pp, j) even)
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if (R.hpos1[k] >= 0) {
-                const bool two = (R.hpos1[k] & (2 * g.P - 1)) + 1 < td.count;
-                *reinterpret_cast<float2 *>(&stage[R.hpos1[k]]) =
-                    make_float2(R.h1a[2 * k] + R.h1b[2 * k], two ? R.h1a[2 * k + 1] + R.h1b[2 * k + 1] : 0.f);
-                *reinterpret_cast<float2 *>(&stage[R.hpos2[k]]) =
-                    make_float2(R.h2a[2 * k] + R.h2b[2 * k], two ? R.h2a[2 * k + 1] + R.h2b[2 * k + 1] : 0.f);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (R.hpos1[k] >= 0) {
-                stage[R.hpos1[k]] = R.h1a[k] + R.h1b[k];
-                stage[R.hpos2[k]] = R.h2a[k] + R.h2b[k];
-            }
-        }
-    }
-    if ((int)threadIdx.x <= 2 * w) win[threadIdx.x] = R.win;
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const int i = t + m * g.T;
-        const bool left = i < w, right = i >= w + nm && i < 2 * w + nm, mid = i >= w && i < w + nm;
-        const int j = i - w - nm;
-        float out[2] = {0.f, 0.f};
-        if (left || right) {
-            const int mpos = left ? (vel ? w - i : w - 1 - i) : (vel ? nm - 2 - j : nm - 1 - j);
-            const float cs = left ? c_s1 : c_s2, cm = left ? c_m1 : c_m2;
-            const float wv = win[left ? i : w + 1 + j];
-            const int ri = (w + mpos) * ps, si = tps + m * mps;
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const float sv = stage[lb[q] + si];
-                const float refl = stage[lb[q] + ri];
-                out[q] = __builtin_fmaf(sv, cs, refl * cm) * wv;
-            }
-        }
-        v[m] = make_float2(mid ? raw[m][0] : out[0], mid ? raw[m][1] : out[1]);
-    }
-}
-
-// Forward transform, spectral derivative (the Hermitian filter h, which carries
-// the 1/F of kernel/core/kernel_functions.cpp:243,306), inverse transform.
-// LEAN: the filter and the twiddles are read from the tables (hsrc, tw) during
-// the transforms instead of the registers preloaded by the caller (h, twr).
-template <int F, int NT, int LAYOUT, bool LEAN>
-__device__ __forceinline__ void derivative_fft(float2 (&v)[8], float2 (&h)[8], const float2 *twr, float2 *buf0,
-                                               float2 *buf1, const float2 *hsrc, const float2 *tw) {
-    constexpr int T = F / 8, P = NT / T;
-    // (p, t) again from the thread index, with F known here
-    const int tid = threadIdx.x;
-    const int p = LAYOUT == 0 ? tid / T : tid % P, t = LAYOUT == 0 ? tid % T : tid / P;
-    if constexpr (LEAN) {
-        // filter and twiddles are loaded while the forward transform runs, the
-        // twiddles one pass ahead (fft_run_ahead)
-#pragma unroll
-        for (int m = 0; m < 8; ++m) h[m] = hsrc[t + m * (F / 8)];
-        const float2 w0[kTwPass] = {};
-        fft_run_ahead<F, P, LAYOUT, false>(v, p, t, buf0, buf1, tw, w0);
-    } else {
-        fft_run<F, P, LAYOUT, false, false>(v, p, t, buf0, buf1, twr);
-    }
-#pragma unroll
-    for (int m = 0; m < 8; ++m) v[m] = cmul(v[m], h[m]);
-    // the inverse's first pass overwrites what the forward's last exchange read
-    pass_sync<F, LAYOUT, true, 0>();
-    if constexpr (LEAN) {
-        const float2 w0[kTwPass] = {};
-        fft_run_ahead<F, P, LAYOUT, true>(v, p, t, buf0, buf1, tw, w0);
-    } else {
-        fft_run<F, P, LAYOUT, true, false>(v, p, t, buf0, buf1, twr);
-    }
-}
-
-constexpr int kMaxTw = 28;  // fft_tw_total(F) for F <= 8192
-
-template <int F>
-__device__ __forceinline__ void prefetch_twiddles(float2 *twr, int t, const float2 *tw) {
-    static_assert(fft_tw_total(F) <= kMaxTw, "twiddle registers");
-    fft_load_twiddles<F>(twr, t, tw);
-}
-
-__device__ __forceinline__ void track_max(const StageArgs &a, int scene, int cls, float m);
 
 // Solver::update_field_values (kernel/Solver.cpp:174-181): out = t_n - s*L*coef,
-// the last stage also t_n = out * PML factor.  Positions outside [0, n_out)
-// and lines past the tile get an out-of-block offset (no store).
-struct UpdateRegs {
-    int off[8][2];
-    float tnv[8][2], pm[8][2];
+// the last stage also t_n = out * PML factor.
+struct OutAddr {
+    int off0, off1, end, rows;
+    __device__ __forceinline__ OutAddr(Seg td, const Tile &x) {
+        const int off = (td->o_f + x.line * td->o_ls + x.t - td->wlen + kShift) * 4;
+        off0 = x.count > 0 ? off : kOOB;
+        off1 = x.count > 1 ? off + td->o_ls * 4 : kOOB;
+        end = td->wlen + td->n_out;
+        rows = x.rows(end);
+    }
 };
 
-template <int LAYOUT>
-__device__ __forceinline__ void prefetch_updates(const StageArgs &a, const TileDesc &td, const TileGeo<LAYOUT> &g,
-                                                 int p, int t, UpdateRegs &u) {
-    const int w = td.wlen, n_out = td.n_out;
-    const bool ok0 = 2 * p < td.count, ok1 = 2 * p + 1 < td.count;
-    const int pstep = td.o_ps * 4;
-    const int base = (td.o_f + (td.line0 + 2 * p) * td.o_ls) * 4 + (t - w) * pstep, lstep = td.o_ls * 4,
-              mstep = g.T * pstep;
-    const bool use_pml = a.last && td.is_pml;
-    const Rsrc rt = block_rsrc(a.tn, td.m_dom, td.m_size);
-    const Rsrc rp = block_rsrc(a.pml, td.m_dom, td.m_size);
+template <int V, bool SHORT>
+__device__ __forceinline__ void update_loads(const StageArgs &a, Seg td, const Tile &x, float2 (&tn)[V]) {
+    const OutAddr o(td, x);
+    const Rsrc rt = lead_rsrc(a.tn, td->m_dom, td->m_size);
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const int pos = t + m * g.T - w;
-        const bool okp = pos >= 0 && pos < n_out;
-        u.off[m][0] = okp && ok0 ? base + m * mstep : kOOB;
-        u.off[m][1] = okp && ok1 ? base + lstep + m * mstep : kOOB;
-        if constexpr (LAYOUT == 1) {
-            // columns: both lines of the pair in one 8-byte access (as in gather_issue)
-            const float2 x = bload2(rt, u.off[m][0]);
-            const float2 f = use_pml ? bload2(rp, u.off[m][0]) : make_float2(1.f, 1.f);
-            u.tnv[m][0] = x.x;
-            u.tnv[m][1] = x.y;
-            u.pm[m][0] = f.x;
-            u.pm[m][1] = f.y;
-        } else {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                u.tnv[m][q] = bload(rt, u.off[m][q]);
-                u.pm[m][q] = use_pml ? bload(rp, u.off[m][q]) : 1.f;
-            }
-        }
-    }
+    for (int m = 0; m < V; ++m)
+        if (m < kFull<V, SHORT> || m < o.rows)
+            tn[m] = make_float2(bload(rt, o.off0, m * x.T * 4), bload(rt, o.off1, m * x.T * 4));
 }
 
-template <int LAYOUT>
-__device__ __forceinline__ void finish_updates(const StageArgs &a, const TileDesc &td, int p, const float2 (&v)[8],
-                                               const UpdateRegs &u) {
-    const float sc = a.s * td.coef;
-    const Rsrc ro = block_rsrc(a.out, td.m_dom, td.m_size);
-    const Rsrc rt = block_rsrc(a.tn, td.m_dom, td.m_size);
-    float nv[8][2];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        nv[m][0] = __builtin_fmaf(-sc, v[m].x, u.tnv[m][0]);
-        nv[m][1] = __builtin_fmaf(-sc, v[m].y, u.tnv[m][1]);
-    }
-    if (a.umax) {
-        float mx = 0.f;
-#pragma unroll
-        for (int m = 0; m < 8; ++m)
-#pragma unroll
-            for (int q = 0; q < 2; ++q)
-                if (u.off[m][q] != kOOB) mx = fmaxf(mx, fabsf(nv[m][q]));
-        track_max(a, td.scene, td.vel ? 0 : 1, mx);
-    }
-    if (LAYOUT == 1 && 2 * p + 1 < td.count) {
-        // columns, both lines in the tile: 8-byte stores
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            bstore2(ro, u.off[m][0], nv[m][0], nv[m][1]);
-            if (a.last) bstore2(rt, u.off[m][0], nv[m][0] * u.pm[m][0], nv[m][1] * u.pm[m][1]);
-        }
-    } else {
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                bstore(ro, u.off[m][q], nv[m][q]);
-                if (a.last) bstore(rt, u.off[m][q], nv[m][q] * u.pm[m][q]);
-            }
-        }
-    }
-}
-
-// One derivative tile of one layout: NT threads, F = td.F in [FMIN, FMAX].
-// Flavours differ only in when the loads that depend on nothing but the
-// descriptor (filter, twiddles, t_n and PML operands) are issued:
-//  kEarly: all before the gather completes (most registers);
-//  kLate:  where they are used (fewest live registers, most resident waves);
-//  kMid:   filter and twiddles up front (the transforms then never wait on
-//          memory: the vector-memory counter is in order, so a late table
-//          load waits for every load before it), t_n where used.
-// All compute the same values in the same order.
-constexpr int kEarly = 0, kLate = 1, kMid = 2;
-template <int NT, int FMIN, int FMAX, int FL, int LAYOUT>
-__device__ __forceinline__ void tile_layout(const StageArgs &a, const TileDesc &td, float2 *buf0, float2 *buf1) {
-    const TileGeo<LAYOUT> g(td.F, NT);
-    const int tid = threadIdx.x;
-    const int p = g.pair(tid), t = g.lane_t(tid);
-    GatherRegs R;
-    gather_issue<NT, LAYOUT>(a, td, g, p, t, R);
-    float2 h[8];
-    constexpr bool LEAN = FL == kLate;
-    float2 twr[LEAN ? 1 : kMaxTw];
-    const float2 *tw = a.ctab + td.tw_off;
-    const float2 *hsrc = a.ctab + td.h_off;
-    if constexpr (!LEAN) {
-#pragma unroll
-        for (int m = 0; m < 8; ++m) h[m] = hsrc[t + m * g.T];
-        switch (td.F) {
-            case 128: if (FMIN <= 128 && FMAX >= 128) prefetch_twiddles<128>(twr, t, tw); break;
-            case 256: if (FMIN <= 256 && FMAX >= 256) prefetch_twiddles<256>(twr, t, tw); break;
-            case 512: if (FMIN <= 512 && FMAX >= 512) prefetch_twiddles<512>(twr, t, tw); break;
-            case 1024: if (FMIN <= 1024 && FMAX >= 1024) prefetch_twiddles<1024>(twr, t, tw); break;
-            case 2048: if (FMIN <= 2048 && FMAX >= 2048) prefetch_twiddles<2048>(twr, t, tw); break;
-            case 4096: if (FMIN <= 4096 && FMAX >= 4096) prefetch_twiddles<4096>(twr, t, tw); break;
-            case 8192: if (FMIN <= 8192 && FMAX >= 8192) prefetch_twiddles<8192>(twr, t, tw); break;
-            default: break;
-        }
-    }
-    UpdateRegs u;
-    if constexpr (FL == kEarly) prefetch_updates<LAYOUT>(a, td, g, p, t, u);
-    // buf1 holds the raw lines (2P lines, at most 18 NT floats); the window
-    // has slots of its own (no pass of any pair writes them)
-    __shared__ float win[2 * 32 + 1];
-    float *stage = reinterpret_cast<float *>(buf1);
-    float2 v[8];
-    gather_finish<LAYOUT>(a, td, g, p, t, R, stage, win, v);
-#define PSTD_FFT_CASE(FV)                                                                                \
-    case FV:                                                                                             \
-        if constexpr (FMIN <= FV && FMAX >= FV) derivative_fft<FV, NT, LAYOUT, LEAN>(v, h, twr, buf0, buf1, hsrc, tw); \
-        break;
-    switch (td.F) {
-        PSTD_FFT_CASE(128)
-        PSTD_FFT_CASE(256)
-        PSTD_FFT_CASE(512)
-        PSTD_FFT_CASE(1024)
-        PSTD_FFT_CASE(2048)
-        PSTD_FFT_CASE(4096)
-        PSTD_FFT_CASE(8192)
-        default: break;
-    }
-#undef PSTD_FFT_CASE
-    if constexpr (FL != kEarly) prefetch_updates<LAYOUT>(a, td, g, p, t, u);
-    finish_updates<LAYOUT>(a, td, p, v, u);
-}
-
-template <int NT, int FMIN, int FMAX, int FL>
-__device__ __forceinline__ void derivative_tile(const StageArgs &a, const TileDesc &td, float2 *buf0, float2 *buf1) {
-    if (td.dir == 0) tile_layout<NT, FMIN, FMAX, FL, 0>(a, td, buf0, buf1);
-    else tile_layout<NT, FMIN, FMAX, FL, 1>(a, td, buf0, buf1);
-}
-
-// F = 8192 lines as two 4096-point transforms.  One line pair per 512-thread
-// block; thread t holds positions n = t + 512 m (m = 0..15) of both lines (as
-// one complex value z, line 0 real, line 1 imaginary).  One radix-2
-// decimation-in-frequency step in registers: with W = e^{-2 pi i / 8192},
-// a[n] = z[n] + z[n+4096] and b[n] = (z[n] - z[n+4096]) W^n are the inputs of
-// the even and odd bins, Z[2k] = FFT4096(a)[k], Z[2k+1] = FFT4096(b)[k].  After
-// the filter H (8192 bins, 1/8192 folded in) the inverse recombines in the same
-// threads: y[n] = e[n] + W^-n o[n], y[n+4096] = e[n] - W^-n o[n], where
-// e = IFFT4096(H[2k] Z[2k]) and o = IFFT4096(H[2k+1] Z[2k+1]).  Half the LDS
-// of one 8192-point transform per block: two blocks share a CU.
-constexpr int kSplitT = 512;
-constexpr size_t kSplitLds = 2 * sizeof(float2) * LdsMap<4096, 1, 0>::SIZE;  // 72 KiB (the raw staging fits)
-
-struct SplitGather {
-    float ra[16][2], rb[16][2];
-    float h1a[2], h1b[2], h2a[2], h2b[2];
-    int hpos1, hpos2;
-    float win;
-};
-
-// raw staging of the pair in LDS (floats): rows line-major at pitch 9F/8,
-// columns position-major with the two lines adjacent
-template <int LAYOUT>
-__device__ __forceinline__ int split_stage_at(int ll, int pos) {
-    return LAYOUT == 0 ? ll * (9 * 8192 / 8) + pos : ll + 2 * pos;
-}
-
-template <int LAYOUT>
-__device__ __forceinline__ void split_gather_issue(const StageArgs &a, const TileDesc &td, int t, SplitGather &R) {
-    const int w = td.wlen, nm = td.n_main, vel = td.vel, count = td.count;
-    __builtin_assume(w > 0 && w <= 32);
-    R.win = (int)threadIdx.x <= 2 * w ? a.ftab[td.win_off + threadIdx.x] : 0.f;
-    const float *A = vel ? a.vsrc : a.p0a;
-    const bool hasB = !vel && a.p0b != nullptr;
-    const float *B = hasB ? a.p0b : A;
-    const Rsrc rmA = block_rsrc(A, td.m_dom, td.m_size);
-    const Rsrc rmB = block_rsrc(B, td.m_dom + (td.m_b - td.m_a), td.m_size - (td.m_b - td.m_a));
-    const int pstep = td.m_ps * 4;
-    const int lbase = (td.m_a + td.line0 * td.m_ls) * 4 + (t - w) * pstep, lstep = td.m_ls * 4,
-              mstep = kSplitT * pstep;
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-        const int e = t + m * kSplitT - w;
-        const bool ok = e >= 0 && e < nm;
-        const int o0 = ok ? lbase + m * mstep : kOOB;
-        const int o1 = ok && 1 < count ? lbase + lstep + m * mstep : kOOB;
-        if constexpr (LAYOUT == 1) {
-            // columns: the two lines are adjacent floats (an odd last line reads
-            // the block's spare float after its partner; dropped below)
-            const float2 x = bload2(rmA, o0);
-            const float2 y = hasB ? bload2(rmB, o0) : make_float2(0.f, 0.f);
-            R.ra[m][0] = x.x;
-            R.ra[m][1] = x.y;
-            R.rb[m][0] = y.x;
-            R.rb[m][1] = y.y;
-        } else {
-            R.ra[m][0] = bload(rmA, o0);
-            R.ra[m][1] = bload(rmA, o1);
-            R.rb[m][0] = hasB ? bload(rmB, o0) : 0.f;
-            R.rb[m][1] = hasB ? bload(rmB, o1) : 0.f;
-        }
-    }
-    // halos: 2 w values per line from the side blocks; rows: item (line, j),
-    // columns: item j with both lines in one 8-byte load
-    const Rsrc r1A = block_rsrc(A, td.s1_dom, td.s1_size);
-    const Rsrc r1B = block_rsrc(B, td.s1_dom + (td.s1_b - td.s1_a), td.s1_size - (td.s1_b - td.s1_a));
-    const Rsrc r2A = block_rsrc(A, td.s2_dom, td.s2_size);
-    const Rsrc r2B = block_rsrc(B, td.s2_dom + (td.s2_b - td.s2_a), td.s2_size - (td.s2_b - td.s2_a));
-    const int i = threadIdx.x;
-    const int ll = LAYOUT == 0 ? i >> td.wlog : 0, j = LAYOUT == 0 ? i & ((1 << td.wlog) - 1) : i;
-    const bool item = LAYOUT == 0 ? (ll < 2 && j < w) : j < w;
-    const bool ok = item && ll < count;
-    const int line = td.line0 + ll;
-    const int o1 = ok && td.s1_len >= 0
-                       ? (td.s1_a + (line + td.s1_line) * td.s1_ls + (td.s1_len - w - vel + j) * td.s1_ps) * 4
-                       : kOOB;
-    const int o2 = ok && td.s2_len >= 0 ? (td.s2_a + (line + td.s2_line) * td.s2_ls + (j + vel) * td.s2_ps) * 4 : kOOB;
-    if constexpr (LAYOUT == 1) {
-        const float2 x1 = bload2(r1A, o1), x2 = bload2(r2A, o2);
-        const float2 y1 = hasB ? bload2(r1B, o1) : make_float2(0.f, 0.f);
-        const float2 y2 = hasB ? bload2(r2B, o2) : make_float2(0.f, 0.f);
-        R.h1a[0] = x1.x; R.h1a[1] = x1.y; R.h2a[0] = x2.x; R.h2a[1] = x2.y;
-        R.h1b[0] = y1.x; R.h1b[1] = y1.y; R.h2b[0] = y2.x; R.h2b[1] = y2.y;
-    } else {
-        R.h1a[0] = bload(r1A, o1);
-        R.h2a[0] = bload(r2A, o2);
-        R.h1b[0] = hasB ? bload(r1B, o1) : 0.f;
-        R.h2b[0] = hasB ? bload(r2B, o2) : 0.f;
-        R.h1a[1] = R.h2a[1] = R.h1b[1] = R.h2b[1] = 0.f;
-    }
-    R.hpos1 = item ? split_stage_at<LAYOUT>(ll, j) : -1;
-    R.hpos2 = item ? split_stage_at<LAYOUT>(ll, w + nm + j) : -1;
-}
-
-// The windowed pair values at positions t + 512 m, combined into a and b.
-template <int LAYOUT>
-__device__ __forceinline__ void split_gather_finish(const TileDesc &td, int t, const SplitGather &R, float *stage,
-                                                    float *win, const float2 *tw8, float2 (&va)[8], float2 (&vb)[8]) {
-    const int w = td.wlen, nm = td.n_main, vel = td.vel;
-    __builtin_assume(w > 0 && w <= 32);
-    const float c_s1 = td.c_s1, c_m1 = td.c_m1, c_s2 = td.c_s2, c_m2 = td.c_m2;
-    const bool ok1 = LAYOUT == 0 || 1 < td.count;
-    float raw[16][2];
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-        const int pos = t + m * kSplitT;
-        const bool mid = pos >= w && pos < w + nm;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            raw[m][q] = q == 0 || ok1 ? R.ra[m][q] + R.rb[m][q] : 0.f;
-            if (mid) stage[split_stage_at<LAYOUT>(q, pos)] = raw[m][q];
-        }
-    }
-    if (R.hpos1 >= 0) {
-        if constexpr (LAYOUT == 1) {
-            *reinterpret_cast<float2 *>(&stage[R.hpos1]) =
-                make_float2(R.h1a[0] + R.h1b[0], ok1 ? R.h1a[1] + R.h1b[1] : 0.f);
-            *reinterpret_cast<float2 *>(&stage[R.hpos2]) =
-                make_float2(R.h2a[0] + R.h2b[0], ok1 ? R.h2a[1] + R.h2b[1] : 0.f);
-        } else {
-            stage[R.hpos1] = R.h1a[0] + R.h1b[0];
-            stage[R.hpos2] = R.h2a[0] + R.h2b[0];
-        }
-    }
-    if ((int)threadIdx.x <= 2 * w) win[threadIdx.x] = R.win;
-    __syncthreads();
-    // positions n and n + 4096 in turn, combined at once (fewer live registers)
-    auto windowed = [&](int m) {
-        const int i = t + m * kSplitT;
-        const bool left = i < w, right = i >= w + nm && i < 2 * w + nm, mid = i >= w && i < w + nm;
-        const int j = i - w - nm;
-        float out[2] = {0.f, 0.f};
-        if (left || right) {
-            const int mpos = left ? (vel ? w - i : w - 1 - i) : (vel ? nm - 2 - j : nm - 1 - j);
-            const float cs = left ? c_s1 : c_s2, cm = left ? c_m1 : c_m2;
-            const float wv = win[left ? i : w + 1 + j];
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const float sv = stage[split_stage_at<LAYOUT>(q, i)];
-                const float refl = stage[split_stage_at<LAYOUT>(q, w + mpos)];
-                out[q] = __builtin_fmaf(sv, cs, refl * cm) * wv;
-            }
-        }
-        return make_float2(mid ? raw[m][0] : out[0], mid ? raw[m][1] : out[1]);
+// v: the conjugate of the derivative (two real lines: the second one negated)
+template <int V, bool SHORT>
+__device__ __forceinline__ void update_stores(const StageArgs &a, Seg td, const Tile &x, float2 (&v)[V],
+                                              const float2 (&tn)[V], int slot) {
+    const OutAddr o(td, x);
+    const int w = td->wlen, T4 = x.T * 4;
+    const float sc = a.s * td->coef;
+    const Rsrc ro = lead_rsrc(a.out, td->m_dom, td->m_size);
+    float mx = 0.f;
+    // the first rows hold the left halo (w <= 32), rows from kFull on can leave the line
+    auto inside = [&](int m) __attribute__((always_inline)) {
+        const int pos = x.t + m * x.T;
+        return (m > (SHORT ? 1 : 0) || pos >= w) && (m < kFull<V, SHORT> || pos < o.end);
     };
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const float2 z0 = windowed(m), z1 = windowed(m + 8);
-        va[m] = cadd(z0, z1);
-        vb[m] = cmul(csub(z0, z1), tw8[t + m * kSplitT]);
-    }
-}
-
-// Update of the outputs at positions base + t + 512 m (out = t_n - s coef L;
-// the last stage also t_n = out * PML), as finish_updates.
-template <int LAYOUT>
-__device__ __forceinline__ float split_update(const StageArgs &a, const TileDesc &td, int t, int base,
-                                              const float2 (&y)[8]) {
-    const int w = td.wlen, n_out = td.n_out;
-    const bool ok1 = 1 < td.count;
-    const int pstep = td.o_ps * 4;
-    const int obase = (td.o_f + td.line0 * td.o_ls) * 4, lstep = td.o_ls * 4;
-    const bool use_pml = a.last && td.is_pml;
-    const Rsrc rt = block_rsrc(a.tn, td.m_dom, td.m_size);
-    const Rsrc rp = block_rsrc(a.pml, td.m_dom, td.m_size);
-    const Rsrc ro = block_rsrc(a.out, td.m_dom, td.m_size);
-    const float sc = a.s * td.coef;
-    int off[8];
-    float tnv[8][2], pm[8][2];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const int pos = base + t + m * kSplitT - w;
-        off[m] = pos >= 0 && pos < n_out ? obase + pos * pstep : kOOB;
-        if constexpr (LAYOUT == 1) {
-            const float2 x = bload2(rt, off[m]);
-            const float2 f = use_pml ? bload2(rp, off[m]) : make_float2(1.f, 1.f);
-            tnv[m][0] = x.x; tnv[m][1] = x.y; pm[m][0] = f.x; pm[m][1] = f.y;
-        } else {
-            const int o1 = off[m] == kOOB || !ok1 ? kOOB : off[m] + lstep;
-            tnv[m][0] = bload(rt, off[m]);
-            tnv[m][1] = bload(rt, o1);
-            pm[m][0] = use_pml ? bload(rp, off[m]) : 1.f;
-            pm[m][1] = use_pml ? bload(rp, o1) : 1.f;
+    for (int m = 0; m < V; ++m) {
+        if ((m < kFull<V, SHORT> || m < o.rows) && inside(m)) {
+            v[m] = make_float2(__builtin_fmaf(-sc, v[m].x, tn[m].x), __builtin_fmaf(sc, v[m].y, tn[m].y));
+            bstore(ro, o.off0, m * T4, v[m].x);
+            bstore(ro, o.off1, m * T4, v[m].y);
+            mx = fmaxf(mx, fmaxf(fabsf(v[m].x), fabsf(v[m].y)));
         }
     }
-    float mx = 0.f;
+    if (a.last) {
+        const Rsrc rt = lead_rsrc(a.tn, td->m_dom, td->m_size);
+        if (td->is_pml) {
+            const Rsrc rp = lead_rsrc(a.pml, td->m_dom, td->m_size);
+            // four rows of threads at a time: few registers
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const float n0 = __builtin_fmaf(-sc, y[m].x, tnv[m][0]);
-        const float n1 = __builtin_fmaf(-sc, y[m].y, tnv[m][1]);
-        if (off[m] != kOOB) mx = fmaxf(mx, ok1 ? fmaxf(fabsf(n0), fabsf(n1)) : fabsf(n0));
-        if (LAYOUT == 1 && ok1) {
-            bstore2(ro, off[m], n0, n1);
-            if (a.last) bstore2(rt, off[m], n0 * pm[m][0], n1 * pm[m][1]);
-        } else {
-            const int o1 = off[m] == kOOB || !ok1 ? kOOB : off[m] + lstep;
-            bstore(ro, off[m], n0);
-            bstore(ro, o1, n1);
-            if (a.last) {
-                bstore(rt, off[m], n0 * pm[m][0]);
-                bstore(rt, o1, n1 * pm[m][1]);
+            for (int m0 = 0; m0 < V; m0 += 4) {
+                if (m0 >= kFull<V, SHORT> && m0 >= o.rows) break;
+                float2 pm[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    if (m0 + m < kFull<V, SHORT> || m0 + m < o.rows)
+                        pm[m] = make_float2(bload(rp, o.off0, (m0 + m) * T4), bload(rp, o.off1, (m0 + m) * T4));
+#pragma unroll
+                for (int m = 0; m < 4; ++m) v[m0 + m] = make_float2(v[m0 + m].x * pm[m].x, v[m0 + m].y * pm[m].y);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < V; ++m) {
+            if ((m < kFull<V, SHORT> || m < o.rows) && inside(m)) {
+                bstore(rt, o.off0, m * T4, v[m].x);
+                bstore(rt, o.off1, m * T4, v[m].y);
             }
         }
     }
-    return mx;
+    track_max(a, slot, mx);
 }
 
-template <int LAYOUT>
-__device__ __forceinline__ void split_tile(const StageArgs &a, const TileDesc &td, float2 *lds) {
-    const int t = threadIdx.x;
-    float2 *buf0 = lds, *buf1 = lds + LdsMap<4096, 1, LAYOUT>::SIZE;
-    __shared__ float win[2 * 32 + 1];
-    SplitGather R;
-    split_gather_issue<LAYOUT>(a, td, t, R);
-    const float2 *tw8 = a.ctab + td.tw_off, *tw4 = a.ctab + td.tw2_off, *h = a.ctab + td.h_off;
-    float2 va[8], vb[8];
-    split_gather_finish<LAYOUT>(td, t, R, reinterpret_cast<float *>(lds), win, tw8, va, vb);
-    const float2 w0[kTwPass] = {};
-    // even bins: e = IFFT(H[2k] FFT(a)); the staging is read before the first pass writes
-    __syncthreads();
-    fft_run_ahead<4096, 1, LAYOUT, false>(va, 0, t, buf0, buf1, tw4, w0);
+// SHORT: F = 128; SPLIT: F = 8192 (fft_line.h's two sequences)
+template <int V, int NT, bool SHORT, bool SPLIT>
+__device__ __forceinline__ void derivative_tile(const StageArgs &a, Seg td, Ref ref, float2 *lds) {
+    constexpr int kLogV = V == 16 ? 4 : 3;
+    const int F = td->F, logT = 31 - kLogV - __builtin_clz(F);
+    Tile x;
+    x.logT = logT;
+    x.T = 1 << logT;
+    x.p = threadIdx.x >> logT;
+    x.t = threadIdx.x & (x.T - 1);
+    x.line = ref->line0 + 2 * x.p;
+    x.count = ref->count - 2 * x.p;
+    x.pitch = lds_pitch(F);
+    float2 *buf = lds + x.p * x.pitch;
+    // the tables through a buffer resource: one lane offset, the rest in scalar registers
+    const Table tab{__builtin_amdgcn_make_buffer_rsrc((void *)a.ctab, (short)0, 0x7fffffff, 0x00020000)};
+    const int t = x.t;
+    // 8 values per thread leave the registers to load t_n and the filter with the
+    // lines (two memory latencies less); with 16 they are loaded where they are used
+    constexpr bool kTnEarly = V == 8;
+    float2 v[V], tn[V], h[V];
+    // pairs of the filter's values as the transforms leave them: m and m + 1, or
+    // (8192) the even and the odd bin of value m
+    auto filter_loads = [&]() __attribute__((always_inline)) {
+        const int h_off = td->h_off * 8;
 #pragma unroll
-    for (int m = 0; m < 8; ++m) va[m] = cmul(va[m], h[2 * (t + m * kSplitT)]);
-    __syncthreads();
-    fft_run_ahead<4096, 1, LAYOUT, true>(va, 0, t, buf0, buf1, tw4, w0);
-    // odd bins: o = IFFT(H[2k+1] FFT(b))
-    __syncthreads();
-    fft_run_ahead<4096, 1, LAYOUT, false>(vb, 0, t, buf0, buf1, tw4, w0);
+        for (int m = 0; m < V; m += 2) tab.pair(h[m], h[m + 1], t * 16, h_off + (m << (logT + 3)));
+    };
+    gather<V, NT, SHORT>(a, td, x, lds, v);
+    if constexpr (kTnEarly) update_loads<V, SHORT>(a, td, x, tn);
+    if constexpr (kTnEarly) filter_loads();
+    if constexpr (SPLIT) split_first(v, t, tab, td->tw_off * 8);
+    // forward transform; spectral derivative: the Hermitian filter, which carries
+    // the 1/F of kernel/core/kernel_functions.cpp:243,306; conjugate; the forward
+    // transform again (the conjugate of the inverse)
+#pragma unroll 1
+    for (int dir = 0; dir < 2; ++dir) {
+        const int tw = again(td->tw_off * 8);
+        int ti = t;
+        asm volatile("" : "+v"(ti));  // LDS addresses per pass, not kept for all lengths across the loop
+#define PSTD_FFT_CASE(FV)                                                                            \
+    case FV:                                                                                         \
+        if constexpr (fft_values(FV) == V && FV <= V * NT && (FV == 128) == SHORT && (FV == 8192) == SPLIT) \
+            fft_run<FV>(v, ti, buf, tab, tw);                                                         \
+        break;
+        switch (F) {
+            PSTD_FFT_CASE(128)
+            PSTD_FFT_CASE(256)
+            PSTD_FFT_CASE(512)
+            PSTD_FFT_CASE(1024)
+            PSTD_FFT_CASE(2048)
+            PSTD_FFT_CASE(4096)
+            PSTD_FFT_CASE(8192)
+            default: break;
+        }
+#undef PSTD_FFT_CASE
+        if (dir == 0) {
+            if constexpr (!kTnEarly) filter_loads();
 #pragma unroll
-    for (int m = 0; m < 8; ++m) vb[m] = cmul(vb[m], h[2 * (t + m * kSplitT) + 1]);
-    __syncthreads();
-    fft_run_ahead<4096, 1, LAYOUT, true>(vb, 0, t, buf0, buf1, tw4, w0);
-    // y[n] = e[n] + W^-n o[n], y[n + 4096] = e[n] - W^-n o[n]
-    float2 lo[8], hi[8];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        float2 wn = tw8[t + m * kSplitT];
-        wn.y = -wn.y;
-        const float2 wo = cmul(vb[m], wn);
-        lo[m] = cadd(va[m], wo);
-        hi[m] = csub(va[m], wo);
+            for (int m = 0; m < V; ++m) {
+                const float2 y = cmul(v[m], h[SPLIT ? 2 * (m & 7) + (m >> 3) : m]);
+                v[m] = make_float2(y.x, -y.y);
+            }
+        }
     }
-    const float mx = fmaxf(split_update<LAYOUT>(a, td, t, 0, lo), split_update<LAYOUT>(a, td, t, 4096, hi));
-    track_max(a, td.scene, td.vel ? 0 : 1, mx);
+    if constexpr (SPLIT) split_last(v, t, tab, td->tw_off * 8);
+    // the descriptor again: the gather's fields need not stay in scalar registers
+    const Seg to = (Seg)a.segs + again(ref->seg);
+    if constexpr (!kTnEarly) update_loads<V, SHORT>(a, to, x, tn);
+    update_stores<V, SHORT>(a, to, x, v, tn, ref->slot);
 }
 
-// One extra workgroup of a launch samples the receivers (p0 = px0 + py0 of the
-// previous step, read from the arena `p0a`/`p0b` point at in the first stage).
+// One extra workgroup of a launch samples the receivers (p0 of the previous
+// step, read from the arena the first stage reads it from).
 __device__ void sample_receivers(const StageArgs &a) {
     if (a.slot < 0) return;
     for (int r = threadIdx.x; r < a.nrec; r += blockDim.x) {
         const ReceiverCell c = a.cells[r];
         if (c.px < 0) continue;  // spectral receiver
-        a.samples[(size_t)a.slot * a.nrec + r] = a.p0a[c.px] + a.p0b[c.py];
+        a.samples[(size_t)a.slot * a.nrec + r] = a.p0_two ? a.p0[c.px] + a.p0[c.py] : a.p0[c.px];
     }
 }
 
@@ -847,38 +499,36 @@ __device__ void sample_receivers(const StageArgs &a) {
 // kernel/Solver.cpp:174-181); the last stage applies the PML factor.  Each
 // thread issues all of its loads before its stores.
 template <int NT>
-__device__ void passthrough_tile(const StageArgs &a, const TileDesc &td) {
+__device__ __forceinline__ void passthrough_tile(const StageArgs &a, Seg td, Ref ref) {
     constexpr int PER = kPassChunk / NT;
-    const Rsrc rt = block_rsrc(a.tn, td.m_dom, td.m_size);
-    const Rsrc rp = block_rsrc(a.pml, td.m_dom, td.m_size);
-    const Rsrc ro = block_rsrc(a.out, td.m_dom, td.m_size);
-    const bool use_pml = a.last && td.is_pml;
+    const Rsrc rt = block_rsrc(a.tn, td->m_dom, td->m_size);
+    const Rsrc rp = block_rsrc(a.pml, td->m_dom, td->m_size);
+    const Rsrc ro = block_rsrc(a.out, td->m_dom, td->m_size);
+    const bool use_pml = a.last && td->is_pml;
     float v[PER], f[PER];
     int off[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int e = threadIdx.x + k * NT;
-        off[k] = e < td.count ? (td.o_f + td.line0 + e) * 4 : kOOB;
+        off[k] = e < ref->count ? (td->o_f + ref->line0 + e) * 4 : kOOB;
         v[k] = bload(rt, off[k]);
         f[k] = use_pml ? bload(rp, off[k]) : 1.f;
     }
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        bstore(ro, off[k], v[k]);
-        if (use_pml) bstore(rt, off[k], v[k] * f[k]);
+        bstore(ro, off[k], 0, v[k]);
+        if (use_pml) bstore(rt, off[k], 0, v[k] * f[k]);
     }
-    if (a.umax) {
-        float mx = 0.f;
+    float mx = 0.f;
 #pragma unroll
-        for (int k = 0; k < PER; ++k) mx = fmaxf(mx, fabsf(v[k]));
-        track_max(a, td.scene, td.vel ? 0 : 1, mx);  // vel: 1 for px/py (as the velocity lines that write them)
-    }
+    for (int k = 0; k < PER; ++k) mx = fmaxf(mx, fabsf(v[k]));
+    track_max(a, ref->slot, mx);
 }
 
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs on XCD
 // b % 8) and every XCD has its own L2.  With `remap`, XCD x works through a
 // contiguous run of the tile list instead of every 8th tile, so tiles of
-// neighbouring lines (the columns of one cache line, the rows of one halo)
+// neighbouring lines (which share the cache lines of the other layout's field)
 // share that L2.  A bijection of [0, n).
 __device__ __forceinline__ int tile_index(int b, int n, int remap) {
     if (!remap) return b;
@@ -887,40 +537,35 @@ __device__ __forceinline__ int tile_index(int b, int n, int remap) {
     return x * q + min(x, r) + l;
 }
 
-// F <= 2048 class, NT = 128, 256 or 512 threads (128: F <= 1024 only): two LDS
-// buffers of P * F = 8 * NT complex values each (padded).  Wider blocks hold
-// more lines per tile (for columns, more of each row per wave access) at the
-// same waves per CU; narrower ones spread a small scene over more CUs.
-template <int NT, int FL>
-__global__ void __launch_bounds__(NT) stage_small_kernel(StageArgs a) {
-    constexpr int kBuf = lds_padded(8 * NT);
-    __shared__ float2 lds[2 * kBuf];
-    // a copy taken before any store: the descriptor stays in scalar registers
-    const TileDesc td = a.tiles[tile_index(blockIdx.x, gridDim.x, a.remap)];
-    if (td.kind == 2) {
-        sample_receivers(a);
-        return;
-    }
-    if (td.kind == 1) {
-        passthrough_tile<NT>(a, td);
-        return;
-    }
-    derivative_tile<NT, 128, (NT >= 256 ? 2048 : 1024), FL>(a, td, lds, lds + kBuf);
-}
+// One launch per RK stage covers every FFT-form line: NT = 128, 256 or 512
+// threads, lines of F <= 16 NT, about 17 NT complex values of LDS.  Pairs of F <=
+// 1024 are one wavefront's (or a part's) business whatever NT is; the block size
+// decides how long the lines may be (8192-point ones take a 512-thread block),
+// how many adjacent lines a tile has and how finely a small scene spreads over
+// the CUs.  Bound by the VALU and the L1 together (16 sources of 512 x 1024 twice:
+// VALU 63 % and L1 address units 67 % busy, 270 us of the 350 us stage; one launch
+// of 8-value tiles, 568 us per stage, had each column access touch 8-16 bytes of a
+// cache line).
+constexpr size_t stage_lds(int nt) { return (size_t)(16 * nt / 256) * lds_pitch(256) * sizeof(float2); }
 
-template <int F, int FL>
-__global__ void __launch_bounds__(F / 8) stage_big_kernel(StageArgs a) {
+// At most 128 VGPRs: four wavefronts per SIMD, what the LDS allows too.
+template <int NT>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
+stage_fft_kernel(StageArgs a) {
     extern __shared__ float2 lds_dyn[];
-    const TileDesc td = a.tiles[tile_index(blockIdx.x, gridDim.x, a.remap)];
-    derivative_tile<F / 8, F, F, FL>(a, td, lds_dyn, lds_dyn + LdsMap<F, 1, 0>::SIZE);
-}
-
-// two blocks per CU: 16 waves, at most 128 VGPRs each
-__global__ void __launch_bounds__(kSplitT) __attribute__((amdgpu_waves_per_eu(4))) stage_split_kernel(StageArgs a) {
-    extern __shared__ float2 lds_split[];
-    const TileDesc td = a.tiles[tile_index(blockIdx.x, gridDim.x, a.remap)];
-    if (td.dir == 0) split_tile<0>(a, td, lds_split);
-    else split_tile<1>(a, td, lds_split);
+    const Ref ref = (Ref)a.tiles + tile_index(blockIdx.x, gridDim.x, a.remap);
+    const Seg td = (Seg)a.segs + ref->seg;
+    switch (td->kind) {
+        case 0:
+            if (td->F == 128) derivative_tile<8, NT, true, false>(a, td, ref, lds_dyn);
+            else if (fft_values(td->F) == 8) derivative_tile<8, NT, false, false>(a, td, ref, lds_dyn);
+            else if (NT == 512 && td->F == 8192) derivative_tile<16, NT, false, NT == 512>(a, td, ref, lds_dyn);
+            else derivative_tile<16, NT, false, false>(a, td, ref, lds_dyn);
+            break;
+        case 1: passthrough_tile<NT>(a, td, ref); break;
+        case 2: sample_receivers(a); break;
+        default: break;
+    }
 }
 
 __global__ void receiver_kernel(const float *__restrict__ arena, const ReceiverCell *__restrict__ cells, int nrec,
@@ -944,9 +589,10 @@ __global__ void receiver_kernel(const float *__restrict__ arena, const ReceiverC
 // [side-1 tail | domain rows | side-2 head].  Pass 2: one wave per receiver,
 // the column buffer against the Y-shift row of the receiver's row.
 struct SILine {
-    long long m_px, m_py;    // arena offsets of the line's first main value in px0, py0
+    long long m_px, m_py;    // arena offsets of the line's first main value in px0 (or p0), py0
     long long s1_px, s1_py;  // first of the w side-1 tail values; -1: no neighbour (zeros)
     long long s2_px, s2_py;  // first of the w side-2 head values; -1: zeros
+    int m_ld, s1_ld, s2_ld;  // py0 is column-major: elements from one value to the next
     int n_main, w;
     int coef;                // first of the line's K weights in the weight table
     int dst;                 // element of the column buffer
@@ -964,8 +610,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 __global__ __launch_bounds__(256) void si_line_kernel(const float *__restrict__ arena, const SILine *__restrict__ lines,
-                                                      int nlines, const float *__restrict__ coef,
+                                                      int nlines, int two, const float *__restrict__ coef,
                                                       float *__restrict__ col) {
+    // two: p0 = px + py of a stage arena; otherwise the arena holds p0 in the px slots
     // jobs are sorted by line: the receivers reading one line are neighbours,
     // and XCD-contiguous runs of blocks put them on one XCD (its L2 serves the
     // line after the first read)
@@ -978,11 +625,16 @@ __global__ __launch_bounds__(256) void si_line_kernel(const float *__restrict__ 
     for (int k = lane; k < K; k += 64) {
         float u = 0.f;
         if (k < w) {
-            if (L.s1_px >= 0) u = arena[L.s1_px + k] + arena[L.s1_py + k];
+            if (L.s1_px >= 0) {
+                u = arena[L.s1_px + k];
+                if (two) u += arena[L.s1_py + (long long)k * L.s1_ld];
+            }
         } else if (k < w + n) {
-            u = arena[L.m_px + (k - w)] + arena[L.m_py + (k - w)];
+            u = arena[L.m_px + (k - w)];
+            if (two) u += arena[L.m_py + (long long)(k - w) * L.m_ld];
         } else if (L.s2_px >= 0) {
-            u = arena[L.s2_px + (k - w - n)] + arena[L.s2_py + (k - w - n)];
+            u = arena[L.s2_px + (k - w - n)];
+            if (two) u += arena[L.s2_py + (long long)(k - w - n) * L.s2_ld];
         }
         acc = fmaf(cf[k], u, acc);
     }
@@ -1000,18 +652,104 @@ __global__ __launch_bounds__(64) void si_point_kernel(const float *__restrict__ 
     if (threadIdx.x == 0) samples[(size_t)slot * nrec + P.rec] = acc;
 }
 
-struct P0Range {
-    long long px, py;  // arena element offsets of px0 and py0 of one domain
-    long long n;
+// One 64 x 64-cell piece of a domain for the passes between the two layouts.
+struct P0Tile {
+    long long px, py;  // arena offsets of the domain's px (row-major) and py (column-major) fields
+    int nx, ny, x0, y0;
 };
+constexpr int kP0Side = 64;
 
-__global__ void p0_materialise_kernel(const float *__restrict__ src, float *__restrict__ p0i,
-                                      const P0Range *__restrict__ ranges, int nr) {
-    // P0I.px-slot = px0 + py0 of every domain
-    for (int k = blockIdx.y; k < nr; k += gridDim.y) {
-        const P0Range r = ranges[k];
-        for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < r.n; e += (long long)gridDim.x * blockDim.x)
-            p0i[r.px + e] = src[r.px + e] + src[r.py + e];
+// p0 = px0 + py0 (kernel/Solver.cpp:114-116) of every cell in both layouts: the
+// px slots of `p0` row-major, the py slots column-major.  Bound by HBM (16
+// bytes per cell); a tile of 64 x 64 is turned through LDS so that all four
+// accesses run along 256-byte pieces of a row (pitch 65: the turned read is
+// free of bank conflicts).
+// `py_src` false: p0's px slots hold p0 already, only its transpose is written.
+// In the GEMM form the first blocks bring the stage's maxima together, one per
+// scene and class (`mx`).
+struct MaxArgs {
+    const float *wmax;
+    const int2 *first;  // group g's slots: first[g].x .. first[g + 1].x of the FFT-form tiles, .y of the GEMM tiles
+    unsigned *umax;
+    int n;              // groups (0: none)
+};
+__device__ void max_reduce(const MaxArgs &x, int g) {
+    __shared__ float part[4];
+    const int2 b = x.first[g], e = x.first[g + 1];
+    float m = 0.f;
+    for (int i = b.x + threadIdx.x; i < e.x; i += 256) m = fmaxf(m, x.wmax[i]);
+    for (int i = b.y + threadIdx.x; i < e.y; i += 256) m = fmaxf(m, x.wmax[i]);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) x.umax[g] = __float_as_uint(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+}
+
+__global__ void __launch_bounds__(256) p0_pass_kernel(const float *__restrict__ src, float *__restrict__ p0,
+                                                      const P0Tile *__restrict__ tiles, int py_src, MaxArgs mx) {
+    __shared__ float turn[kP0Side][kP0Side + 1];
+    if ((int)blockIdx.x < mx.n) {
+        max_reduce(mx, blockIdx.x);
+        return;
+    }
+    const P0Tile T = tiles[blockIdx.x - mx.n];
+    const int lane = threadIdx.x & 63, row0 = threadIdx.x >> 6;
+    const int w = min(kP0Side, T.nx - T.x0), h = min(kP0Side, T.ny - T.y0);
+    float v[kP0Side / 4];
+    // row-major side: rows y0 + r, columns x0 + lane
+    const float *row = (py_src ? src : p0) + T.px + (long long)T.y0 * T.nx + T.x0 + lane;
+#pragma unroll
+    for (int i = 0; i < kP0Side / 4; ++i) {
+        const int r = row0 + 4 * i;
+        v[i] = r < h && lane < w ? row[(long long)r * T.nx] : 0.f;
+    }
+    if (py_src) {
+        // column-major side: columns x0 + c, rows y0 + lane
+        const float *col = src + T.py + (long long)T.x0 * T.ny + T.y0 + lane;
+#pragma unroll
+        for (int i = 0; i < kP0Side / 4; ++i) {
+            const int c = row0 + 4 * i;
+            turn[lane][c] = c < w && lane < h ? col[(long long)c * T.ny] : 0.f;
+        }
+        __syncthreads();
+        float *out = p0 + T.px + (long long)T.y0 * T.nx + T.x0 + lane;
+#pragma unroll
+        for (int i = 0; i < kP0Side / 4; ++i) {
+            const int r = row0 + 4 * i;
+            v[i] += turn[r][lane];
+            if (r < h && lane < w) out[(long long)r * T.nx] = v[i];
+        }
+        // every thread rewrites the slots that it alone has read
+    }
+#pragma unroll
+    for (int i = 0; i < kP0Side / 4; ++i) turn[row0 + 4 * i][lane] = v[i];
+    __syncthreads();
+    float *out = p0 + T.py + (long long)T.x0 * T.ny + T.y0 + lane;
+#pragma unroll
+    for (int i = 0; i < kP0Side / 4; ++i) {
+        const int c = row0 + 4 * i;
+        if (c < w && lane < h) out[(long long)c * T.ny] = turn[lane][c];
+    }
+}
+
+// dst (cols x rows) = transpose of src (rows x cols): host fields are row-major,
+// vy and py are stored column-major.
+__global__ void __launch_bounds__(256) transpose_kernel(const float *__restrict__ src, float *__restrict__ dst, int rows,
+                                                        int cols) {
+    __shared__ float turn[kP0Side][kP0Side + 1];
+    const int lane = threadIdx.x & 63, row0 = threadIdx.x >> 6;
+    const int x0 = blockIdx.x * kP0Side, y0 = blockIdx.y * kP0Side;
+#pragma unroll
+    for (int i = 0; i < kP0Side / 4; ++i) {
+        const int r = y0 + row0 + 4 * i;
+        if (r < rows && x0 + lane < cols) turn[row0 + 4 * i][lane] = src[(long long)r * cols + x0 + lane];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kP0Side / 4; ++i) {
+        const int c = x0 + row0 + 4 * i;
+        if (c < cols && y0 + lane < rows) dst[(long long)c * rows + y0 + lane] = turn[lane][row0 + 4 * i];
     }
 }
 
@@ -1021,8 +759,9 @@ __global__ void p0_materialise_kernel(const float *__restrict__ src, float *__re
 // u = [side1 tail | main | side2 head] (K values).  One workgroup (4 waves,
 // two per CU) computes 128 lines x 128 outputs of C = U D^T on MFMA and
 // applies the RK update:
-//  * the input lines are read as FP32 straight from the stage state (p0 as
-//    px + py), scaled by the scene's power of two 2^e and split into two
+//  * the input lines are read as FP32 (p0 as the pass after each stage left it,
+//    vx and vy straight from the stage state), scaled by the scene's power of
+//    two 2^e and split into two
 //    16-bit parts while they are staged into LDS (U = hi + lo: FP16 keeps 22
 //    bits when every scaled value is below 2^15, BF16 16 bits at any scale);
 //  * D is stored split the same way (one power of two per matrix), as the
@@ -1031,17 +770,16 @@ __global__ void p0_materialise_kernel(const float *__restrict__ src, float *__re
 //    FP32 accumulation, over k-chunks of 32 through double-buffered LDS (one
 //    workgroup barrier per chunk; the loads of chunk c+1 are in flight while
 //    chunk c is multiplied);
-//  * the scene's scale comes from the largest |value| every kernel of the
-//    previous stage wrote (a per-scene atomic maximum in three rotating
-//    slots: stage k reads slot (k+2)%3, writes slot k%3 and clears slot
-//    (k+1)%3), so no pass over the inputs precedes the multiplication;
+//  * the scene's scale comes from the largest |value| every wavefront of the
+//    previous stage wrote (track_max, max_reduce), so no pass over the inputs
+//    precedes the multiplication;
 //  * pressure lines have n+1 outputs: the multiplication covers the first n,
 //    the last is an FP32 dot product of the raw line with D's last row,
 //    accumulated by the threads while they stage the line (its 128-wide
 //    output tiles then fit n exactly instead of wasting most of a tile).
-// X lines put U on the MFMA A side (rows of C = lines, columns = outputs),
-// Y lines put D there (rows = outputs, columns = lines), so that consecutive
-// lanes store consecutive floats in both directions.
+// U is on the MFMA A side (rows of C = lines, columns = outputs): consecutive
+// lanes store consecutive floats of a line, in both directions (vy and py are
+// stored column-major).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1085,48 +823,28 @@ struct GemmTile {
     int n_g;               // outputs the multiplication produces (n_out, or n_out - 1 with the dot row)
     int d_exp;             // D was stored as D * 2^d_exp
     int K;                 // line length
+    int slot;              // of the first wavefront's maximum (track_max)
     int dot_off;           // >= 0: ftab offset of D's last row (FP32): this tile writes output n_out - 1
 };
-
-// Per-scene maxima of |value| written in a stage: umax[(slot * n_scenes + scene) * 2 + class],
-// class 0 the pressure fields (px, py), class 1 the velocities; float bits.
-__device__ __forceinline__ void track_max(const StageArgs &a, int scene, int cls, float m) {
-    if (!a.umax) return;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if ((threadIdx.x & 63) == 0 && m > 0.f)
-        atomicMax(&a.umax[((size_t)a.slot_w * a.n_scenes + scene) * 2 + cls], __float_as_uint(m));
-}
 
 // Power of two that brings a line whose values are bounded by m below 2^15
 // (FP16 keeps both parts normal down to 2^-3 of that bound).
 __device__ __forceinline__ int gemm_scale_exp(const StageArgs &a, int scene, int vel) {
-    const unsigned bits = a.umax[((size_t)a.slot_r * a.n_scenes + scene) * 2 + (vel ? 1 : 0)];
+    const unsigned bits = a.umax[scene * 2 + (vel ? 1 : 0)];
     const float m = __uint_as_float(bits) * (vel ? 1.f : 2.f);  // p0 = px + py
     return m > 0.f ? min(max(14 - ilogbf(m), -100), 100) : 0;
 }
 
 // Raw input values of one chunk held by a thread: 8 consecutive k of one line
-// (X lines: 4 threads per line, so 4 lanes read 128 contiguous bytes of a row;
-// Y lines: one line per lane, so a wavefront reads 64 adjacent columns of a
-// row).  The second array of p0 = px + py is kept apart and added when the
-// chunk is converted, so that nothing waits for the loads of chunk c+2 before
-// the MFMAs of chunk c; dk: the FP32 dot row's coefficients of these k.
+// (4 threads per line, so 4 lanes read 128 contiguous bytes); dk: the FP32 dot
+// row's coefficients of these k.
 struct UChunk {
-    float a[kGSlots][8], b[kGSlots][8], dk[kGSlots][8];
+    float a[kGSlots][8], dk[kGSlots][8];
 };
 
-// Staging map of slot q: X lines 4 threads per line (lines tid/4 and tid/4 +
-// 64); Y lines one line per lane, the k-group that of the whole wavefront
-// (groups tid/128 and tid/128 + 2).
-template <int DIR>
-__device__ __forceinline__ int stage_line(int tid, int q) {
-    return DIR == 0 ? (tid >> 2) + q * (kGemmThreads / 4) : tid & (kGL - 1);
-}
-template <int DIR>
-__device__ __forceinline__ int stage_kq(int tid, int q) {
-    return DIR == 0 ? (tid & 3) * 8 : __builtin_amdgcn_readfirstlane((tid >> 7) + q * (kGemmThreads / kGL)) * 8;
-}
+// Staging map of slot q: 4 threads per line, lines tid/4 and tid/4 + 64.
+__device__ __forceinline__ int stage_line(int tid, int q) { return (tid >> 2) + q * (kGemmThreads / 4); }
+__device__ __forceinline__ int stage_kq(int tid) { return (tid & 3) * 8; }
 
 // raw buffer over `bytes` bytes at byte offset `byte_off` of `base`
 __device__ __forceinline__ Rsrc bytes_rsrc(const void *base, long long byte_off, int bytes) {
@@ -1140,43 +858,24 @@ __device__ __forceinline__ float4 bload4(Rsrc r, int off_bytes) {
 // Line `line` (absolute) of a tile: byte offsets of position k of its raw
 // input line in the three blocks it comes from (main, side1, side2).
 struct LineAddr {
-    int w, nm, vel, K;
-    int m_base, m_ps, s1_base, s1_ps, s2_base, s2_ps;  // offset of k = 0 of each piece, byte step per k
+    int w, nm, K;
+    int m_base, s1_base, s2_base;  // offset of k = 0 of each piece (4 bytes per k)
     bool s1, s2;
     __device__ LineAddr(const TileDesc &td, int line, int K_) {
+        const int vel = td.vel;
         w = td.wlen;
         nm = td.n_main;
-        vel = td.vel;
         K = K_;
-        m_ps = td.m_ps * 4;
-        m_base = (td.m_a + line * td.m_ls) * 4 - w * m_ps;
+        m_base = (td.m_a + line * td.m_ls - w) * 4;
         s1 = td.s1_len >= 0;
         s2 = td.s2_len >= 0;
-        s1_base = (td.s1_a + (line + td.s1_line) * td.s1_ls + (td.s1_len - w - vel) * td.s1_ps) * 4;
-        s1_ps = td.s1_ps * 4;
-        s2_base = (td.s2_a + (line + td.s2_line) * td.s2_ls + (vel - w - nm) * td.s2_ps) * 4;
-        s2_ps = td.s2_ps * 4;
+        s1_base = (td.s1_a + (line + td.s1_line) * td.s1_ls + td.s1_len - w - vel) * 4;
+        s2_base = (td.s2_a + (line + td.s2_line) * td.s2_ls + vel - w - nm) * 4;
     }
-    __device__ int main_off(int k) const { return k >= w && k < w + nm ? m_base + k * m_ps : kOOB; }
-    __device__ int s1_off(int k) const { return s1 && k < w ? s1_base + k * s1_ps : kOOB; }
-    __device__ int s2_off(int k) const { return s2 && k >= w + nm && k < K ? s2_base + k * s2_ps : kOOB; }
+    __device__ int main_off(int k) const { return k >= w && k < w + nm ? m_base + k * 4 : kOOB; }
+    __device__ int s1_off(int k) const { return s1 && k < w ? s1_base + k * 4 : kOOB; }
+    __device__ int s2_off(int k) const { return s2 && k >= w + nm && k < K ? s2_base + k * 4 : kOOB; }
 };
-
-// The arrays a tile's lines are read from: A (vx / vy for velocity lines, px
-// or the explicit p0 for pressure lines) and, for p0 = px + py, B (py).  The
-// three pieces of a line differ only in the domain block.
-struct GemmSrc {
-    const float *A, *B;
-    bool hasB;
-};
-
-__device__ __forceinline__ GemmSrc gemm_src(const StageArgs &a, const TileDesc &td) {
-    GemmSrc r;
-    r.A = td.vel ? a.vsrc : a.p0a;
-    r.hasB = !td.vel && a.p0b != nullptr;
-    r.B = r.hasB ? a.p0b : r.A;
-    return r;
-}
 
 // Which piece of the line a whole chunk [k0, k0 + kGK) lies in (the same for
 // every line of a tile).  kPieceS2 chunks may run past K: positions from K on
@@ -1192,69 +891,47 @@ __device__ __forceinline__ int chunk_piece(const TileDesc &td, int K, int k0) {
                                                 : kPieceMixed;
 }
 
-// Buffer resources (A, B arrays) of one piece's domain block.
 // (Selections are between values, never between struct members: a select of
 // member lvalues keeps the struct in scratch memory.)
 template <class T>
 __device__ __forceinline__ T pick3(int piece, T main, T s1, T s2) {
     return piece == kPieceMain ? main : piece == kPieceS1 ? s1 : s2;
 }
-__device__ __forceinline__ void piece_rsrc(const GemmSrc &src, const TileDesc &td, int piece, Rsrc &rA, Rsrc &rB) {
-    const long long dom = pick3<long long>(piece, td.m_dom, td.s1_dom, td.s2_dom);
-    const int size = pick3<int>(piece, td.m_size, td.s1_size, td.s2_size);
-    const int ab = pick3<int>(piece, td.m_b - td.m_a, td.s1_b - td.s1_a, td.s2_b - td.s2_a);
-    rA = block_rsrc(src.A, dom, size);
-    rB = block_rsrc(src.B, dom + ab, size - ab);
+// Buffer resource of one piece's domain block.
+__device__ __forceinline__ Rsrc piece_rsrc(const float *src, const TileDesc &td, int piece) {
+    return block_rsrc(src, pick3<long long>(piece, td.m_dom, td.s1_dom, td.s2_dom),
+                      pick3<int>(piece, td.m_size, td.s1_size, td.s2_size));
 }
 
-template <int DIR, bool HASB>
-__device__ __forceinline__ void gemm_load_u1(const GemmSrc &src, const TileDesc &td, const LineAddr &L, bool ok, int k0,
+__device__ __forceinline__ void gemm_load_u1(const float *src, const TileDesc &td, const LineAddr &L, bool ok, int k0,
                                              int q, Rsrc dotr, bool dot, UChunk &u) {
-    const int kb = k0 + stage_kq<DIR>(threadIdx.x, q);
+    const int kb = k0 + stage_kq(threadIdx.x);
     const int piece = chunk_piece(td, L.K, k0);
     if (piece == kPieceMixed) {
         // a chunk across a piece boundary: each value from whichever block holds it
-        Rsrc mA, mB, s1A, s1B, s2A, s2B;
-        piece_rsrc(src, td, kPieceMain, mA, mB);
-        piece_rsrc(src, td, kPieceS1, s1A, s1B);
-        piece_rsrc(src, td, kPieceS2, s2A, s2B);
+        const Rsrc m = piece_rsrc(src, td, kPieceMain), s1 = piece_rsrc(src, td, kPieceS1),
+                   s2 = piece_rsrc(src, td, kPieceS2);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int k = kb + j;
             const int om = ok ? L.main_off(k) : kOOB, o1 = ok ? L.s1_off(k) : kOOB, o2 = ok ? L.s2_off(k) : kOOB;
-            u.a[q][j] = bload(mA, om) + bload(s1A, o1) + bload(s2A, o2);
-            u.b[q][j] = HASB ? bload(mB, om) + bload(s1B, o1) + bload(s2B, o2) : 0.f;
+            u.a[q][j] = bload(m, om) + bload(s1, o1) + bload(s2, o2);
         }
     } else {
         // one block for the whole chunk
-        Rsrc rA, rB;
-        piece_rsrc(src, td, piece, rA, rB);
+        const Rsrc r = piece_rsrc(src, td, piece);
         const bool in = ok && (piece == kPieceMain || (piece == kPieceS1 && L.s1) || (piece == kPieceS2 && L.s2));
         const int base = pick3<int>(piece, L.m_base, L.s1_base, L.s2_base);
-        const int ps = pick3<int>(piece, L.m_ps, L.s1_ps, L.s2_ps);
-        const int off = in && piece != kPieceNone ? base + kb * ps : kOOB;
-        if (DIR == 0 && piece != kPieceS2) {
-            // X lines inside a row: two 16-byte loads per array
-            const float4 x0 = bload4(rA, off), x1 = bload4(rA, off == kOOB ? kOOB : off + 16);
+        const int off = in && piece != kPieceNone ? base + kb * 4 : kOOB;
+        if (piece != kPieceS2) {
+            // inside a line: two 16-byte loads
+            const float4 x0 = bload4(r, off), x1 = bload4(r, off == kOOB ? kOOB : off + 16);
             u.a[q][0] = x0.x; u.a[q][1] = x0.y; u.a[q][2] = x0.z; u.a[q][3] = x0.w;
             u.a[q][4] = x1.x; u.a[q][5] = x1.y; u.a[q][6] = x1.z; u.a[q][7] = x1.w;
-            if constexpr (HASB) {
-                const float4 y0 = bload4(rB, off), y1 = bload4(rB, off == kOOB ? kOOB : off + 16);
-                u.b[q][0] = y0.x; u.b[q][1] = y0.y; u.b[q][2] = y0.z; u.b[q][3] = y0.w;
-                u.b[q][4] = y1.x; u.b[q][5] = y1.y; u.b[q][6] = y1.z; u.b[q][7] = y1.w;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) u.b[q][j] = 0.f;
-            }
         } else {
-            // Y lines (a wavefront reads a row segment per k), or the side-2
-            // chunks of X lines (they may run to the end of the block): 4-byte loads
+            // side-2 chunks may run to the end of the block: 4-byte loads
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int o = off == kOOB || kb + j >= L.K ? kOOB : off + j * ps;
-                u.a[q][j] = bload(rA, o);
-                u.b[q][j] = HASB ? bload(rB, o) : 0.f;
-            }
+            for (int j = 0; j < 8; ++j) u.a[q][j] = bload(r, off == kOOB || kb + j >= L.K ? kOOB : off + j * 4);
         }
     }
     if (dot) {
@@ -1263,11 +940,10 @@ __device__ __forceinline__ void gemm_load_u1(const GemmSrc &src, const TileDesc 
     }
 }
 
-template <int DIR, bool HASB>
-__device__ __forceinline__ void gemm_load_u(const GemmSrc &src, const TileDesc &td, const LineAddr (&L)[kGSlots],
+__device__ __forceinline__ void gemm_load_u(const float *src, const TileDesc &td, const LineAddr (&L)[kGSlots],
                                             const bool (&ok)[kGSlots], int k0, Rsrc dotr, bool dot, UChunk &u) {
 #pragma unroll
-    for (int q = 0; q < kGSlots; ++q) gemm_load_u1<DIR, HASB>(src, td, L[q], ok[q], k0, q, dotr, dot, u);
+    for (int q = 0; q < kGSlots; ++q) gemm_load_u1(src, td, L[q], ok[q], k0, q, dotr, dot, u);
 }
 
 // Main-piece addressing of a tile's lines: every k of a main chunk lies in the
@@ -1276,63 +952,33 @@ __device__ __forceinline__ void gemm_load_u(const GemmSrc &src, const TileDesc &
 // chunk's k, passed as the buffer instruction's scalar offset).  Both parts
 // are non-negative.
 struct MainU {
-    Rsrc rA, rB;
+    Rsrc r;
     int voff[kGSlots];  // per lane and slot
-    int ps;    // bytes per k
-    int kofs;  // k of the first main position (the line's halo length)
+    int kofs;           // k of the first main position (the line's halo length)
 };
 
-template <int DIR, bool HASB>
-__device__ __forceinline__ MainU main_u(const GemmSrc &src, const TileDesc &td, const bool (&ok)[kGSlots]) {
+__device__ __forceinline__ MainU main_u(const float *src, const TileDesc &td, const bool (&ok)[kGSlots]) {
     MainU m;
-    m.rA = block_rsrc(src.A, td.m_dom, td.m_size);
-    m.rB = block_rsrc(src.B, td.m_dom + (td.m_b - td.m_a), td.m_size - (td.m_b - td.m_a));
-    m.ps = td.m_ps * 4;
+    m.r = block_rsrc(src, td.m_dom, td.m_size);
     m.kofs = td.wlen;
 #pragma unroll
     for (int q = 0; q < kGSlots; ++q) {
-        const int line = td.line0 + stage_line<DIR>(threadIdx.x, q);
-        m.voff[q] = ok[q] ? (td.m_a + line * td.m_ls) * 4 + stage_kq<DIR>(threadIdx.x, q) * m.ps : kOOB;
+        const int line = td.line0 + stage_line(threadIdx.x, q);
+        m.voff[q] = ok[q] ? (td.m_a + line * td.m_ls + stage_kq(threadIdx.x)) * 4 : kOOB;
     }
     return m;
 }
 
-template <int DIR, bool HASB>
 __device__ __forceinline__ void gemm_load_u_main(const MainU &m, int k0, Rsrc dotr, bool dot, UChunk &u) {
-    const int kk = k0 - m.kofs;  // >= 0 in a main chunk
+    const int so = (k0 - m.kofs) * 4;  // >= 0 in a main chunk
 #pragma unroll
     for (int q = 0; q < kGSlots; ++q) {
-        if constexpr (DIR == 0) {
-            // X lines (element stride 1): two 16-byte loads per array
-            const int so = kk * 4;
-            const float4 x0 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.rA, m.voff[q], so, 0));
-            const float4 x1 =
-                __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.rA, m.voff[q] + 16, so, 0));
-            u.a[q][0] = x0.x; u.a[q][1] = x0.y; u.a[q][2] = x0.z; u.a[q][3] = x0.w;
-            u.a[q][4] = x1.x; u.a[q][5] = x1.y; u.a[q][6] = x1.z; u.a[q][7] = x1.w;
-            if constexpr (HASB) {
-                const float4 y0 =
-                    __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.rB, m.voff[q], so, 0));
-                const float4 y1 =
-                    __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.rB, m.voff[q] + 16, so, 0));
-                u.b[q][0] = y0.x; u.b[q][1] = y0.y; u.b[q][2] = y0.z; u.b[q][3] = y0.w;
-                u.b[q][4] = y1.x; u.b[q][5] = y1.y; u.b[q][6] = y1.z; u.b[q][7] = y1.w;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) u.b[q][j] = 0.f;
-            }
-        } else {
-            // Y lines: a wavefront reads 64 adjacent columns of a row per k
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int so = (kk + j) * m.ps;
-                u.a[q][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(m.rA, m.voff[q], so, 0));
-                u.b[q][j] =
-                    HASB ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(m.rB, m.voff[q], so, 0)) : 0.f;
-            }
-        }
+        const float4 x0 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.r, m.voff[q], so, 0));
+        const float4 x1 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.r, m.voff[q] + 16, so, 0));
+        u.a[q][0] = x0.x; u.a[q][1] = x0.y; u.a[q][2] = x0.z; u.a[q][3] = x0.w;
+        u.a[q][4] = x1.x; u.a[q][5] = x1.y; u.a[q][6] = x1.z; u.a[q][7] = x1.w;
         if (dot) {
-            const int kb = k0 + stage_kq<DIR>(threadIdx.x, q);
+            const int kb = k0 + stage_kq(threadIdx.x);
 #pragma unroll
             for (int j = 0; j < 8; ++j) u.dk[q][j] = bload(dotr, (kb + j) * 4);
         }
@@ -1352,7 +998,7 @@ __device__ __forceinline__ void gemm_dma_d(const Rsrc &dr, void *dbuf, int c) {
 // Converts and writes one chunk into LDS buffer `buf` (8 k of one line per
 // thread as one 16-byte write per part); accumulates the FP32 dot product of
 // the last output row (dot).
-template <typename E, int DIR, bool HASB>
+template <typename E>
 __device__ __forceinline__ void gemm_stage(E *ulds, int buf, const UChunk &u, float sc, bool dot,
                                            float (&gv)[kGSlots]) {
     using V8 = typename MfmaOps<E>::v8;
@@ -1360,12 +1006,11 @@ __device__ __forceinline__ void gemm_stage(E *ulds, int buf, const UChunk &u, fl
     E *U0 = ulds + (buf * 2 + 0) * kGL * kGP, *U1 = ulds + (buf * 2 + 1) * kGL * kGP;
 #pragma unroll
     for (int q = 0; q < kGSlots; ++q) {
-        const int row = stage_line<DIR>(tid, q), kq = stage_kq<DIR>(tid, q);
+        const int row = stage_line(tid, q), kq = stage_kq(tid);
         V8 hi, lo;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float raw = HASB ? u.a[q][j] + u.b[q][j] : u.a[q][j];
-            const float x = raw * sc;
+            const float x = u.a[q][j] * sc;
             const E h = (E)x;
             hi[j] = h;
             lo[j] = (E)(x - (float)h);
@@ -1379,52 +1024,52 @@ __device__ __forceinline__ void gemm_stage(E *ulds, int buf, const UChunk &u, fl
         for (int q = 0; q < kGSlots; ++q)
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                gv[q] = __builtin_fmaf(HASB ? u.a[q][j] + u.b[q][j] : u.a[q][j], u.dk[q][j], gv[q]);
+                gv[q] = __builtin_fmaf(u.a[q][j], u.dk[q][j], gv[q]);
     }
 }
 
 // The MFMAs of one chunk (LDS buffer `buf`): wave (lg, og) accumulates lines
 // 64 lg .. +63 x outputs 64 og .. +63 (2 x 2 blocks of 32 x 32).
-template <typename E, int DIR>
-__device__ __forceinline__ void gemm_chunk(const E *ulds, const E *dlds, int buf, int lg, int og, f32x16 (&acc)[2][2]) {
+template <typename E>
+__device__ __forceinline__ void gemm_chunk(const E *ulds, const E *dlds, int buf, int lg, int og, int dir,
+                                           f32x16 (&acc)[2][2]) {
     using V8 = typename MfmaOps<E>::v8;
     const int lane = threadIdx.x & 63;
     const E *U0 = ulds + (buf * 2 + 0) * kGL * kGP, *U1 = ulds + (buf * 2 + 1) * kGL * kGP;
     const E *D0 = dlds + (buf * 2 + 0) * kGN * kGP, *D1 = dlds + (buf * 2 + 1) * kGN * kGP;
-    // rows of C from R (U for X, D for Y) at r_base, columns from Q at q_base
-    const E *R0 = DIR == 0 ? U0 : D0, *R1 = DIR == 0 ? U1 : D1;
-    const E *Q0 = DIR == 0 ? D0 : U0, *Q1 = DIR == 0 ? D1 : U1;
-    const int r_base = DIR == 0 ? 64 * lg : 64 * og, q_base = DIR == 0 ? 64 * og : 64 * lg;
 #pragma unroll
     for (int s = 0; s < kGK / 16; ++s) {
         const int kk = s * 16 + (lane >> 5) * 8;
         V8 ah[2], al[2], bh[2], bl[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int rr = (r_base + 32 * i + (lane & 31)) * kGP + kk, qq = (q_base + 32 * i + (lane & 31)) * kGP + kk;
-            ah[i] = *reinterpret_cast<const V8 *>(R0 + rr);
-            al[i] = *reinterpret_cast<const V8 *>(R1 + rr);
-            bh[i] = *reinterpret_cast<const V8 *>(Q0 + qq);
-            bl[i] = *reinterpret_cast<const V8 *>(Q1 + qq);
+            const int rr = (64 * lg + 32 * i + (lane & 31)) * kGP + kk, qq = (64 * og + 32 * i + (lane & 31)) * kGP + kk;
+            ah[i] = *reinterpret_cast<const V8 *>(U0 + rr);
+            al[i] = *reinterpret_cast<const V8 *>(U1 + rr);
+            bh[i] = *reinterpret_cast<const V8 *>(D0 + qq);
+            bl[i] = *reinterpret_cast<const V8 *>(D1 + qq);
         }
         // each product over the four independent accumulators in turn (no
-        // back-to-back MFMAs on one accumulator)
+        // back-to-back MFMAs on one accumulator); the low parts of D first for X
+        // lines, those of U for Y lines (a fixed order of the sums per direction)
+        auto product = [&](const V8 (&x)[2], const V8 (&y)[2]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = MfmaOps<E>::mfma(ah[i], bh[j], acc[i][j]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = MfmaOps<E>::mfma(ah[i], bl[j], acc[i][j]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = MfmaOps<E>::mfma(al[i], bh[j], acc[i][j]);
+                for (int j = 0; j < 2; ++j) acc[i][j] = MfmaOps<E>::mfma(x[i], y[j], acc[i][j]);
+        };
+        product(ah, bh);
+        if (dir == 0) {
+            product(ah, bl);
+            product(al, bh);
+        } else {
+            product(al, bh);
+            product(ah, bl);
+        }
     }
 }
 
-template <typename E, int DIR, bool HASB>
+template <typename E>
 __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt, const float *ftab,
                                           unsigned char *gemm_lds) {
     E *ulds = reinterpret_cast<E *>(gemm_lds);
@@ -1433,16 +1078,16 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lg = wave >> 1, og = wave & 1;
     const int e = gemm_scale_exp(a, td.scene, td.vel);
     const float sc = ldexpf(1.f, e);
-    const GemmSrc r = gemm_src(a, td);
+    const float *src = source(a, td.vel);
     const Rsrc dr = bytes_rsrc(a.dmat, gt.d_img * 2, (int)(gt.d_len * 2));
     const bool dot = gt.dot_off >= 0;
     const Rsrc dotr = bytes_rsrc(ftab, dot ? (long long)gt.dot_off * 4 : 0, dot ? gt.K * 4 : 0);
     const int nch = gt.k_pad / kGK;
     bool line_ok[kGSlots];
 #pragma unroll
-    for (int q = 0; q < kGSlots; ++q) line_ok[q] = stage_line<DIR>(tid, q) < td.count;
-    const LineAddr L[kGSlots] = {LineAddr(td, td.line0 + stage_line<DIR>(tid, 0), gt.K),
-                                 LineAddr(td, td.line0 + stage_line<DIR>(tid, 1), gt.K)};
+    for (int q = 0; q < kGSlots; ++q) line_ok[q] = stage_line(tid, q) < td.count;
+    const LineAddr L[kGSlots] = {LineAddr(td, td.line0 + stage_line(tid, 0), gt.K),
+                                 LineAddr(td, td.line0 + stage_line(tid, 1), gt.K)};
     // waves whose lines or outputs lie outside the tile skip their MFMAs
     const bool active = 64 * lg < td.count && 64 * og < gt.n_g - gt.n0;
     f32x16 acc[2][2];
@@ -1457,9 +1102,9 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
     // barrier that makes chunk c visible, and are in flight while the MFMAs of
     // chunk c run; then chunk c+1 is converted into the other LDS buffer.
     UChunk u;
-    gemm_load_u<DIR, HASB>(r, td, L, line_ok, 0, dotr, dot, u);
+    gemm_load_u(src, td, L, line_ok, 0, dotr, dot, u);
     gemm_dma_d(dr, dlds, 0);
-    gemm_stage<E, DIR, HASB>(ulds, 0, u, sc, dot, gv);
+    gemm_stage<E>(ulds, 0, u, sc, dot, gv);
     __syncthreads();
     // Chunks whose every k lies in the main piece, [cm0, cm1), load through
     // MainU (no per-chunk piece logic); the halo chunks around them through
@@ -1471,23 +1116,23 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
         load_next((c + 1) * kGK);
         // D of chunk c + 1 into the other buffer (read last before the previous barrier)
         gemm_dma_d(dr, dlds + (buf ^ 1) * kGemmDChunk, c + 1);
-        if (active) gemm_chunk<E, DIR>(ulds, dlds, buf, lg, og, acc);
-        gemm_stage<E, DIR, HASB>(ulds, buf ^ 1, u, sc, dot, gv);
+        if (active) gemm_chunk<E>(ulds, dlds, buf, lg, og, td.dir, acc);
+        gemm_stage<E>(ulds, buf ^ 1, u, sc, dot, gv);
         __syncthreads();  // also waits for the D copy
         ++c;
     };
-    auto generic = [&](int k0) { gemm_load_u<DIR, HASB>(r, td, L, line_ok, k0, dotr, dot, u); };
+    auto generic = [&](int k0) { gemm_load_u(src, td, L, line_ok, k0, dotr, dot, u); };
     while (c + 1 < min(cm0, nch)) step(generic);
     {
-        const MainU m = main_u<DIR, HASB>(r, td, line_ok);
+        const MainU m = main_u(src, td, line_ok);
         // the same step with the LDS buffer parity known at compile time
         // (LDS addresses as immediate offsets): two chunks per iteration
         auto step_p = [&](auto parity) {
             constexpr int buf = decltype(parity)::value;
-            gemm_load_u_main<DIR, HASB>(m, (c + 1) * kGK, dotr, dot, u);
+            gemm_load_u_main(m, (c + 1) * kGK, dotr, dot, u);
             gemm_dma_d(dr, dlds + (buf ^ 1) * kGemmDChunk, c + 1);
-            if (active) gemm_chunk<E, DIR>(ulds, dlds, buf, lg, og, acc);
-            gemm_stage<E, DIR, HASB>(ulds, buf ^ 1, u, sc, dot, gv);
+            if (active) gemm_chunk<E>(ulds, dlds, buf, lg, og, td.dir, acc);
+            gemm_stage<E>(ulds, buf ^ 1, u, sc, dot, gv);
             __syncthreads();
             ++c;
         };
@@ -1501,7 +1146,7 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
         if (c + 1 < cm1) step_p(P0{});
     }
     while (c + 1 < nch) step(generic);
-    if (active) gemm_chunk<E, DIR>(ulds, dlds, c & 1, lg, og, acc);
+    if (active) gemm_chunk<E>(ulds, dlds, c & 1, lg, og, td.dir, acc);
     __syncthreads();
     // epilogue: L = C / (2^e 2^d_exp); out = t_n - s*coef*L (Solver::update_field_values)
     const float sc_upd = a.s * td.coef, inv = ldexpf(1.f, -(e + gt.d_exp));
@@ -1513,25 +1158,20 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
     if (active) {
         // value q of block (i, j): row 32 i + 8 (q >> 2) + 4 (lane >> 5) + (q & 3), column 32 j + (lane & 31)
         // of the wave's 64 x 64; all t_n loads are issued before the first is used
-        const int lrow0 = DIR == 0 ? 64 * lg + 4 * (lane >> 5) : 64 * lg + (lane & 31);
-        const int nrow0 = gt.n0 + (DIR == 0 ? 64 * og + (lane & 31) : 64 * og + 4 * (lane >> 5));
+        const int lrow0 = 64 * lg + 4 * (lane >> 5), nrow0 = gt.n0 + 64 * og + (lane & 31);
         auto offset = [&](int i, int j, int q, bool &ok) {
-            const int rowd = 32 * i + 8 * (q >> 2) + (q & 3), cold = 32 * j;
-            const int line = lrow0 + (DIR == 0 ? rowd : cold), n = nrow0 + (DIR == 0 ? cold : rowd);
+            const int line = lrow0 + 32 * i + 8 * (q >> 2) + (q & 3), n = nrow0 + 32 * j;
             ok = line < td.count && n < gt.n_g;
-            return ok ? (td.o_f + (td.line0 + line) * td.o_ls + n * td.o_ps) * 4 : kOOB;
+            return ok ? (td.o_f + (td.line0 + line) * td.o_ls + n) * 4 : kOOB;
         };
         float tnv[2][2][16];
         if (64 * lg + 64 <= td.count && 64 * og + 64 <= gt.n_g - gt.n0) {
             // the wave's whole 64 x 64 block lies inside the tile: a per-lane
             // offset and, per value, a uniform one (the buffer instruction's
             // scalar offset; no address arithmetic on the vector unit)
-            const int base = (td.o_f + (td.line0 + lrow0) * td.o_ls + nrow0 * td.o_ps) * 4;
-            const int sl = td.o_ls * 4, sp = td.o_ps * 4;
-            auto uoff = [&](int i, int j, int q) {
-                const int rowd = 32 * i + 8 * (q >> 2) + (q & 3), cold = 32 * j;
-                return DIR == 0 ? rowd * sl + cold * sp : cold * sl + rowd * sp;
-            };
+            const int base = (td.o_f + (td.line0 + lrow0) * td.o_ls + nrow0) * 4;
+            const int sl = td.o_ls * 4;
+            auto uoff = [&](int i, int j, int q) { return (32 * i + 8 * (q >> 2) + (q & 3)) * sl + 128 * j; };
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1576,8 +1216,8 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
                         bool ok;
                         const int off = offset(i, j, q, ok);
                         const float nv = __builtin_fmaf(-sc_upd, acc[i][j][q] * inv, tnv[i][j][q]);
-                        bstore(ro, off, nv);
-                        if (a.last) bstore(rt, off, nv * (use_pml ? bload(rp, off) : 1.f));
+                        bstore(ro, off, 0, nv);
+                        if (a.last) bstore(rt, off, 0, nv * (use_pml ? bload(rp, off) : 1.f));
                         if (ok) mx = fmaxf(mx, fabsf(nv));
                     }
         }
@@ -1587,60 +1227,37 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
         const int n = gt.n_g;
         auto write_dot = [&](int line, float Ldot) {
             if (line < 0 || line >= td.count) return;
-            const int off = (td.o_f + (td.line0 + line) * td.o_ls + n * td.o_ps) * 4;
+            const int off = (td.o_f + (td.line0 + line) * td.o_ls + n) * 4;
             const float tnv = bload(rt, off), pm = use_pml ? bload(rp, off) : 1.f;
             const float nv = __builtin_fmaf(-sc_upd, Ldot, tnv);
-            bstore(ro, off, nv);
-            if (a.last) bstore(rt, off, nv * pm);
+            bstore(ro, off, 0, nv);
+            if (a.last) bstore(rt, off, 0, nv * pm);
             mx = fmaxf(mx, fabsf(nv));
         };
-        if constexpr (DIR == 0) {
-            // the 4 threads of a line are adjacent lanes; slot q holds line tid/4 + 64 q
+        // the 4 threads of a line are adjacent lanes; slot q holds line tid/4 + 64 q
 #pragma unroll
-            for (int q = 0; q < kGSlots; ++q) {
-                float g = gv[q];
-                g += __shfl_xor(g, 1);
-                g += __shfl_xor(g, 2);
-                write_dot((tid & 3) == 0 ? stage_line<DIR>(tid, q) : -1, g);
-            }
-        } else {
-            // partial sums of the 4 k-groups (2 per thread) through LDS (the ring is no longer read)
-            float *red = reinterpret_cast<float *>(gemm_lds);
-            red[(tid >> 7) * kGL + (tid & (kGL - 1))] = gv[0] + gv[1];
-            __syncthreads();
-            float Ldot = 0.f;
-            if (tid < kGL) {
-#pragma unroll
-                for (int k = 0; k < kGemmThreads / kGL; ++k) Ldot += red[k * kGL + tid];
-            }
-            write_dot(tid < kGL ? tid : -1, Ldot);
+        for (int q = 0; q < kGSlots; ++q) {
+            float g = gv[q];
+            g += __shfl_xor(g, td.dir == 0 ? 1 : 2);
+            g += __shfl_xor(g, td.dir == 0 ? 2 : 1);
+            write_dot((tid & 3) == 0 ? stage_line(tid, q) : -1, g);
         }
     }
-    track_max(a, td.scene, td.vel ? 0 : 1, mx);
+    track_max(a, gt.slot, mx);
 }
 
 template <typename E>
 __global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2))) stage_gemm_kernel(StageArgs a, const GemmTile *__restrict__ tiles,
                                                                   const float *__restrict__ ftab) {
-    // clears the slot the next stage writes (nothing reads or writes it in this stage)
-    if (blockIdx.x == 0 && a.umax)
-        for (int i = threadIdx.x; i < 2 * a.n_scenes; i += blockDim.x) a.umax[(size_t)a.slot_z * a.n_scenes * 2 + i] = 0u;
     extern __shared__ __attribute__((aligned(16))) unsigned char gemm_lds[];
     // XCD-contiguous runs of tiles always (the tiles of one matrix and of one
     // line block share an XCD's L2), whatever order the FFT-form tiles use
     const GemmTile gt = tiles[tile_index(blockIdx.x, gridDim.x, 1)];
-    const bool hasB = !gt.t.vel && a.p0b != nullptr;  // p0 = px + py
-    if (gt.t.dir == 0) {
-        if (hasB) gemm_tile<E, 0, true>(a, gt, ftab, gemm_lds);
-        else gemm_tile<E, 0, false>(a, gt, ftab, gemm_lds);
-    } else {
-        if (hasB) gemm_tile<E, 1, true>(a, gt, ftab, gemm_lds);
-        else gemm_tile<E, 1, false>(a, gt, ftab, gemm_lds);
-    }
+    gemm_tile<E>(a, gt, ftab, gemm_lds);
 }
 
 // Largest |p0| and |vx|, |vy| of every scene in the state a first stage reads
-// after the host wrote fields (it has no previous stage): into slot `slot`.
+// after the host wrote fields (it has no previous stage).
 struct MaxRange {
     long long off;  // element offset from the arena base
     long long n;
@@ -1652,7 +1269,7 @@ __global__ void fill_zero_kernel(unsigned *__restrict__ p, int n) {
 }
 
 __global__ void state_max_kernel(const float *__restrict__ arena, unsigned *__restrict__ umax,
-                                 const MaxRange *__restrict__ ranges, int nr, int n_scenes, int slot) {
+                                 const MaxRange *__restrict__ ranges, int nr) {
     for (int k = blockIdx.y; k < nr; k += gridDim.y) {
         const MaxRange r = ranges[k];
         float m = 0.f;
@@ -1660,7 +1277,7 @@ __global__ void state_max_kernel(const float *__restrict__ arena, unsigned *__re
             m = fmaxf(m, fabsf(arena[r.off + e]));
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-        if ((threadIdx.x & 63) == 0 && m > 0.f) atomicMax(&umax[(size_t)slot * n_scenes * 2 + r.idx], __float_as_uint(m));
+        if ((threadIdx.x & 63) == 0 && m > 0.f) atomicMax(&umax[r.idx], __float_as_uint(m));
     }
 }
 
@@ -1686,6 +1303,20 @@ int next_pow2(int n) {
 // Time steps per captured hipGraph unless pstd_ctx_set_graph_steps says otherwise.
 constexpr int kDefaultGraphSteps = 20;
 
+// p0 on the fly or in a pass of its own: the pass moves 16 bytes per cell and costs
+// a launch (5 us); on the fly, a tile of n adjacent lines reads 4 n bytes of every
+// 64-byte sector the other layout's field has in it.  The pass is taken where the
+// fly moves this many bytes per stage more (about 5 us at 4 TB/s).  Measured, us
+// per stage on the fly / with the pass: 333 000 cells 12.8 / 19.7, one 900^2 domain
+// 24.3 / 27.1, 1024^2 32.9 / 32.9, 1200^2 37.5 / 36.5, 1500^2 49.5 / 43.9, 4096^2
+// 406 / 352, 16 sources of 512 x 1024 twice 368 / 362; twelve scenes of lines up to
+// 600 (at least 8 lines per tile) 111 / 117.
+constexpr long long kP0PassBytes = 20000000;
+// 64-byte sectors read per 64 bytes used by a tile's strided reads (256 threads)
+static int strided_factor(int F) {
+    return std::max(1, 16 / std::max(2, 2 * 256 / (F / fft_values(F))));
+}
+
 struct pstd_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -1702,13 +1333,16 @@ struct pstd_ctx {
     // plan
     std::vector<DomainDev> doms;
     std::vector<pstd_plan_domain> plan_domains;
-    std::vector<TileDesc> tiles_small, tiles_4096, tiles_8192;
-    // FFT-form segments (line0/count = the segment's line range) and the
-    // passthrough/receiver tiles: the tile lists are cut from them for the
-    // block size of the F <= 2048 class (small_nt, autotuned: 256 or 512)
-    std::vector<TileDesc> fft_segs, tiles_extra, tiles_all;
-    int small_nt = 256;
+    // FFT-form segments (line0/count = the segment's line range), passthrough
+    // fields and the receivers: the tile list is cut from them for the block size
+    // (stage_threads)
+    std::vector<TileDesc> fft_segs;
+    int n_tiles = 0;
+    int small_nt = 256;  // block size where the lines leave the choice (autotuned: 128 or 256)
     int small_fmax = 0;  // largest F of the F <= 2048 class (128 threads need F <= 1024)
+    int fmax = 0;        // largest F
+    // block size of the stage launch: the threads of one line pair
+    int stage_threads() const { return std::max(small_nt, fmax / fft_values(fmax)); }
     std::vector<GemmTile> tiles_gemm;
     int n_scenes = 1;
     std::vector<MaxRange> max_ranges;  // state read by a first stage after host writes (GEMM form)
@@ -1725,10 +1359,14 @@ struct pstd_ctx {
     float *pml = nullptr;
     float2 *ctab = nullptr;
     float *ftab = nullptr;
-    TileDesc *d_tiles = nullptr;  // small | 4096 | 8192
+    TileDesc *d_segs = nullptr;
+    TileRef *d_tiles = nullptr;
     GemmTile *d_gemm = nullptr;
     void *dmat = nullptr;         // derivative matrices of the GEMM form (hi, lo parts; 2-byte elements)
-    unsigned *umax = nullptr;     // per-scene maxima of the written values, 3 slots x scenes x 2 classes
+    unsigned *umax = nullptr;     // maxima of the written values, scenes x 2 classes
+    float *wmax = nullptr;        // per wavefront (track_max): the FFT-form tiles' slots, then the GEMM tiles'
+    int2 *d_max_first = nullptr;
+    std::vector<int> gemm_first;  // first GEMM slot of every group (scene, class), then their number
     MaxRange *d_max_ranges = nullptr;
     ReceiverCell *d_cells = nullptr;
     // spectral receivers: line jobs, per-receiver jobs, weights, column buffer
@@ -1737,14 +1375,17 @@ struct pstd_ctx {
     float *d_si_coef = nullptr;
     float *d_si_col = nullptr;
     int n_si_lines = 0, n_si = 0;
-    P0Range *d_ranges = nullptr;
-    int n_ranges = 0;
+    P0Tile *d_p0_tiles = nullptr;
+    std::vector<int> p0_first;   // first tile of every domain, then the number of tiles
+    // p0 is formed by p0_pass_kernel after every stage (P0I then always holds the
+    // current p0), otherwise by the tiles that read it
+    bool p0_pass = false;
     float *d_samples = nullptr;
     int sample_cap = 0;
     int steps_done = 0;
     bool p0_explicit = true;
     int xcd_remap = 1;
-    int lean = 0;  // stage kernel flavour (kEarly, kLate, kMid)
+    int lean = 1;  // stage kernel flavour as set (0 early, 1 late, 2 mid): one kernel serves them all
     float tuned_stage_ms = 0;
     // the GEMM form's maxima in `umax` no longer describe the state (an
     // allocation-free advance used the shared array): recompute before the next step
@@ -1785,9 +1426,14 @@ struct pstd_ctx {
         (void)hipFree(ctab);
         (void)hipFree(ftab);
         (void)hipFree(d_tiles);
+        (void)hipFree(d_segs);
         (void)hipFree(d_gemm);
         (void)hipFree(dmat);
         (void)hipFree(umax);
+        (void)hipFree(wmax);
+        (void)hipFree(d_max_first);
+        wmax = nullptr;
+        d_max_first = nullptr;
         (void)hipFree(d_max_ranges);
         d_gemm = nullptr;
         dmat = nullptr;
@@ -1802,13 +1448,14 @@ struct pstd_ctx {
         d_si_points = nullptr;
         d_si_coef = d_si_col = nullptr;
         n_si_lines = n_si = 0;
-        (void)hipFree(d_ranges);
+        (void)hipFree(d_p0_tiles);
         (void)hipFree(d_samples);
         arena = pml = ftab = d_samples = nullptr;
         ctab = nullptr;
         d_tiles = nullptr;
+        d_segs = nullptr;
         d_cells = nullptr;
-        d_ranges = nullptr;
+        d_p0_tiles = nullptr;
         planned = false;
     }
 };
@@ -1819,15 +1466,31 @@ namespace {
 void build_filter(int F, int L, int field, double dx, std::vector<float2> &out) {
     const std::vector<std::complex<double>> h = pstdamd::derivative_filter(F, L, field, dx);
     out.resize(F);
-    for (int m = 0; m < F; ++m) out[m] = make_float2((float)h[m].real(), (float)h[m].imag());
+    // thread t's values t + m T in pairs of m, [m / 2][t][m % 2]; length 8192: the even
+    // and the odd bin of t + 512 m, [m][t][bin % 2]
+    const int T = F / fft_values(F);
+    for (int k = 0; k < F; ++k) {
+        const int m = k / T, t = k % T;
+        out[F == 8192 ? k : ((m / 2) * T + t) * 2 + m % 2] = make_float2((float)h[k].real(), (float)h[k].imag());
+    }
 }
 
+// The tables of fft_line.h.
 void build_twiddles(int F, std::vector<float2> &out) {
-    out.resize(F);
-    for (int i = 0; i < F; ++i) {
-        double a = -2.0 * M_PI * (double)i / (double)F;
-        out[i] = make_float2((float)std::cos(a), (float)std::sin(a));
-    }
+    out.clear();
+    auto root = [](int i, int n) {
+        const double a = -2.0 * M_PI * (double)i / (double)n;
+        return make_float2((float)std::cos(a), (float)std::sin(a));
+    };
+    const int Fp = std::min(F, 4096);
+    for (int p = 1; p < fft_npasses(Fp); ++p)
+        for (int r = 0; r < fft_radix(Fp, p); r += 2)
+            for (int k = 0; k < fft_span(Fp, p); ++k)
+                for (int q = r; q < r + 2; ++q) out.push_back(root(q * k * (Fp / (fft_span(Fp, p) * fft_radix(Fp, p))), Fp));
+    if (F == 8192)
+        for (int m = 0; m < 8; m += 2)
+            for (int t = 0; t < 512; ++t)
+                for (int q = m; q < m + 2; ++q) out.push_back(root(t + 512 * q, F));
 }
 
 void build_window(int w, int patch_error, std::vector<float> &out) {
@@ -1835,8 +1498,14 @@ void build_window(int w, int patch_error, std::vector<float> &out) {
     out.assign(win.begin(), win.end());
 }
 
-// Kernel classes of pstd_ctx_profile_kernels.
+// Kernel classes of pstd_ctx_profile_kernels: the FFT-form launch counts for the
+// class of its longest lines.
 constexpr int kClassSmall = 0, kClass4096 = 1, kClass8192 = 2, kClassGemm = 3, kClasses = 4;
+
+typedef void (*StageKernel)(StageArgs);
+StageKernel stage_kernel(int nt) {
+    return nt <= 128 ? stage_fft_kernel<128> : nt <= 256 ? stage_fft_kernel<256> : stage_fft_kernel<512>;
+}
 
 // Brackets the launches issued by `launch` with an event pair when profiling.
 template <class Fn>
@@ -1863,20 +1532,9 @@ int launch_stage(pstd_ctx *ctx, int k, int sample_slot) {
     a.ctab = ctx->ctab;
     a.ftab = ctx->ftab;
     const int in = (k + 1) & 1, outi = k & 1;
-    if (k == 0) {
-        if (ctx->p0_explicit) {
-            a.p0a = ctx->P0I();
-            a.p0b = nullptr;
-        } else {
-            a.p0a = ctx->S(1);
-            a.p0b = ctx->S(1);
-        }
-        a.vsrc = ctx->TN();
-    } else {
-        a.p0a = ctx->S(in);
-        a.p0b = ctx->S(in);
-        a.vsrc = ctx->S(in);
-    }
+    a.p0_two = !ctx->p0_pass && !(k == 0 && ctx->p0_explicit);
+    a.p0 = a.p0_two ? ctx->S(in) : ctx->P0I();
+    a.vsrc = k == 0 ? ctx->TN() : ctx->S(in);
     a.cells = ctx->d_cells;
     a.nrec = ctx->nrec;
     a.samples = ctx->d_samples;
@@ -1889,57 +1547,31 @@ int launch_stage(pstd_ctx *ctx, int k, int sample_slot) {
     a.remap = ctx->xcd_remap;
     const int ng = (int)ctx->tiles_gemm.size();
     if (ng) {
-        // stage k writes slot k%3, reads (k+2)%3 and clears (k+1)%3 (6 stages per
-        // step: the same slots in every step, so a captured graph replays them)
+        a.wmax = ctx->wmax;
         a.umax = ctx->umax;
-        a.slot_w = k % 3;
-        a.slot_r = (k + 2) % 3;
-        a.slot_z = (k + 1) % 3;
-        a.n_scenes = ctx->n_scenes;
         a.dmat = ctx->dmat;
         if (k == 0 && ctx->p0_explicit && !ctx->max_ranges.empty()) {
             const int nr = (int)ctx->max_ranges.size();
+            const int n = 2 * ctx->n_scenes;
+            hipLaunchKernelGGL(fill_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, ctx->umax, n);
             hipLaunchKernelGGL(state_max_kernel, dim3(16, std::min(nr, 4096)), dim3(256), 0, ctx->stream, ctx->arena,
-                               ctx->umax, ctx->d_max_ranges, nr, ctx->n_scenes, a.slot_r);
+                               ctx->umax, ctx->d_max_ranges, nr);
         }
     }
-    const int ns = (int)ctx->tiles_small.size(), n4 = (int)ctx->tiles_4096.size(), n8 = (int)ctx->tiles_8192.size();
-    const int fl = ctx->lean;
+    const int ns = ctx->n_tiles;
+    const int nt = ctx->stage_threads();
     // FFT-form tiles beside a GEMM launch: on the side stream, forked after
     // everything issued so far and joined before anything issued later
-    const bool fork = ng && (ns || n4 || n8) && ctx->overlap && ctx->side;
+    const bool fork = ng && ns && ctx->overlap && ctx->side;
     const hipStream_t fs = fork ? ctx->side : ctx->stream;
     if (fork) {
         HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
         HIP_TRY(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
     }
-    if (ns) timed_launch(ctx, fs, kClassSmall, [&] {
+    if (ns) timed_launch(ctx, fs, ctx->fmax >= 8192 ? kClass8192 : ctx->fmax >= 4096 ? kClass4096 : kClassSmall, [&] {
         a.tiles = ctx->d_tiles;
-        if (ctx->small_nt == 512) {
-            if (fl == kLate) hipLaunchKernelGGL((stage_small_kernel<512, kLate>), dim3(ns), dim3(512), 0, fs, a);
-            else if (fl == kMid) hipLaunchKernelGGL((stage_small_kernel<512, kMid>), dim3(ns), dim3(512), 0, fs, a);
-            else hipLaunchKernelGGL((stage_small_kernel<512, kEarly>), dim3(ns), dim3(512), 0, fs, a);
-        } else if (ctx->small_nt == 128) {
-            if (fl == kLate) hipLaunchKernelGGL((stage_small_kernel<128, kLate>), dim3(ns), dim3(128), 0, fs, a);
-            else if (fl == kMid) hipLaunchKernelGGL((stage_small_kernel<128, kMid>), dim3(ns), dim3(128), 0, fs, a);
-            else hipLaunchKernelGGL((stage_small_kernel<128, kEarly>), dim3(ns), dim3(128), 0, fs, a);
-        } else {
-            if (fl == kLate) hipLaunchKernelGGL((stage_small_kernel<256, kLate>), dim3(ns), dim3(256), 0, fs, a);
-            else if (fl == kMid) hipLaunchKernelGGL((stage_small_kernel<256, kMid>), dim3(ns), dim3(256), 0, fs, a);
-            else hipLaunchKernelGGL((stage_small_kernel<256, kEarly>), dim3(ns), dim3(256), 0, fs, a);
-        }
-    });
-    if (n4) timed_launch(ctx, fs, kClass4096, [&] {
-        a.tiles = ctx->d_tiles + ns;
-        size_t lds = 2 * sizeof(float2) * LdsMap<4096, 1, 0>::SIZE;
-        if (fl == kLate) hipLaunchKernelGGL((stage_big_kernel<4096, kLate>), dim3(n4), dim3(512), lds, fs, a);
-        else if (fl == kMid) hipLaunchKernelGGL((stage_big_kernel<4096, kMid>), dim3(n4), dim3(512), lds, fs, a);
-        else hipLaunchKernelGGL((stage_big_kernel<4096, kEarly>), dim3(n4), dim3(512), lds, fs, a);
-    });
-    if (n8) timed_launch(ctx, fs, kClass8192, [&] {
-        // one line pair per 512-thread block as two 4096-point transforms
-        a.tiles = ctx->d_tiles + ns + n4;
-        hipLaunchKernelGGL(stage_split_kernel, dim3(n8), dim3(kSplitT), kSplitLds, fs, a);
+        a.segs = ctx->d_segs;
+        hipLaunchKernelGGL(stage_kernel(nt), dim3(ns), dim3(nt), stage_lds(nt), fs, a);
     });
     if (fork) HIP_TRY(hipEventRecord(ctx->ev_join, ctx->side));
     if (ng) timed_launch(ctx, ctx->stream, kClassGemm, [&] {
@@ -1951,6 +1583,11 @@ int launch_stage(pstd_ctx *ctx, int k, int sample_slot) {
                                ctx->d_gemm, ctx->ftab);
     });
     if (fork) HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
+    if (ctx->p0_pass) {
+        const MaxArgs mx{ctx->wmax, ctx->d_max_first, ctx->umax, ng ? 2 * ctx->n_scenes : 0};
+        hipLaunchKernelGGL(p0_pass_kernel, dim3(mx.n + ctx->p0_first.back()), dim3(256), 0, ctx->stream, ctx->S(outi),
+                           ctx->P0I(), ctx->d_p0_tiles, 1, mx);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         ctx->err = std::string("stage launch: ") + hipGetErrorString(e);
@@ -1977,18 +1614,38 @@ long long field_off(const DomainDev &d, int f) {
     }
 }
 
-int materialise_p0(pstd_ctx *ctx) {
-    // P0I <- S1.px + S1.py for every domain (the current, stale p0)
-    if (ctx->p0_explicit) return PSTD_OK;
-    if (ctx->steps_done == 0) return PSTD_OK;
-    hipLaunchKernelGGL(p0_materialise_kernel, dim3(64, std::min(ctx->n_ranges, 64)), dim3(256), 0, ctx->stream,
-                       ctx->S(1), ctx->P0I(), ctx->d_ranges, ctx->n_ranges);
+// P0I's slots of domain d (all domains: d < 0) from S1, or (px slots set) the
+// transposed ones alone.
+int launch_p0(pstd_ctx *ctx, int d, bool from_stage) {
+    const int t0 = d < 0 ? 0 : ctx->p0_first[d], t1 = d < 0 ? ctx->p0_first.back() : ctx->p0_first[d + 1];
+    hipLaunchKernelGGL(p0_pass_kernel, dim3(t1 - t0), dim3(256), 0, ctx->stream, ctx->S(1), ctx->P0I(),
+                       ctx->d_p0_tiles + t0, from_stage ? 1 : 0, MaxArgs{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         ctx->err = std::string("p0 launch: ") + hipGetErrorString(e);
         return PSTD_ERR_DEVICE;
     }
+    return PSTD_OK;
+}
+
+int materialise_p0(pstd_ctx *ctx) {
+    // P0I <- S1.px + S1.py for every domain (the current, stale p0)
+    if (ctx->p0_explicit) return PSTD_OK;
+    if (ctx->steps_done == 0) return PSTD_OK;
+    if (!ctx->p0_pass) {
+        const int rc = launch_p0(ctx, -1, true);
+        if (rc) return rc;
+    }
     ctx->p0_explicit = true;
+    return PSTD_OK;
+}
+
+// Row-major rows x cols field <-> column-major: the host's and the device's
+// layout of vy and py.
+int launch_transpose(pstd_ctx *ctx, const float *src, float *dst, int rows, int cols) {
+    hipLaunchKernelGGL(transpose_kernel, dim3((cols + kP0Side - 1) / kP0Side, (rows + kP0Side - 1) / kP0Side), dim3(256),
+                       0, ctx->stream, src, dst, rows, cols);
+    HIP_TRY(hipGetLastError());
     return PSTD_OK;
 }
 
@@ -2033,13 +1690,9 @@ int pstd_ctx_create(int device, pstd_ctx **out) {
     if (hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess) ctx->side = nullptr;
     if (hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess) ctx->ev_fork = nullptr;
     if (hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess) ctx->ev_join = nullptr;
-    // the long-line classes need more than 64 KiB of LDS per workgroup
-    const size_t lds4 = 2 * sizeof(float2) * LdsMap<4096, 1, 0>::SIZE;
+    // more than 64 KiB of LDS per workgroup: 512-thread stage blocks, the GEMM kernel
     const hipFuncAttribute attr = hipFuncAttributeMaxDynamicSharedMemorySize;
-    const void *big4[3] = {(const void *)stage_big_kernel<4096, kEarly>, (const void *)stage_big_kernel<4096, kLate>,
-                           (const void *)stage_big_kernel<4096, kMid>};
-    bool lds_ok = hipFuncSetAttribute((const void *)stage_split_kernel, attr, kSplitLds) == hipSuccess;
-    for (int f = 0; f < 3; ++f) lds_ok = lds_ok && hipFuncSetAttribute(big4[f], attr, lds4) == hipSuccess;
+    bool lds_ok = hipFuncSetAttribute((const void *)stage_kernel(512), attr, stage_lds(512)) == hipSuccess;
     lds_ok = lds_ok &&
              hipFuncSetAttribute((const void *)stage_gemm_kernel<_Float16>, attr, kGemmLdsBytes) == hipSuccess &&
              hipFuncSetAttribute((const void *)stage_gemm_kernel<__bf16>, attr, kGemmLdsBytes) == hipSuccess;
@@ -2083,8 +1736,9 @@ static int enqueue_steps(pstd_ctx *ctx, int chunk, int base = 0) {
         }
         if (ctx->n_si > 0) {
             // spectral receivers of this step, from its raw stage-5 output
-            hipLaunchKernelGGL(si_line_kernel, dim3((ctx->n_si_lines + 3) / 4), dim3(256), 0, ctx->stream, ctx->S(1),
-                               ctx->d_si_lines, ctx->n_si_lines, ctx->d_si_coef, ctx->d_si_col);
+            hipLaunchKernelGGL(si_line_kernel, dim3((ctx->n_si_lines + 3) / 4), dim3(256), 0, ctx->stream,
+                               ctx->p0_pass ? ctx->P0I() : ctx->S(1), ctx->d_si_lines, ctx->n_si_lines,
+                               ctx->p0_pass ? 0 : 1, ctx->d_si_coef, ctx->d_si_col);
             hipLaunchKernelGGL(si_point_kernel, dim3(ctx->n_si), dim3(64), 0, ctx->stream, ctx->d_si_col,
                                ctx->d_si_points, ctx->d_si_coef, ctx->d_samples, ctx->nrec, base + s);
             HIP_TRY(hipGetLastError());
@@ -2098,43 +1752,70 @@ static int enqueue_steps(pstd_ctx *ctx, int chunk, int base = 0) {
     return PSTD_OK;
 }
 
-// Tile lists for the current block size of the F <= 2048 class: a segment's
-// lines in tiles of NL = 2 P lines (P = NT / (F/8) pairs; one pair per tile
-// above 2048), then the passthrough/receiver tiles; uploaded as
-// small | 4096 | 8192.  The pairs (line0 + 2p, line0 + 2p + 1) are the same
-// for every NT, so results do not depend on it.
+// The tile list for the current block size NT: a segment's lines in tiles of 2 P
+// lines (P = NT / T pairs), passthrough fields in chunks.  The pairs (line0 + 2p,
+// line0 + 2p + 1) are the same for every NT, so results do not depend on it.
 static int upload_tiles(pstd_ctx *ctx) {
-    ctx->tiles_small.clear();
-    ctx->tiles_4096.clear();
-    ctx->tiles_8192.clear();
-    for (const TileDesc &g : ctx->fft_segs) {
-        const int per = 2 * (g.F >= 4096 ? 1 : ctx->small_nt / (g.F / 8));
-        for (int l = 0; l < g.count; l += per) {
-            TileDesc t = g;
-            t.line0 = g.line0 + l;
-            t.count = std::min(per, g.count - l);
-            if (g.F == 4096) ctx->tiles_4096.push_back(t);
-            else if (g.F == 8192) ctx->tiles_8192.push_back(t);
-            else ctx->tiles_small.push_back(t);
-        }
+    const int nt = ctx->stage_threads();
+    std::vector<TileRef> tiles;
+    // the longest tiles first, so that none of them starts last — where there are
+    // more wavefronts than the chip holds at once (4 x 1024 SIMDs); a scene that
+    // fits is better off with its kinds of tiles mixed over the CUs
+    long long waves = 0;
+    for (const TileDesc &g : ctx->fft_segs)
+        if (g.kind == 0) waves += (long long)g.count / 2 * (g.F / fft_values(g.F)) / 64;
+    std::vector<int> order(ctx->fft_segs.size());
+    for (size_t k = 0; k < order.size(); ++k) order[k] = (int)k;
+    auto length = [&](int k) { return ctx->fft_segs[k].kind == 0 ? ctx->fft_segs[k].F : 0; };
+    if (waves > 4096) std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return length(x) > length(y); });
+    for (int k : order) {
+        const TileDesc &g = ctx->fft_segs[k];
+        const int per = g.kind == 0 ? 2 * nt / (g.F / fft_values(g.F)) : kPassChunk;
+        for (int l = 0; l < g.count; l += per) tiles.push_back({k, g.line0 + l, std::min(per, g.count - l), 0});
     }
-    ctx->tiles_small.insert(ctx->tiles_small.end(), ctx->tiles_extra.begin(), ctx->tiles_extra.end());
-    ctx->tiles_all = ctx->tiles_small;
-    ctx->tiles_all.insert(ctx->tiles_all.end(), ctx->tiles_4096.begin(), ctx->tiles_4096.end());
-    ctx->tiles_all.insert(ctx->tiles_all.end(), ctx->tiles_8192.begin(), ctx->tiles_8192.end());
+    ctx->n_tiles = (int)tiles.size();
     HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (!ctx->tiles_gemm.empty()) {
+        // maxima slots: a group (scene, class) after the other
+        const int groups = 2 * ctx->n_scenes;
+        auto group = [&](const TileRef &r) { return 2 * ctx->fft_segs[r.seg].scene + (ctx->fft_segs[r.seg].vel ? 0 : 1); };
+        std::vector<int2> first(groups + 1, make_int2(0, 0));
+        auto writes = [&](const TileRef &r) { return ctx->fft_segs[r.seg].kind != 2; };  // (receivers store no maximum)
+        for (const TileRef &r : tiles)
+            if (writes(r)) first[group(r) + 1].x += nt / 64;
+        for (int i = 0; i < groups; ++i) first[i + 1].x += first[i].x;
+        std::vector<int2> next = first;
+        for (TileRef &r : tiles) {
+            if (!writes(r)) continue;
+            int &n = next[group(r)].x;
+            r.slot = n;
+            n += nt / 64;
+        }
+        const int base = first[groups].x;
+        for (int i = 0; i <= groups; ++i) first[i].y = base + ctx->gemm_first[i];
+        std::vector<GemmTile> gemm = ctx->tiles_gemm;
+        for (GemmTile &t : gemm) t.slot += base;
+        if (ctx->wmax) HIP_TRY(hipFree(ctx->wmax));
+        ctx->wmax = nullptr;
+        HIP_TRY(hipMalloc(&ctx->wmax, (size_t)(base + ctx->gemm_first.back()) * sizeof(float)));
+        HIP_TRY(hipMemcpyAsync(ctx->d_gemm, gemm.data(), gemm.size() * sizeof(GemmTile), hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(hipMemcpyAsync(ctx->d_max_first, first.data(), first.size() * sizeof(int2), hipMemcpyHostToDevice,
+                               ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+    }
     if (ctx->d_tiles) HIP_TRY(hipFree(ctx->d_tiles));
     ctx->d_tiles = nullptr;
-    HIP_TRY(hipMalloc(&ctx->d_tiles, std::max<size_t>(1, ctx->tiles_all.size()) * sizeof(TileDesc)));
-    if (!ctx->tiles_all.empty())
-        HIP_TRY(hipMemcpyAsync(ctx->d_tiles, ctx->tiles_all.data(), ctx->tiles_all.size() * sizeof(TileDesc),
-                               hipMemcpyHostToDevice, ctx->stream));
+    HIP_TRY(hipMalloc(&ctx->d_tiles, std::max<size_t>(1, tiles.size()) * sizeof(TileRef)));
+    if (!tiles.empty()) {
+        HIP_TRY(hipMemcpyAsync(ctx->d_tiles, tiles.data(), tiles.size() * sizeof(TileRef), hipMemcpyHostToDevice,
+                               ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+    }
     return PSTD_OK;
 }
 
-// Launch-shape autotuner.  Times every (block size, stage-kernel flavour, tile
-// order) candidate on the freshly uploaded (all-zero) state and keeps the
-// fastest.  Zero fields stay exactly zero under the update, and the arenas are
+// Launch-shape autotuner.  Times every (block size, tile order) candidate on the
+// freshly uploaded (all-zero) state and keeps the fastest.  Zero fields stay exactly zero under the update, and the arenas are
 // cleared again afterwards, so tuning leaves no trace in the results.
 // The autotuner's choices, per (device, plan signature): a later context with a
 // plan of the same launch geometry on the same device takes the choice and
@@ -2171,7 +1852,6 @@ uint64_t plan_signature(const pstd_ctx *ctx) {
         mix(t.vel);
         mix(t.n_out);
     }
-    mix((long long)ctx->tiles_extra.size());
     mix((long long)ctx->tiles_gemm.size());
     for (const GemmTile &g : ctx->tiles_gemm) {
         mix(g.t.dir);
@@ -2204,7 +1884,6 @@ static int autotune(pstd_ctx *ctx) {
             return PSTD_OK;
         }
     }
-    static const int cand[6][2] = {{kLate, 1}, {kMid, 1}, {kEarly, 1}, {kLate, 0}, {kMid, 0}, {kEarly, 0}};  // (flavour, xcd order)
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
@@ -2231,10 +1910,10 @@ static int autotune(pstd_ctx *ctx) {
         rc = time_steps(ms);
         if (rc == PSTD_OK && ms > 0.f) n = std::min(50, std::max(3, (int)std::ceil(2.0f / (ms / 3.0f))));
     }
-    // block sizes of the F <= 2048 class (it alone depends on them)
+    // block sizes, where the lines leave a choice
     std::vector<int> nts = {ctx->small_nt};
-    if (ctx->small_fmax > 0)
-        for (int nt : {128, 256, 512})
+    if (ctx->small_fmax > 0 && ctx->fmax <= 2048)
+        for (int nt : {128, 256})
             if (nt != ctx->small_nt && (nt >= 256 || ctx->small_fmax <= 1024)) nts.push_back(nt);
     for (int nt : nts) {
         if (rc != PSTD_OK) break;
@@ -2242,9 +1921,8 @@ static int autotune(pstd_ctx *ctx) {
             ctx->small_nt = nt;
             rc = upload_tiles(ctx);
         }
-        for (int c = 0; c < 6 && rc == PSTD_OK; ++c) {
-            ctx->lean = cand[c][0];
-            ctx->xcd_remap = cand[c][1];
+        for (int c = 1; c >= 0 && rc == PSTD_OK; --c) {
+            ctx->xcd_remap = c;
             float ms = 0;
             rc = time_steps(ms);
             if (rc == PSTD_OK && (first || ms < best)) {
@@ -2256,8 +1934,7 @@ static int autotune(pstd_ctx *ctx) {
         }
     }
     if (rc == PSTD_OK) {
-        ctx->lean = cand[bi][0];
-        ctx->xcd_remap = cand[bi][1];
+        ctx->xcd_remap = bi;
         if (bnt != ctx->small_nt) {
             ctx->small_nt = bnt;
             rc = upload_tiles(ctx);
@@ -2275,7 +1952,7 @@ static int autotune(pstd_ctx *ctx) {
         g_tune[key] = {ctx->lean, ctx->xcd_remap, ctx->small_nt, ctx->tuned_stage_ms};
     }
     HIP_TRY(hipMemsetAsync(ctx->arena, 0, 4 * (size_t)ctx->arena_floats * sizeof(float), ctx->stream));
-    if (ctx->umax) HIP_TRY(hipMemsetAsync(ctx->umax, 0, 3 * 2 * (size_t)ctx->n_scenes * sizeof(unsigned), ctx->stream));
+    if (ctx->umax) HIP_TRY(hipMemsetAsync(ctx->umax, 0, 2 * (size_t)ctx->n_scenes * sizeof(unsigned), ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->steps_done = 0;
     ctx->p0_explicit = true;
@@ -2484,19 +2161,22 @@ static int build_spectral_receivers(pstd_ctx *ctx, const pstd_plan_desc *plan) {
             }
             SILine L{};
             L.m_px = d.base + d.f_px + (long long)q.row * d.nx;
-            L.m_py = d.base + d.f_py + (long long)q.row * d.nx;
+            L.m_py = d.base + d.f_py + q.row;
+            L.m_ld = d.ny;
             L.s1_px = L.s1_py = L.s2_px = L.s2_py = -1;
             if (sx.side1 >= 0) {
                 const DomainDev &n = ctx->doms[sx.side1];
-                const long long rr = (long long)(q.row + sx.side1_offset) * n.nx + n.nx - sx.wlen;
-                L.s1_px = n.base + n.f_px + rr;
-                L.s1_py = n.base + n.f_py + rr;
+                const int row = q.row + sx.side1_offset, col = n.nx - sx.wlen;
+                L.s1_px = n.base + n.f_px + (long long)row * n.nx + col;
+                L.s1_py = n.base + n.f_py + (long long)col * n.ny + row;
+                L.s1_ld = n.ny;
             }
             if (sx.side2 >= 0) {
                 const DomainDev &n = ctx->doms[sx.side2];
-                const long long rr = (long long)(q.row + sx.side2_offset) * n.nx;
-                L.s2_px = n.base + n.f_px + rr;
-                L.s2_py = n.base + n.f_py + rr;
+                const int row = q.row + sx.side2_offset;
+                L.s2_px = n.base + n.f_px + (long long)row * n.nx;
+                L.s2_py = n.base + n.f_py + row;
+                L.s2_ld = n.ny;
             }
             L.n_main = d.nx;
             L.w = sx.wlen;
@@ -2541,13 +2221,10 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->release();
     ctx->doms.clear();
-    ctx->tiles_small.clear();
     ctx->small_fmax = 0;
+    ctx->fmax = 0;
     ctx->small_nt = 256;
     ctx->fft_segs.clear();
-    ctx->tiles_extra.clear();
-    ctx->tiles_4096.clear();
-    ctx->tiles_8192.clear();
     ctx->tiles_gemm.clear();
     ctx->max_ranges.clear();
     ctx->n_scenes = 1;
@@ -2558,7 +2235,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     ctx->gemm_cells = 0;
     ctx->plan_domains.assign(plan->domains, plan->domains + plan->n_domains);
     // arena layout: one block per domain (vx, vy, px, py), 256 B aligned
-    long long off = 0;
+    long long off = kLead;  // zeros before the first block
     auto align = [](long long v) { return (v + 63) & ~63LL; };
     for (int i = 0; i < plan->n_domains; ++i) {
         const pstd_plan_domain &p = plan->domains[i];
@@ -2585,12 +2262,12 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         d.f_px = (int)f;
         f = align(f + cells);
         d.f_py = (int)f;
-        f = align(f + cells + 1);  // a spare float after py (8-byte column accesses)
+        f = align(f + cells + 1);  // a spare float after py (8-byte accesses of line pairs)
         d.size = (int)f;
         off += f;
         ctx->doms.push_back(d);
     }
-    ctx->arena_floats = (size_t)std::max(off, 64LL);
+    ctx->arena_floats = (size_t)(off + kLead);  // a matrix tile reads up to 3 floats past a block
     ctx->dt = plan->dt;
     ctx->c1 = plan->c1;
     for (int k = 0; k < 6; ++k) ctx->alpha[k] = plan->rk_alpha[k];
@@ -2602,24 +2279,24 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     std::map<int, int> win_cache;
     const double dx = plan->dx;
     // source addressing of a domain's derivative input for (direction, field):
-    // pressure reads p0 = px + py (row stride nx), velocity vx (X, stride nx+1) or vy (Y)
-    // (field offsets within the domain block; velocity lines have no second array)
-    auto src_addr = [&](const DomainDev &d, int dir, int field, int &a, int &b, int &ls, int &ps) {
+    // pressure reads p0 (px slot row-major for X, py slot column-major for Y; on
+    // the fly plus the other field across its layout), velocity vx (X) or vy (Y)
+    // (field offsets within the domain block)
+    auto src_addr = [&](const DomainDev &d, int dir, int field, int &a, int &b, int &ls, int &bp) {
+        const int n = dir == 0 ? d.nx : d.ny;
         if (field == 0) {
-            a = d.f_px;
-            b = d.f_py;
-            ls = dir == 0 ? d.nx : 1;
-            ps = dir == 0 ? 1 : d.nx;
-        } else if (dir == 0) {
-            a = b = d.f_vx;
-            ls = d.nx + 1;
-            ps = 1;
+            a = dir == 0 ? d.f_px : d.f_py;
+            b = dir == 0 ? d.f_py : d.f_px;
+            ls = n;
+            bp = dir == 0 ? d.ny : d.nx;
         } else {
-            a = b = d.f_vy;
-            ls = 1;
-            ps = d.nx;
+            a = b = dir == 0 ? d.f_vx : d.f_vy;
+            ls = n + 1;
+            bp = 0;
         }
     };
+    long long strided_bytes = 0, pass_cells = 0;  // p0 on the fly, or by the pass
+    for (const DomainDev &d : ctx->doms) pass_cells += (long long)d.nx * d.ny;
     std::vector<std::vector<char>> covered(plan->n_domains, std::vector<char>(4, 0));
     std::vector<uint16_t> dmat;
     std::map<std::string, std::tuple<long long, int, int>> dcache;  // matrix key -> (hi offset, d_exp, dot row)
@@ -2673,7 +2350,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             ctx->err = "window longer than the domain";
             return PSTD_ERR_INVALID;
         }
-        src_addr(dm, s.direction, s.field, g.m_a, g.m_b, g.m_ls, g.m_ps);
+        src_addr(dm, s.direction, s.field, g.m_a, g.m_b, g.m_ls, g.m_bp);
         g.s1_len = g.s2_len = -1;
         // neighbour bounds: lines and halo columns must exist in the neighbour
         for (int side = 0; side < 2; ++side) {
@@ -2688,13 +2365,13 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
                 return PSTD_ERR_INVALID;
             }
             if (side == 0) {
-                src_addr(dn, s.direction, s.field, g.s1_a, g.s1_b, g.s1_ls, g.s1_ps);
+                src_addr(dn, s.direction, s.field, g.s1_a, g.s1_b, g.s1_ls, g.s1_bp);
                 g.s1_line = o;
                 g.s1_len = nlen;
                 g.s1_dom = dn.base;
                 g.s1_size = dn.size;
             } else {
-                src_addr(dn, s.direction, s.field, g.s2_a, g.s2_b, g.s2_ls, g.s2_ps);
+                src_addr(dn, s.direction, s.field, g.s2_a, g.s2_b, g.s2_ls, g.s2_bp);
                 g.s2_line = o;
                 g.s2_len = nlen;
                 g.s2_dom = dn.base;
@@ -2709,15 +2386,8 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             continue;  // read by the spectral receivers only
         }
         // output field: X pressure -> vx, X velocity -> px, Y pressure -> vy, Y velocity -> py
-        if (s.direction == 0) {
-            g.o_f = s.field == 0 ? dm.f_vx : dm.f_px;
-            g.o_ls = s.field == 0 ? dm.nx + 1 : dm.nx;
-            g.o_ps = 1;
-        } else {
-            g.o_f = s.field == 0 ? dm.f_vy : dm.f_py;
-            g.o_ls = 1;
-            g.o_ps = dm.nx;
-        }
+        g.o_f = s.direction == 0 ? (s.field == 0 ? dm.f_vx : dm.f_px) : (s.field == 0 ? dm.f_vy : dm.f_py);
+        g.o_ls = s.field == 0 ? n + 1 : n;
         covered[s.domain][s.direction == 0 ? (s.field == 0 ? 2 : 0) : (s.field == 0 ? 3 : 1)] = 1;
         auto fk = std::make_tuple(g.F, s.table_len, s.field);
         auto it = filt_cache.find(fk);
@@ -2736,18 +2406,6 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             ctab.insert(ctab.end(), tw.begin(), tw.end());
         }
         g.tw_off = tt->second;
-        g.tw2_off = 0;
-        if (g.F == 8192) {
-            // the split transform's two 4096-point halves
-            auto t2 = tw_cache.find(4096);
-            if (t2 == tw_cache.end()) {
-                std::vector<float2> tw;
-                build_twiddles(4096, tw);
-                t2 = tw_cache.emplace(4096, (int)ctab.size()).first;
-                ctab.insert(ctab.end(), tw.begin(), tw.end());
-            }
-            g.tw2_off = t2->second;
-        }
         auto wt = win_cache.find(s.wlen);
         if (wt == win_cache.end()) {
             std::vector<float> w;
@@ -2757,6 +2415,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         }
         g.win_off = wt->second;
         g.scene = scene_of(s.domain);
+        if (s.field == 0) strided_bytes += 4LL * (s.line_end - s.line_begin) * n * strided_factor(g.F);
         // GEMM form: segments that fill the 128 x 256 tiles at least to 3/4
         // become GEMM tiles; thin ones (PML strips) stay FFT tiles
         const int nlines_seg = s.line_end - s.line_begin;
@@ -2768,6 +2427,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         }
         g.line0 = s.line_begin;
         g.count = s.line_end - s.line_begin;
+        ctx->fmax = std::max(ctx->fmax, g.F);
         if (g.F <= 2048) ctx->small_fmax = std::max(ctx->small_fmax, g.F);
         ctx->fft_segs.push_back(g);
     }
@@ -2779,25 +2439,23 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         const int sizes[4] = {d.nx * d.ny, d.nx * d.ny, d.ny * (d.nx + 1), (d.ny + 1) * d.nx};
         for (int f = 0; f < 4; ++f) {
             if (covered[i][f]) continue;
-            for (int e = 0; e < sizes[f]; e += kPassChunk) {
-                TileDesc t{};
-                t.kind = 1;
-                t.line0 = e;
-                t.count = std::min(kPassChunk, sizes[f] - e);
-                t.m_dom = d.base;
-                t.m_size = d.size;
-                t.o_f = offs[f];
-                t.is_pml = d.is_pml;
-                t.scene = scene_of(i);
-                t.vel = f < 2 ? 1 : 0;  // maxima class: px/py as written by velocity lines
-                ctx->tiles_extra.push_back(t);
-            }
+            TileDesc t{};
+            t.kind = 1;
+            t.count = sizes[f];
+            t.m_dom = d.base;
+            t.m_size = d.size;
+            t.o_f = offs[f];
+            t.is_pml = d.is_pml;
+            t.scene = scene_of(i);
+            t.vel = f < 2 ? 1 : 0;  // maxima class: px/py as written by velocity lines
+            ctx->fft_segs.push_back(t);
         }
     }
     if (plan->n_receivers > 0) {
         TileDesc t{};
         t.kind = 2;  // receiver sampling of the previous step (first stage only)
-        ctx->tiles_extra.push_back(t);
+        t.count = 1;
+        ctx->fft_segs.push_back(t);
     }
     if (ctab.empty()) ctab.push_back(make_float2(0, 0));
     if (ftab.empty()) ftab.push_back(0);
@@ -2816,7 +2474,14 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
                 ctx->err = "PML domain without factor arrays";
                 return PSTD_ERR_INVALID;
             }
-            std::memcpy(pml.data() + offs[f], src[f], sizeof(float) * sizes[f]);
+            if (f == 0 || f == 2) {
+                std::memcpy(pml.data() + offs[f], src[f], sizeof(float) * sizes[f]);
+            } else {  // vy, py: column-major
+                const int rows = f == 1 ? p.ny + 1 : p.ny;
+                float *dst = pml.data() + offs[f];
+                for (int x = 0; x < p.nx; ++x)
+                    for (int y = 0; y < rows; ++y) dst[(size_t)x * rows + y] = src[f][(size_t)y * p.nx + x];
+            }
         }
     }
     // receivers
@@ -2830,16 +2495,22 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         }
         const DomainDev &d = ctx->doms[rc.domain];
         if (rc.spectral) cells.push_back({-1, -1});
-        else cells.push_back({d.base + d.f_px + rc.index, d.base + d.f_py + rc.index});
+        else cells.push_back({d.base + d.f_px + rc.index, d.base + d.f_py + (long long)(rc.index % d.nx) * d.ny + rc.index / d.nx});
     }
     ctx->nrec = (int)cells.size();
     {
         int rc = build_spectral_receivers(ctx, plan);
         if (rc) return rc;
     }
-    std::vector<P0Range> ranges;
-    for (const DomainDev &d : ctx->doms) ranges.push_back({d.base + d.f_px, d.base + d.f_py, (long long)d.nx * d.ny});
-    ctx->n_ranges = (int)ranges.size();
+    std::vector<P0Tile> p0_tiles;
+    ctx->p0_first.clear();
+    for (const DomainDev &d : ctx->doms) {
+        ctx->p0_first.push_back((int)p0_tiles.size());
+        for (int y = 0; y < d.ny; y += kP0Side)
+            for (int x = 0; x < d.nx; x += kP0Side) p0_tiles.push_back({d.base + d.f_px, d.base + d.f_py, d.nx, d.ny, x, y});
+    }
+    ctx->p0_first.push_back((int)p0_tiles.size());
+    ctx->p0_pass = !ctx->tiles_gemm.empty() || strided_bytes - 16 * pass_cells > kP0PassBytes;
     if (!ctx->tiles_gemm.empty()) {
         // what a first stage after host writes reads: p0 (P0I) and vx, vy (TN)
         for (int i = 0; i < plan->n_domains; ++i) {
@@ -2860,33 +2531,47 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     HIP_TRY(hipMemcpyAsync(ctx->ctab, ctab.data(), ctab.size() * sizeof(float2), hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(hipMalloc(&ctx->ftab, ftab.size() * sizeof(float)));
     HIP_TRY(hipMemcpyAsync(ctx->ftab, ftab.data(), ftab.size() * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    {
-        const int rc = upload_tiles(ctx);
-        if (rc) return rc;
-    }
+    HIP_TRY(hipMalloc(&ctx->d_segs, std::max<size_t>(1, ctx->fft_segs.size()) * sizeof(TileDesc)));
+    if (!ctx->fft_segs.empty())
+        HIP_TRY(hipMemcpyAsync(ctx->d_segs, ctx->fft_segs.data(), ctx->fft_segs.size() * sizeof(TileDesc),
+                               hipMemcpyHostToDevice, ctx->stream));
     if (!ctx->tiles_gemm.empty()) {
+        // the GEMM tiles' maxima slots, numbered like those of upload_tiles
+        const int groups = 2 * ctx->n_scenes;
+        ctx->gemm_first.assign(groups + 1, 0);
+        auto group = [](const GemmTile &t) { return 2 * t.t.scene + (t.t.vel ? 0 : 1); };
+        for (const GemmTile &t : ctx->tiles_gemm) ctx->gemm_first[group(t) + 1] += kGemmThreads / 64;
+        for (int i = 0; i < groups; ++i) ctx->gemm_first[i + 1] += ctx->gemm_first[i];
+        std::vector<int> next = ctx->gemm_first;
+        for (GemmTile &t : ctx->tiles_gemm) {
+            t.slot = next[group(t)];
+            next[group(t)] += kGemmThreads / 64;
+        }
         // segment order (a scene's segments together, a line block's output
         // tiles adjacent): measured faster than grouping the tiles by matrix
         HIP_TRY(hipMalloc(&ctx->d_gemm, ctx->tiles_gemm.size() * sizeof(GemmTile)));
-        HIP_TRY(hipMemcpyAsync(ctx->d_gemm, ctx->tiles_gemm.data(), ctx->tiles_gemm.size() * sizeof(GemmTile),
-                               hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(hipMalloc(&ctx->d_max_first, (size_t)(groups + 1) * sizeof(int2)));
         HIP_TRY(hipMalloc(&ctx->dmat, std::max<size_t>(1, dmat.size()) * sizeof(uint16_t)));
         HIP_TRY(hipMemcpyAsync(ctx->dmat, dmat.data(), dmat.size() * sizeof(uint16_t), hipMemcpyHostToDevice,
                                ctx->stream));
-        const size_t nmax = 3 * 2 * (size_t)ctx->n_scenes;
+        const size_t nmax = 2 * (size_t)ctx->n_scenes;
         HIP_TRY(hipMalloc(&ctx->umax, nmax * sizeof(unsigned)));
         HIP_TRY(hipMemsetAsync(ctx->umax, 0, nmax * sizeof(unsigned), ctx->stream));
         HIP_TRY(hipMalloc(&ctx->d_max_ranges, ctx->max_ranges.size() * sizeof(MaxRange)));
         HIP_TRY(hipMemcpyAsync(ctx->d_max_ranges, ctx->max_ranges.data(), ctx->max_ranges.size() * sizeof(MaxRange),
                                hipMemcpyHostToDevice, ctx->stream));
     }
+    {
+        const int rc = upload_tiles(ctx);
+        if (rc) return rc;
+    }
     HIP_TRY(hipMalloc(&ctx->d_cells, std::max<size_t>(1, cells.size()) * sizeof(ReceiverCell)));
     if (!cells.empty())
         HIP_TRY(hipMemcpyAsync(ctx->d_cells, cells.data(), cells.size() * sizeof(ReceiverCell), hipMemcpyHostToDevice,
                                ctx->stream));
-    HIP_TRY(hipMalloc(&ctx->d_ranges, std::max<size_t>(1, ranges.size()) * sizeof(P0Range)));
-    if (!ranges.empty())
-        HIP_TRY(hipMemcpyAsync(ctx->d_ranges, ranges.data(), ranges.size() * sizeof(P0Range), hipMemcpyHostToDevice,
+    HIP_TRY(hipMalloc(&ctx->d_p0_tiles, std::max<size_t>(1, p0_tiles.size()) * sizeof(P0Tile)));
+    if (!p0_tiles.empty())
+        HIP_TRY(hipMemcpyAsync(ctx->d_p0_tiles, p0_tiles.data(), p0_tiles.size() * sizeof(P0Tile), hipMemcpyHostToDevice,
                                ctx->stream));
     ctx->sample_cap = 4096;
     HIP_TRY(hipMalloc(&ctx->d_samples, (size_t)ctx->sample_cap * std::max(1, ctx->nrec) * sizeof(float)));
@@ -3015,21 +2700,27 @@ int pstd_ctx_set_field(pstd_ctx *ctx, int domain, int field, const float *host, 
         return PSTD_ERR_INVALID;
     }
     HIP_TRY(hipSetDevice(ctx->device));
-    float *dst;
-    if (ctx->umax && field != PSTD_FIELD_P0) {
+    const DomainDev &d = ctx->doms[domain];
+    const size_t bytes = count * sizeof(float);
+    if (field == PSTD_FIELD_P0 || ctx->umax) {
         // GEMM form: the next first stage recomputes the scaling maxima from
         // the state, which needs p0 in its explicit array
         int rc = materialise_p0(ctx);
         if (rc) return rc;
     }
     if (field == PSTD_FIELD_P0) {
-        int rc = materialise_p0(ctx);
+        HIP_TRY(hipMemcpyAsync(ctx->P0I() + field_off(d, PSTD_FIELD_PX), host, bytes, hipMemcpyHostToDevice, ctx->stream));
+        int rc = launch_p0(ctx, domain, false);
         if (rc) return rc;
-        dst = ctx->P0I() + field_off(ctx->doms[domain], PSTD_FIELD_PX);
+    } else if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
+        // column-major on the device; S0 holds nothing between time steps
+        float *rows = ctx->S(0) + field_off(d, field);
+        HIP_TRY(hipMemcpyAsync(rows, host, bytes, hipMemcpyHostToDevice, ctx->stream));
+        int rc = launch_transpose(ctx, rows, ctx->TN() + field_off(d, field), (int)(count / d.nx), d.nx);
+        if (rc) return rc;
     } else {
-        dst = ctx->TN() + field_off(ctx->doms[domain], field);
+        HIP_TRY(hipMemcpyAsync(ctx->TN() + field_off(d, field), host, bytes, hipMemcpyHostToDevice, ctx->stream));
     }
-    HIP_TRY(hipMemcpyAsync(dst, host, count * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return PSTD_OK;
 }
@@ -3044,24 +2735,22 @@ int pstd_ctx_get_field(pstd_ctx *ctx, int domain, int field, float *host, size_t
     }
     HIP_TRY(hipSetDevice(ctx->device));
     const DomainDev &d = ctx->doms[domain];
+    const float *src = ctx->TN() + field_off(d, field);
     if (field == PSTD_FIELD_P0) {
-        if (ctx->p0_explicit) {
-            HIP_TRY(hipMemcpyAsync(host, ctx->P0I() + field_off(d, PSTD_FIELD_PX), count * sizeof(float), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-            HIP_TRY(hipStreamSynchronize(ctx->stream));
-        } else {
-            std::vector<float> py(count);
-            HIP_TRY(hipMemcpyAsync(host, ctx->S(1) + field_off(d, PSTD_FIELD_PX), count * sizeof(float), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-            HIP_TRY(hipMemcpyAsync(py.data(), ctx->S(1) + field_off(d, PSTD_FIELD_PY), count * sizeof(float), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-            HIP_TRY(hipStreamSynchronize(ctx->stream));
-            for (size_t i = 0; i < count; ++i) host[i] = host[i] + py[i];
+        // P0I's slots are free where the tiles form p0 on the fly
+        if (!ctx->p0_explicit && !ctx->p0_pass) {
+            int rc = launch_p0(ctx, domain, true);
+            if (rc) return rc;
         }
-        return PSTD_OK;
+        src = ctx->P0I() + field_off(d, PSTD_FIELD_PX);
+    } else if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
+        // row-major for the host; S0 holds nothing between time steps
+        float *rows = ctx->S(0) + field_off(d, field);
+        int rc = launch_transpose(ctx, src, rows, d.nx, (int)(count / d.nx));
+        if (rc) return rc;
+        src = rows;
     }
-    HIP_TRY(hipMemcpyAsync(host, ctx->TN() + field_off(d, field), count * sizeof(float), hipMemcpyDeviceToHost,
-                           ctx->stream));
+    HIP_TRY(hipMemcpyAsync(host, src, count * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return PSTD_OK;
 }
@@ -3218,7 +2907,7 @@ int pstd_ctx_set_form(pstd_ctx *ctx, int form) {
 int pstd_ctx_get_form(const pstd_ctx *ctx) { return ctx ? ctx->form : PSTD_ERR_INVALID; }
 
 int pstd_ctx_set_kernel_flavour(pstd_ctx *ctx, int flavour) {
-    if (!ctx || flavour < kEarly || flavour > kMid) return PSTD_ERR_INVALID;
+    if (!ctx || flavour < 0 || flavour > 2) return PSTD_ERR_INVALID;
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->drop_graph();
@@ -3310,13 +2999,10 @@ int pstd_ctx_advance_static(pstd_ctx *ctx, int steps) {
             ctx->err = "allocation-free advance: no device address for the scratch array";
             return PSTD_ERR_DEVICE;
         }
-        // the shared array starts from zero and the maxima of the current state
-        // (explicit p0, then the first stage's reduction), as after host writes
+        // the shared array starts from the maxima of the current state (explicit
+        // p0, then the first stage's reduction), as after host writes
         int rc = materialise_p0(ctx);
         if (rc) return rc;
-        const int n = 3 * 2 * ctx->n_scenes;
-        hipLaunchKernelGGL(fill_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, sp, n);
-        HIP_TRY(hipGetLastError());
     }
     unsigned *own = ctx->umax;
     if (gemm) ctx->umax = sp;

@@ -261,12 +261,12 @@ class _Context:
     FLAVOURS = {"early": 0, "late": 1, "mid": 2}
 
     def set_kernel_flavour(self, flavour):
-        """Stage-kernel flavour: "early", "late" or "mid" (or 0, 1, 2)."""
+        """Stage-kernel flavour: "early", "late" or "mid" (or 0, 1, 2); one kernel serves them all."""
         f = self.FLAVOURS.get(flavour, flavour)
         _check(lib().pstd_ctx_set_kernel_flavour(self.ctx, int(f)), self._err)
 
     def set_tile_threads(self, threads):
-        """Block size (128, 256 or 512; 128 needs F <= 1024) of the stage kernel for lines of FFT length <= 2048."""
+        """Block size (128, 256 or 512; 128 needs F <= 1024) of the stage kernel, where its lines leave the choice."""
         _check(lib().pstd_ctx_set_tile_threads(self.ctx, int(threads)), self._err)
 
     def form(self):
