@@ -26,9 +26,11 @@ HEADERS = ["device/fft_line.h", "host/kernel_api.h", "host/scene_model.h", "host
 # Packed FP32 instructions are kept out of the device code.  No implicit FMA
 # contraction: the device code writes its fused multiply-adds explicitly, so
 # every kernel flavour and launch shape rounds the same way (bitwise-equal
-# results whichever the autotuner picks).
+# results whichever the autotuner picks).  The first eight words of kernel
+# arguments arrive in scalar registers (the stage kernel's finds its tile's record
+# with them, without a load of its arguments first).
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
-             "-packed-fp32-ops", "-ffp-contract=off", "-Wall", "-Wno-unused-function"]
+             "-packed-fp32-ops", "-ffp-contract=off", "-mllvm", "-amdgpu-kernarg-preload-count=8", "-Wall", "-Wno-unused-function"]
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]
 
 

@@ -69,9 +69,14 @@ struct DomainDev {
     int is_pml;
 };
 
-// A line segment of a domain (Domain::calc, kernel/core/Domain.cpp:149-370) with
-// everything a workgroup needs in one scalar-loadable record, shared by all of
-// the segment's tiles.
+// One workgroup of a stage launch: `count` lines from line0 on of a line segment
+// of a domain (Domain::calc, kernel/core/Domain.cpp:149-370), with everything the
+// workgroup needs in one scalar-loadable record.  Caches are cold when a launch
+// begins, and a small scene's stage is a chain of memory latencies: a record per
+// workgroup is one of them, a reference to a record shared by the segment's tiles
+// two (100 x 50 room 6.0 against 5.8 us per stage, three rooms of 333 000 cells 12.1
+// / 11.5, 12 scenes of 64..600 a side 95.2 / 93.6, 16 sources of 512 x 1024 twice 350 /
+// 351 with the launch arguments' first words in registers, kernel arguments below).
 //  kind 0: derivative lines: gather, derivative, update.
 //  kind 1: passthrough: a field that no segment updates (rigid domains,
 //          directions openPSTD skips); lines are elements.
@@ -87,7 +92,7 @@ struct TileDesc {
     int kind;
     int F;
     int line0, count;
-    int wlen, wlog, n_main, n_out, vel, dir;  // wlog: log2 of the halo slot (2^wlog >= wlen)
+    int wlen, n_main, n_out, vel, dir;
     int h_off, tw_off, win_off;
     long long m_dom, s1_dom, s2_dom;
     int m_size, s1_size, s2_size;
@@ -99,24 +104,15 @@ struct TileDesc {
     float coef;           // 1/rho (velocity update) or rho*c1^2 (pressure update)
     int is_pml;
     int scene;            // scene of the batch (per-scene maxima of the GEMM form's scaling)
+    int slot;             // GEMM form: of the first wavefront's maximum (track_max)
 };
-
-// One workgroup of a stage launch: `count` lines of a segment from line0 on.  16
-// bytes: neighbouring workgroups share a cache line, and the segments they name
-// stay in the caches (a whole descriptor per workgroup came from memory before
-// anything else could start).
-struct TileRef {
-    int seg, line0, count;
-    int slot;  // GEMM form: of the first wavefront's maximum
-};
+static_assert(sizeof(TileDesc) == 192, "three 64-byte lines");
 
 struct ReceiverCell {
     long long px, py;  // arena element offsets of the cell's px0 and py0; px < 0: spectral receiver
 };
 
 struct StageArgs {
-    const TileRef *tiles;
-    const TileDesc *segs;
     const float2 *ctab;
     const float *ftab;
     const float *p0;   // p0 arena: P0I, or (p0_two) a stage arena whose px + py it is
@@ -133,7 +129,6 @@ struct StageArgs {
     int nrec;
     float *samples;    // samples[slot * nrec + r], slot < 0: no sampling in this launch
     int slot;
-    int remap;         // XCD-contiguous tile order (tile_index)
     // GEMM form (wmax == nullptr otherwise): the largest |value| each wavefront
     // wrote, and what the previous stage's came to per scene (max_reduce)
     float *wmax;
@@ -199,7 +194,6 @@ __device__ __forceinline__ const float *source(const StageArgs &a, int vel) { re
 // Descriptors are read through the constant address space: by scalar loads,
 // wherever they are needed, also after stores.
 typedef const __attribute__((address_space(4))) TileDesc *Seg;
-typedef const __attribute__((address_space(4))) TileRef *Ref;
 
 // A derivative tile: F-point lines, T = F/V threads per line pair; thread (p, t)
 // holds the values at positions t + m*T (m = 0..V-1) of lines 2p and 2p+1 as one
@@ -298,14 +292,16 @@ __device__ __forceinline__ void gather(const StageArgs &a, Seg td, const Tile &x
             y2[c] = bload2(r2, j0 + c * T < w && has2 ? (td->s2_b + l2 + (j0 + c * T) * td->s2_bp) * 4 : kOOB);
         }
         float2 *to = lds + pair * x.pitch;
+        const int nm2 = again(nm);
 #pragma unroll
         for (int k = 0; k < V; ++k)
-            if ((k == 0 || k * step < nm) && pos + k * step < nm) to[lds_slot(w + pos + k * step)] = b[k];
+            if ((k == 0 || k * step < nm2) && pos + k * step < nm) to[lds_slot(w + pos + k * step)] = b[k];
         __syncthreads();
         const float2 *buf = lds + x.p * x.pitch;
+        const int rows2 = again(rows);
 #pragma unroll
         for (int m = 0; m < V; ++m)
-            if (m < FULL || m < rows) add(v[m], buf[lds_slot(t + m * T)]);
+            if (m < FULL || m < rows2) add(v[m], buf[lds_slot(t + m * T)]);
 #pragma unroll
         for (int c = 0; c < NI; ++c) {
             const int i = t + c * T, j = j0 + c * T;
@@ -326,7 +322,7 @@ __device__ __forceinline__ void gather(const StageArgs &a, Seg td, const Tile &x
         if (t + c * T < w) v[c] = hl;
     }
     // thread row lo + c holds right item c from column `col` on, item c - 1 before it
-    const int lo = end >> x.logT;
+    const int lo = again(end >> x.logT);
     const bool at_end = t >= col;
 #pragma unroll
     for (int m = FULL; m < V; ++m)
@@ -414,7 +410,7 @@ __device__ __forceinline__ void update_stores(const StageArgs &a, Seg td, const 
 
 // SHORT: F = 128; SPLIT: F = 8192 (fft_line.h's two sequences)
 template <int V, int NT, bool SHORT, bool SPLIT>
-__device__ __forceinline__ void derivative_tile(const StageArgs &a, Seg td, Ref ref, float2 *lds) {
+__device__ __forceinline__ void derivative_tile(const StageArgs &a, Seg td, float2 *lds) {
     constexpr int kLogV = V == 16 ? 4 : 3;
     const int F = td->F, logT = 31 - kLogV - __builtin_clz(F);
     Tile x;
@@ -422,8 +418,8 @@ __device__ __forceinline__ void derivative_tile(const StageArgs &a, Seg td, Ref 
     x.T = 1 << logT;
     x.p = threadIdx.x >> logT;
     x.t = threadIdx.x & (x.T - 1);
-    x.line = ref->line0 + 2 * x.p;
-    x.count = ref->count - 2 * x.p;
+    x.line = td->line0 + 2 * x.p;
+    x.count = td->count - 2 * x.p;
     x.pitch = lds_pitch(F);
     float2 *buf = lds + x.p * x.pitch;
     // the tables through a buffer resource: one lane offset, the rest in scalar registers
@@ -479,9 +475,9 @@ __device__ __forceinline__ void derivative_tile(const StageArgs &a, Seg td, Ref 
     }
     if constexpr (SPLIT) split_last(v, t, tab, td->tw_off * 8);
     // the descriptor again: the gather's fields need not stay in scalar registers
-    const Seg to = (Seg)a.segs + again(ref->seg);
+    const Seg to = td + again(0);
     if constexpr (!kTnEarly) update_loads<V, SHORT>(a, to, x, tn);
-    update_stores<V, SHORT>(a, to, x, v, tn, ref->slot);
+    update_stores<V, SHORT>(a, to, x, v, tn, to->slot);
 }
 
 // One extra workgroup of a launch samples the receivers (p0 of the previous
@@ -499,7 +495,7 @@ __device__ void sample_receivers(const StageArgs &a) {
 // kernel/Solver.cpp:174-181); the last stage applies the PML factor.  Each
 // thread issues all of its loads before its stores.
 template <int NT>
-__device__ __forceinline__ void passthrough_tile(const StageArgs &a, Seg td, Ref ref) {
+__device__ __forceinline__ void passthrough_tile(const StageArgs &a, Seg td) {
     constexpr int PER = kPassChunk / NT;
     const Rsrc rt = block_rsrc(a.tn, td->m_dom, td->m_size);
     const Rsrc rp = block_rsrc(a.pml, td->m_dom, td->m_size);
@@ -510,7 +506,7 @@ __device__ __forceinline__ void passthrough_tile(const StageArgs &a, Seg td, Ref
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int e = threadIdx.x + k * NT;
-        off[k] = e < ref->count ? (td->o_f + ref->line0 + e) * 4 : kOOB;
+        off[k] = e < td->count ? (td->o_f + td->line0 + e) * 4 : kOOB;
         v[k] = bload(rt, off[k]);
         f[k] = use_pml ? bload(rp, off[k]) : 1.f;
     }
@@ -522,7 +518,7 @@ __device__ __forceinline__ void passthrough_tile(const StageArgs &a, Seg td, Ref
     float mx = 0.f;
 #pragma unroll
     for (int k = 0; k < PER; ++k) mx = fmaxf(mx, fabsf(v[k]));
-    track_max(a, ref->slot, mx);
+    track_max(a, td->slot, mx);
 }
 
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs on XCD
@@ -548,21 +544,26 @@ __device__ __forceinline__ int tile_index(int b, int n, int remap) {
 // cache line).
 constexpr size_t stage_lds(int nt) { return (size_t)(16 * nt / 256) * lds_pitch(256) * sizeof(float2); }
 
-// At most 128 VGPRs: four wavefronts per SIMD, what the LDS allows too.
+// At most 128 VGPRs: four wavefronts per SIMD, what the LDS allows too.  What finds
+// the record comes first: the build has the first eight words of kernel arguments
+// in scalar registers when a wavefront starts, which saves another latency before
+// the record's (100 x 50 room 6.05 -> 5.94 us per stage, 1024^2 31.0 -> 30.7).
 template <int NT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
-stage_fft_kernel(StageArgs a) {
+stage_fft_kernel(const TileDesc *tiles, int ntiles, int remap, StageArgs a) {
     extern __shared__ float2 lds_dyn[];
-    const Ref ref = (Ref)a.tiles + tile_index(blockIdx.x, gridDim.x, a.remap);
-    const Seg td = (Seg)a.segs + ref->seg;
+    const Seg td = (Seg)tiles + tile_index(blockIdx.x, ntiles, remap);
+    // one word of each of the record's 64-byte lines: fetched together, not one
+    // after the other as the code comes to need them
+    asm volatile("" ::"s"(td->kind), "s"(td->m_size), "s"(td->is_pml));
     switch (td->kind) {
         case 0:
-            if (td->F == 128) derivative_tile<8, NT, true, false>(a, td, ref, lds_dyn);
-            else if (fft_values(td->F) == 8) derivative_tile<8, NT, false, false>(a, td, ref, lds_dyn);
-            else if (NT == 512 && td->F == 8192) derivative_tile<16, NT, false, NT == 512>(a, td, ref, lds_dyn);
-            else derivative_tile<16, NT, false, false>(a, td, ref, lds_dyn);
+            if (td->F == 128) derivative_tile<8, NT, true, false>(a, td, lds_dyn);
+            else if (fft_values(td->F) == 8) derivative_tile<8, NT, false, false>(a, td, lds_dyn);
+            else if (NT == 512 && td->F == 8192) derivative_tile<16, NT, false, NT == 512>(a, td, lds_dyn);
+            else derivative_tile<16, NT, false, false>(a, td, lds_dyn);
             break;
-        case 1: passthrough_tile<NT>(a, td, ref); break;
+        case 1: passthrough_tile<NT>(a, td); break;
         case 2: sample_receivers(a); break;
         default: break;
     }
@@ -823,7 +824,6 @@ struct GemmTile {
     int n_g;               // outputs the multiplication produces (n_out, or n_out - 1 with the dot row)
     int d_exp;             // D was stored as D * 2^d_exp
     int K;                 // line length
-    int slot;              // of the first wavefront's maximum (track_max)
     int dot_off;           // >= 0: ftab offset of D's last row (FP32): this tile writes output n_out - 1
 };
 
@@ -1243,7 +1243,7 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
             write_dot((tid & 3) == 0 ? stage_line(tid, q) : -1, g);
         }
     }
-    track_max(a, gt.slot, mx);
+    track_max(a, gt.t.slot, mx);
 }
 
 template <typename E>
@@ -1359,8 +1359,7 @@ struct pstd_ctx {
     float *pml = nullptr;
     float2 *ctab = nullptr;
     float *ftab = nullptr;
-    TileDesc *d_segs = nullptr;
-    TileRef *d_tiles = nullptr;
+    TileDesc *d_tiles = nullptr;
     GemmTile *d_gemm = nullptr;
     void *dmat = nullptr;         // derivative matrices of the GEMM form (hi, lo parts; 2-byte elements)
     unsigned *umax = nullptr;     // maxima of the written values, scenes x 2 classes
@@ -1426,7 +1425,6 @@ struct pstd_ctx {
         (void)hipFree(ctab);
         (void)hipFree(ftab);
         (void)hipFree(d_tiles);
-        (void)hipFree(d_segs);
         (void)hipFree(d_gemm);
         (void)hipFree(dmat);
         (void)hipFree(umax);
@@ -1453,7 +1451,6 @@ struct pstd_ctx {
         arena = pml = ftab = d_samples = nullptr;
         ctab = nullptr;
         d_tiles = nullptr;
-        d_segs = nullptr;
         d_cells = nullptr;
         d_p0_tiles = nullptr;
         planned = false;
@@ -1502,7 +1499,7 @@ void build_window(int w, int patch_error, std::vector<float> &out) {
 // class of its longest lines.
 constexpr int kClassSmall = 0, kClass4096 = 1, kClass8192 = 2, kClassGemm = 3, kClasses = 4;
 
-typedef void (*StageKernel)(StageArgs);
+typedef void (*StageKernel)(const TileDesc *, int, int, StageArgs);
 StageKernel stage_kernel(int nt) {
     return nt <= 128 ? stage_fft_kernel<128> : nt <= 256 ? stage_fft_kernel<256> : stage_fft_kernel<512>;
 }
@@ -1544,7 +1541,6 @@ int launch_stage(pstd_ctx *ctx, int k, int sample_slot) {
     a.pml = ctx->pml;
     a.s = ctx->dt * ctx->alpha[k];
     a.last = k == 5;
-    a.remap = ctx->xcd_remap;
     const int ng = (int)ctx->tiles_gemm.size();
     if (ng) {
         a.wmax = ctx->wmax;
@@ -1569,9 +1565,7 @@ int launch_stage(pstd_ctx *ctx, int k, int sample_slot) {
         HIP_TRY(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
     }
     if (ns) timed_launch(ctx, fs, ctx->fmax >= 8192 ? kClass8192 : ctx->fmax >= 4096 ? kClass4096 : kClassSmall, [&] {
-        a.tiles = ctx->d_tiles;
-        a.segs = ctx->d_segs;
-        hipLaunchKernelGGL(stage_kernel(nt), dim3(ns), dim3(nt), stage_lds(nt), fs, a);
+        hipLaunchKernelGGL(stage_kernel(nt), dim3(ns), dim3(nt), stage_lds(nt), fs, (const TileDesc *)ctx->d_tiles, ns, ctx->xcd_remap, a);
     });
     if (fork) HIP_TRY(hipEventRecord(ctx->ev_join, ctx->side));
     if (ng) timed_launch(ctx, ctx->stream, kClassGemm, [&] {
@@ -1757,7 +1751,7 @@ static int enqueue_steps(pstd_ctx *ctx, int chunk, int base = 0) {
 // line0 + 2p + 1) are the same for every NT, so results do not depend on it.
 static int upload_tiles(pstd_ctx *ctx) {
     const int nt = ctx->stage_threads();
-    std::vector<TileRef> tiles;
+    std::vector<TileDesc> tiles;
     // the longest tiles first, so that none of them starts last — where there are
     // more wavefronts than the chip holds at once (4 x 1024 SIMDs); a scene that
     // fits is better off with its kinds of tiles mixed over the CUs
@@ -1771,30 +1765,34 @@ static int upload_tiles(pstd_ctx *ctx) {
     for (int k : order) {
         const TileDesc &g = ctx->fft_segs[k];
         const int per = g.kind == 0 ? 2 * nt / (g.F / fft_values(g.F)) : kPassChunk;
-        for (int l = 0; l < g.count; l += per) tiles.push_back({k, g.line0 + l, std::min(per, g.count - l), 0});
+        for (int l = 0; l < g.count; l += per) {
+            tiles.push_back(g);
+            tiles.back().line0 = g.line0 + l;
+            tiles.back().count = std::min(per, g.count - l);
+        }
     }
     ctx->n_tiles = (int)tiles.size();
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     if (!ctx->tiles_gemm.empty()) {
         // maxima slots: a group (scene, class) after the other
         const int groups = 2 * ctx->n_scenes;
-        auto group = [&](const TileRef &r) { return 2 * ctx->fft_segs[r.seg].scene + (ctx->fft_segs[r.seg].vel ? 0 : 1); };
+        auto group = [](const TileDesc &t) { return 2 * t.scene + (t.vel ? 0 : 1); };
         std::vector<int2> first(groups + 1, make_int2(0, 0));
-        auto writes = [&](const TileRef &r) { return ctx->fft_segs[r.seg].kind != 2; };  // (receivers store no maximum)
-        for (const TileRef &r : tiles)
-            if (writes(r)) first[group(r) + 1].x += nt / 64;
+        auto writes = [](const TileDesc &t) { return t.kind != 2; };  // (receivers store no maximum)
+        for (const TileDesc &t : tiles)
+            if (writes(t)) first[group(t) + 1].x += nt / 64;
         for (int i = 0; i < groups; ++i) first[i + 1].x += first[i].x;
         std::vector<int2> next = first;
-        for (TileRef &r : tiles) {
-            if (!writes(r)) continue;
-            int &n = next[group(r)].x;
-            r.slot = n;
+        for (TileDesc &t : tiles) {
+            if (!writes(t)) continue;
+            int &n = next[group(t)].x;
+            t.slot = n;
             n += nt / 64;
         }
         const int base = first[groups].x;
         for (int i = 0; i <= groups; ++i) first[i].y = base + ctx->gemm_first[i];
         std::vector<GemmTile> gemm = ctx->tiles_gemm;
-        for (GemmTile &t : gemm) t.slot += base;
+        for (GemmTile &t : gemm) t.t.slot += base;
         if (ctx->wmax) HIP_TRY(hipFree(ctx->wmax));
         ctx->wmax = nullptr;
         HIP_TRY(hipMalloc(&ctx->wmax, (size_t)(base + ctx->gemm_first.back()) * sizeof(float)));
@@ -1805,9 +1803,9 @@ static int upload_tiles(pstd_ctx *ctx) {
     }
     if (ctx->d_tiles) HIP_TRY(hipFree(ctx->d_tiles));
     ctx->d_tiles = nullptr;
-    HIP_TRY(hipMalloc(&ctx->d_tiles, std::max<size_t>(1, tiles.size()) * sizeof(TileRef)));
+    HIP_TRY(hipMalloc(&ctx->d_tiles, std::max<size_t>(1, tiles.size()) * sizeof(TileDesc)));
     if (!tiles.empty()) {
-        HIP_TRY(hipMemcpyAsync(ctx->d_tiles, tiles.data(), tiles.size() * sizeof(TileRef), hipMemcpyHostToDevice,
+        HIP_TRY(hipMemcpyAsync(ctx->d_tiles, tiles.data(), tiles.size() * sizeof(TileDesc), hipMemcpyHostToDevice,
                                ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
     }
@@ -2334,8 +2332,6 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         // in double: 1/rho for the velocity fields, rho*c1^2 for the pressure fields
         g.coef = s.field == 0 ? (float)(1.0 / (double)dm.rho) : (float)((double)dm.rho * plan->c1 * plan->c1);
         g.is_pml = dm.is_pml;
-        g.wlog = 0;
-        while ((1 << g.wlog) < s.wlen) ++g.wlog;
         g.m_dom = g.s1_dom = g.s2_dom = dm.base;
         g.m_size = g.s1_size = g.s2_size = dm.size;
         if (g.F < 128 || g.F > 8192) {
@@ -2531,10 +2527,6 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     HIP_TRY(hipMemcpyAsync(ctx->ctab, ctab.data(), ctab.size() * sizeof(float2), hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(hipMalloc(&ctx->ftab, ftab.size() * sizeof(float)));
     HIP_TRY(hipMemcpyAsync(ctx->ftab, ftab.data(), ftab.size() * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    HIP_TRY(hipMalloc(&ctx->d_segs, std::max<size_t>(1, ctx->fft_segs.size()) * sizeof(TileDesc)));
-    if (!ctx->fft_segs.empty())
-        HIP_TRY(hipMemcpyAsync(ctx->d_segs, ctx->fft_segs.data(), ctx->fft_segs.size() * sizeof(TileDesc),
-                               hipMemcpyHostToDevice, ctx->stream));
     if (!ctx->tiles_gemm.empty()) {
         // the GEMM tiles' maxima slots, numbered like those of upload_tiles
         const int groups = 2 * ctx->n_scenes;
@@ -2544,7 +2536,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         for (int i = 0; i < groups; ++i) ctx->gemm_first[i + 1] += ctx->gemm_first[i];
         std::vector<int> next = ctx->gemm_first;
         for (GemmTile &t : ctx->tiles_gemm) {
-            t.slot = next[group(t)];
+            t.t.slot = next[group(t)];
             next[group(t)] += kGemmThreads / 64;
         }
         // segment order (a scene's segments together, a line block's output
