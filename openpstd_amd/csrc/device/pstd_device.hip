@@ -765,12 +765,14 @@ __global__ void __launch_bounds__(256) transpose_kernel(const float *__restrict_
 //    two 2^e and split into two
 //    16-bit parts while they are staged into LDS (U = hi + lo: FP16 keeps 22
 //    bits when every scaled value is below 2^15, BF16 16 bits at any scale);
-//  * D is stored split the same way (one power of two per matrix), as the
-//    LDS images of its 32-k chunks, copied straight from memory into LDS;
+//  * D is stored split the same way (one power of two per matrix), in the order
+//    of the MFMA operands, and goes from memory to registers: every wave has 32
+//    outputs of its own and all of the tile's lines, so no part of D is loaded
+//    twice, and the LDS (reads and writes took as many of its cycles as the
+//    multiplication takes when D passed through it too) holds the lines only;
 //  * C = U_hi D_hi + U_hi D_lo + U_lo D_hi with v_mfma_f32_32x32x16_{f16,bf16},
 //    FP32 accumulation, over k-chunks of 32 through double-buffered LDS (one
-//    workgroup barrier per chunk; the loads of chunk c+1 are in flight while
-//    chunk c is multiplied);
+//    workgroup barrier per chunk, which waits for no load in flight);
 //  * the scene's scale comes from the largest |value| every wavefront of the
 //    previous stage wrote (track_max, max_reduce), so no pass over the inputs
 //    precedes the multiplication;
@@ -781,6 +783,13 @@ __global__ void __launch_bounds__(256) transpose_kernel(const float *__restrict_
 // U is on the MFMA A side (rows of C = lines, columns = outputs): consecutive
 // lanes store consecutive floats of a line, in both directions (vy and py are
 // stored column-major).
+// Measured (launch alone, D through the LDS -> D straight to registers and the
+// lines two chunks ahead): 1024^2 in BF16 53.6 -> 47.3 us, 16 scenes of 512 x 1024
+// twice in FP16 536 -> 492 us (335 GFLOP of products: 680 TFLOP/s, and 3.2 TB/s of
+// memory traffic).  Neither bounds it alone: without its MFMAs it takes three
+// quarters of the time, without its stores and t_n four fifths.  Three workgroups
+// per CU (168 registers, one chunk ahead) do the 16 scenes in 502 us and the one
+// scene, which has one workgroup per CU, in 62.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -799,25 +808,33 @@ struct MfmaOps<__bf16> {
     __device__ static f32x16 mfma(v8 a, v8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 };
 
-constexpr int kGemmThreads = 256;  // 4 waves: 2 line groups x 2 output groups of 64 x 64
+constexpr int kGemmThreads = 256;  // 4 waves, each all lines x 32 outputs
 constexpr int kGL = 128;           // lines per tile
 constexpr int kGN = 128;           // outputs per tile
 // (line, 8-k group) pieces of a chunk each thread stages: 2
 constexpr int kGSlots = kGL * 32 / 8 / kGemmThreads;
 constexpr int kGK = 32;            // k per LDS chunk (two MFMA k-steps)
-constexpr int kGP = kGK + 8;       // LDS row pitch in 2-byte elements (80 B: conflict-free 16-byte operand reads)
-constexpr int kGemmLdsU = 2 * 2 * kGL * kGP;  // elements: [buffer][part][line][k]
-constexpr int kGemmLdsD = 2 * 2 * kGN * kGP;  // elements: [buffer][part][output][k]
-constexpr size_t kGemmLdsBytes = (size_t)(kGemmLdsU + kGemmLdsD) * 2;  // 80 KiB: two workgroups per CU
-constexpr int kGemmDChunk = 2 * kGN * kGP;  // elements of one chunk's D image (both parts)
-static_assert(kGemmDChunk * 2 == 5 * 1024 * (kGemmThreads / 64), "D image: 5 KiB-loads per wave");
+constexpr int kGPart = kGL * kGK;            // elements of one part (hi or lo) of a chunk of U
+constexpr int kGemmDChunk = 2 * kGN * kGK;   // elements of one chunk of D (both parts)
+constexpr size_t kGemmLdsBytes = (size_t)2 * 2 * kGPart * 2;  // U: [buffer][part][line][k], 32 KiB
+// Element of (row, 8-k group g) in a part: rows of 64 bytes, the groups of a row
+// permuted so that 8 rows (32 banks) or 16 rows (64 banks) read with one group
+// touch every bank once.
+__host__ __device__ constexpr int gemm_slot(int row, int g) {
+    return row * kGK + ((g ^ ((row >> 1) & 3) ^ ((row >> 3) & 1)) * 8);
+}
+// Element of D's value (output, k) of a tile: the operands of one MFMA (32 outputs,
+// 16 k, one part) lie together in the order of the lanes that read them, as
+// [chunk][k-step][part][output / 32][lane][k % 8].
+__host__ __device__ constexpr long long gemm_d_at(int output, int k, int part) {
+    return (((long long)(k / 16) * 2 + part) * (kGN / 32) + output / 32) * 512 + (k / 8 % 2 * 32 + output % 32) * 8 + k % 8;
+}
 static_assert(kGSlots == 2, "staging map assumes two slots per thread");
 
 struct GemmTile {
     TileDesc t;            // segment addressing; line0/count: the tile's lines (count <= 128)
-    // D of the tile's 128 outputs as LDS images (2-byte elements): chunk c's
-    // image [part hi, lo][128 outputs][kGP] (k of the chunk, then zero pad) at
-    // element d_img + c * kGemmDChunk; d_len elements in all
+    // D of the tile's 128 outputs (2-byte elements): value (output, k, part hi or
+    // lo) at element d_img + gemm_d_at(); d_len elements in all
     long long d_img, d_len;
     int n_rows, k_pad;     // rows of D (multiple of kGN) and columns (multiple of kGK)
     int n0;                // first output of the tile
@@ -826,6 +843,7 @@ struct GemmTile {
     int K;                 // line length
     int dot_off;           // >= 0: ftab offset of D's last row (FP32): this tile writes output n_out - 1
 };
+typedef const __attribute__((address_space(4))) GemmTile *GTile;
 
 // Power of two that brings a line whose values are bounded by m below 2^15
 // (FP16 keeps both parts normal down to 2^-3 of that bound).
@@ -835,11 +853,10 @@ __device__ __forceinline__ int gemm_scale_exp(const StageArgs &a, int scene, int
     return m > 0.f ? min(max(14 - ilogbf(m), -100), 100) : 0;
 }
 
-// Raw input values of one chunk held by a thread: 8 consecutive k of one line
-// (4 threads per line, so 4 lanes read 128 contiguous bytes); dk: the FP32 dot
-// row's coefficients of these k.
+// Raw input values of one chunk held by a thread: 8 consecutive k of two lines
+// (4 threads per line, so 4 lanes read 128 contiguous bytes).
 struct UChunk {
-    float a[kGSlots][8], dk[kGSlots][8];
+    float a[kGSlots][8];
 };
 
 // Staging map of slot q: 4 threads per line, lines tid/4 and tid/4 + 64.
@@ -851,26 +868,22 @@ __device__ __forceinline__ Rsrc bytes_rsrc(const void *base, long long byte_off,
     return __builtin_amdgcn_make_buffer_rsrc((void *)((const char *)base + byte_off), (short)0, bytes, 0x00020000);
 }
 
-__device__ __forceinline__ float4 bload4(Rsrc r, int off_bytes) {
-    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off_bytes, 0, 0));
-}
-
 // Line `line` (absolute) of a tile: byte offsets of position k of its raw
 // input line in the three blocks it comes from (main, side1, side2).
 struct LineAddr {
     int w, nm, K;
     int m_base, s1_base, s2_base;  // offset of k = 0 of each piece (4 bytes per k)
     bool s1, s2;
-    __device__ LineAddr(const TileDesc &td, int line, int K_) {
-        const int vel = td.vel;
-        w = td.wlen;
-        nm = td.n_main;
+    __device__ __forceinline__ LineAddr(Seg td, int line, int K_) {
+        const int vel = td->vel;
+        w = td->wlen;
+        nm = td->n_main;
         K = K_;
-        m_base = (td.m_a + line * td.m_ls - w) * 4;
-        s1 = td.s1_len >= 0;
-        s2 = td.s2_len >= 0;
-        s1_base = (td.s1_a + (line + td.s1_line) * td.s1_ls + td.s1_len - w - vel) * 4;
-        s2_base = (td.s2_a + (line + td.s2_line) * td.s2_ls + vel - w - nm) * 4;
+        m_base = (td->m_a + line * td->m_ls - w) * 4;
+        s1 = td->s1_len >= 0;
+        s2 = td->s2_len >= 0;
+        s1_base = (td->s1_a + (line + td->s1_line) * td->s1_ls + td->s1_len - w - vel) * 4;
+        s2_base = (td->s2_a + (line + td->s2_line) * td->s2_ls + vel - w - nm) * 4;
     }
     __device__ int main_off(int k) const { return k >= w && k < w + nm ? m_base + k * 4 : kOOB; }
     __device__ int s1_off(int k) const { return s1 && k < w ? s1_base + k * 4 : kOOB; }
@@ -882,8 +895,8 @@ struct LineAddr {
 // read zero (a value from past the halo could be another field, outside the
 // range the scene's scale was chosen for).
 constexpr int kPieceMain = 0, kPieceS1 = 1, kPieceS2 = 2, kPieceMixed = 3, kPieceNone = 4;
-__device__ __forceinline__ int chunk_piece(const TileDesc &td, int K, int k0) {
-    const int w = td.wlen, nm = td.n_main;
+__device__ __forceinline__ int chunk_piece(Seg td, int K, int k0) {
+    const int w = td->wlen, nm = td->n_main;
     return k0 >= K                              ? kPieceNone
            : k0 >= w && k0 + kGK <= w + nm      ? kPieceMain
            : k0 + kGK <= w                      ? kPieceS1
@@ -898,115 +911,95 @@ __device__ __forceinline__ T pick3(int piece, T main, T s1, T s2) {
     return piece == kPieceMain ? main : piece == kPieceS1 ? s1 : s2;
 }
 // Buffer resource of one piece's domain block.
-__device__ __forceinline__ Rsrc piece_rsrc(const float *src, const TileDesc &td, int piece) {
-    return block_rsrc(src, pick3<long long>(piece, td.m_dom, td.s1_dom, td.s2_dom),
-                      pick3<int>(piece, td.m_size, td.s1_size, td.s2_size));
+__device__ __forceinline__ Rsrc piece_rsrc(const float *src, Seg td, int piece) {
+    return block_rsrc(src, pick3<long long>(piece, td->m_dom, td->s1_dom, td->s2_dom),
+                      pick3<int>(piece, td->m_size, td->s1_size, td->s2_size));
 }
 
-__device__ __forceinline__ void gemm_load_u1(const float *src, const TileDesc &td, const LineAddr &L, bool ok, int k0,
-                                             int q, Rsrc dotr, bool dot, UChunk &u) {
+// A chunk that is not all main values (one or two at either end of a line).
+__device__ __forceinline__ void gemm_load_ends(const float *src, Seg td, int K, const bool (&ok)[kGSlots], int k0,
+                                               UChunk &u) {
     const int kb = k0 + stage_kq(threadIdx.x);
-    const int piece = chunk_piece(td, L.K, k0);
-    if (piece == kPieceMixed) {
-        // a chunk across a piece boundary: each value from whichever block holds it
-        const Rsrc m = piece_rsrc(src, td, kPieceMain), s1 = piece_rsrc(src, td, kPieceS1),
-                   s2 = piece_rsrc(src, td, kPieceS2);
+    const int piece = chunk_piece(td, K, k0);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = kb + j;
-            const int om = ok ? L.main_off(k) : kOOB, o1 = ok ? L.s1_off(k) : kOOB, o2 = ok ? L.s2_off(k) : kOOB;
-            u.a[q][j] = bload(m, om) + bload(s1, o1) + bload(s2, o2);
+    for (int q = 0; q < kGSlots; ++q) {
+        const LineAddr L(td, td->line0 + stage_line(threadIdx.x, q), K);
+        if (piece == kPieceMixed) {
+            // a chunk across a piece boundary: each value from whichever block holds it
+            const Rsrc m = piece_rsrc(src, td, kPieceMain), s1 = piece_rsrc(src, td, kPieceS1),
+                       s2 = piece_rsrc(src, td, kPieceS2);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int k = kb + j;
+                const int om = ok[q] ? L.main_off(k) : kOOB, o1 = ok[q] ? L.s1_off(k) : kOOB,
+                          o2 = ok[q] ? L.s2_off(k) : kOOB;
+                u.a[q][j] = bload(m, om) + bload(s1, o1) + bload(s2, o2);
+            }
+        } else {
+            // one block for the whole chunk; side-2 chunks may run to the end of the
+            // block: 4-byte loads
+            const Rsrc r = piece_rsrc(src, td, piece);
+            const bool in = ok[q] && ((piece == kPieceS1 && L.s1) || (piece == kPieceS2 && L.s2));
+            const int base = piece == kPieceS1 ? L.s1_base : L.s2_base;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) u.a[q][j] = bload(r, in && kb + j < K ? base + (kb + j) * 4 : kOOB);
         }
-    } else {
-        // one block for the whole chunk
-        const Rsrc r = piece_rsrc(src, td, piece);
-        const bool in = ok && (piece == kPieceMain || (piece == kPieceS1 && L.s1) || (piece == kPieceS2 && L.s2));
-        const int base = pick3<int>(piece, L.m_base, L.s1_base, L.s2_base);
-        const int off = in && piece != kPieceNone ? base + kb * 4 : kOOB;
-        if (piece != kPieceS2) {
-            // inside a line: two 16-byte loads
-            const float4 x0 = bload4(r, off), x1 = bload4(r, off == kOOB ? kOOB : off + 16);
+    }
+}
+
+// The input lines of a tile.  In a chunk of main values every k lies in the
+// line's own block: a per-lane part of the byte offset (line and k-group; kOOB
+// for lanes past the tile's lines) and a uniform part (the chunk's k), both
+// non-negative.
+struct GemmLines {
+    const float *src;
+    Seg td;
+    int K;
+    bool ok[kGSlots];
+    Rsrc r;
+    int voff[kGSlots];
+    __device__ __forceinline__ void load_main(int c, UChunk &u) const {
+        const int so = (c * kGK - td->wlen) * 4;
+#pragma unroll
+        for (int q = 0; q < kGSlots; ++q) {
+            const float4 x0 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[q], so, 0));
+            const float4 x1 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[q] + 16, so, 0));
             u.a[q][0] = x0.x; u.a[q][1] = x0.y; u.a[q][2] = x0.z; u.a[q][3] = x0.w;
             u.a[q][4] = x1.x; u.a[q][5] = x1.y; u.a[q][6] = x1.z; u.a[q][7] = x1.w;
-        } else {
-            // side-2 chunks may run to the end of the block: 4-byte loads
-#pragma unroll
-            for (int j = 0; j < 8; ++j) u.a[q][j] = bload(r, off == kOOB || kb + j >= L.K ? kOOB : off + j * 4);
         }
     }
-    if (dot) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) u.dk[q][j] = bload(dotr, (kb + j) * 4);  // zero from K on
+    __device__ __forceinline__ void load(int c, UChunk &u) const {
+        if (chunk_piece(td, K, c * kGK) == kPieceMain) load_main(c, u);
+        else gemm_load_ends(src, td, K, ok, c * kGK, u);
     }
-}
-
-__device__ __forceinline__ void gemm_load_u(const float *src, const TileDesc &td, const LineAddr (&L)[kGSlots],
-                                            const bool (&ok)[kGSlots], int k0, Rsrc dotr, bool dot, UChunk &u) {
-#pragma unroll
-    for (int q = 0; q < kGSlots; ++q) gemm_load_u1(src, td, L[q], ok[q], k0, q, dotr, dot, u);
-}
-
-// Main-piece addressing of a tile's lines: every k of a main chunk lies in the
-// line's own block, so the byte offset splits into a per-lane part (line and
-// k-group; kOOB for lanes past the tile's lines) and a uniform part (the
-// chunk's k, passed as the buffer instruction's scalar offset).  Both parts
-// are non-negative.
-struct MainU {
-    Rsrc r;
-    int voff[kGSlots];  // per lane and slot
-    int kofs;           // k of the first main position (the line's halo length)
 };
 
-__device__ __forceinline__ MainU main_u(const float *src, const TileDesc &td, const bool (&ok)[kGSlots]) {
-    MainU m;
-    m.r = block_rsrc(src, td.m_dom, td.m_size);
-    m.kofs = td.wlen;
+// A wave's operands of a chunk of D: 32 outputs, straight from memory to
+// registers (1 KiB per load; the matrix stays in the caches).
+template <typename E>
+struct DChunk {
+    typename MfmaOps<E>::v8 b[2][2];  // [k-step][part]
+    __device__ __forceinline__ void load(Rsrc dr, int voff, int c) {
 #pragma unroll
-    for (int q = 0; q < kGSlots; ++q) {
-        const int line = td.line0 + stage_line(threadIdx.x, q);
-        m.voff[q] = ok[q] ? (td.m_a + line * td.m_ls + stage_kq(threadIdx.x)) * 4 : kOOB;
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                b[s][p] = __builtin_bit_cast(typename MfmaOps<E>::v8, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 dr, voff, c * kGemmDChunk * 2 + (s * 2 + p) * (kGN / 32) * 1024, 0));
     }
-    return m;
-}
-
-__device__ __forceinline__ void gemm_load_u_main(const MainU &m, int k0, Rsrc dotr, bool dot, UChunk &u) {
-    const int so = (k0 - m.kofs) * 4;  // >= 0 in a main chunk
-#pragma unroll
-    for (int q = 0; q < kGSlots; ++q) {
-        const float4 x0 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.r, m.voff[q], so, 0));
-        const float4 x1 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(m.r, m.voff[q] + 16, so, 0));
-        u.a[q][0] = x0.x; u.a[q][1] = x0.y; u.a[q][2] = x0.z; u.a[q][3] = x0.w;
-        u.a[q][4] = x1.x; u.a[q][5] = x1.y; u.a[q][6] = x1.z; u.a[q][7] = x1.w;
-        if (dot) {
-            const int kb = k0 + stage_kq(threadIdx.x);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) u.dk[q][j] = bload(dotr, (kb + j) * 4);
-        }
-    }
-}
-
-// Copies chunk c of the tile's D image into LDS buffer `dbuf` (20 KiB, straight
-// from memory into LDS: 20 wavefront loads of 1 KiB, 5 per wave).
-__device__ __forceinline__ void gemm_dma_d(const Rsrc &dr, void *dbuf, int c) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-    for (int j = 0; j < kGemmDChunk * 2 / 1024 / (kGemmThreads / 64); ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(dr, (char *)dbuf + (j * (kGemmThreads / 64) + w) * 1024, 16,
-                                                 lane * 16 + w * 1024, c * kGemmDChunk * 2 + j * 4096, 0, 0);
-}
+};
 
 // Converts and writes one chunk into LDS buffer `buf` (8 k of one line per
-// thread as one 16-byte write per part); accumulates the FP32 dot product of
-// the last output row (dot).
+// thread as one 16-byte write per part).
 template <typename E>
-__device__ __forceinline__ void gemm_stage(E *ulds, int buf, const UChunk &u, float sc, bool dot,
-                                           float (&gv)[kGSlots]) {
+__device__ __forceinline__ void gemm_stage(E *ulds, int buf, const UChunk &u, float sc) {
     using V8 = typename MfmaOps<E>::v8;
     const int tid = threadIdx.x;
-    E *U0 = ulds + (buf * 2 + 0) * kGL * kGP, *U1 = ulds + (buf * 2 + 1) * kGL * kGP;
+    E *U0 = ulds + buf * 2 * kGPart, *U1 = U0 + kGPart;
 #pragma unroll
     for (int q = 0; q < kGSlots; ++q) {
-        const int row = stage_line(tid, q), kq = stage_kq(tid);
+        // (a slot's rows lie 64 apart: the same permutation)
+        const int at = gemm_slot(stage_line(tid, 0), tid & 3) + q * (kGemmThreads / 4) * kGK;
         V8 hi, lo;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -1015,219 +1008,227 @@ __device__ __forceinline__ void gemm_stage(E *ulds, int buf, const UChunk &u, fl
             hi[j] = h;
             lo[j] = (E)(x - (float)h);
         }
-        *reinterpret_cast<V8 *>(U0 + row * kGP + kq) = hi;
-        *reinterpret_cast<V8 *>(U1 + row * kGP + kq) = lo;
-    }
-    // the dot row (a uniform branch: only the last output tile of a line block)
-    if (dot) {
-#pragma unroll
-        for (int q = 0; q < kGSlots; ++q)
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                gv[q] = __builtin_fmaf(u.a[q][j], u.dk[q][j], gv[q]);
+        *reinterpret_cast<V8 *>(U0 + at) = hi;
+        *reinterpret_cast<V8 *>(U1 + at) = lo;
     }
 }
 
-// The MFMAs of one chunk (LDS buffer `buf`): wave (lg, og) accumulates lines
-// 64 lg .. +63 x outputs 64 og .. +63 (2 x 2 blocks of 32 x 32).
-template <typename E>
-__device__ __forceinline__ void gemm_chunk(const E *ulds, const E *dlds, int buf, int lg, int og, int dir,
-                                           f32x16 (&acc)[2][2]) {
+// The chunk's part of the lines' FP32 dot products with the last output row
+// (dotr; only in the last output tile of a line block).
+__device__ __forceinline__ void gemm_dot(const UChunk &u, Rsrc dotr, int c, float (&gv)[kGSlots]) {
+    float dk[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) dk[j] = bload(dotr, (c * kGK + stage_kq(threadIdx.x) + j) * 4);  // zero from K on
+#pragma unroll
+    for (int q = 0; q < kGSlots; ++q)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) gv[q] = __builtin_fmaf(u.a[q][j], dk[j], gv[q]);
+}
+
+// The MFMAs of one chunk (U0: its buffer): the tile's 128 lines (4 blocks of 32)
+// x the wave's 32 outputs.
+template <typename E, int DIR>
+__device__ __forceinline__ void gemm_chunk(const E *U0, const DChunk<E> &d, f32x16 (&acc)[4]) {
     using V8 = typename MfmaOps<E>::v8;
     const int lane = threadIdx.x & 63;
-    const E *U0 = ulds + (buf * 2 + 0) * kGL * kGP, *U1 = ulds + (buf * 2 + 1) * kGL * kGP;
-    const E *D0 = dlds + (buf * 2 + 0) * kGN * kGP, *D1 = dlds + (buf * 2 + 1) * kGN * kGP;
 #pragma unroll
     for (int s = 0; s < kGK / 16; ++s) {
-        const int kk = s * 16 + (lane >> 5) * 8;
-        V8 ah[2], al[2], bh[2], bl[2];
+        // (rows 32 apart: the same permutation)
+        const int at = gemm_slot(lane & 31, 2 * s + (lane >> 5));
+        V8 ah[4], al[4];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int rr = (64 * lg + 32 * i + (lane & 31)) * kGP + kk, qq = (64 * og + 32 * i + (lane & 31)) * kGP + kk;
-            ah[i] = *reinterpret_cast<const V8 *>(U0 + rr);
-            al[i] = *reinterpret_cast<const V8 *>(U1 + rr);
-            bh[i] = *reinterpret_cast<const V8 *>(D0 + qq);
-            bl[i] = *reinterpret_cast<const V8 *>(D1 + qq);
+        for (int i = 0; i < 4; ++i) {
+            ah[i] = *reinterpret_cast<const V8 *>(U0 + at + 32 * i * kGK);
+            al[i] = *reinterpret_cast<const V8 *>(U0 + kGPart + at + 32 * i * kGK);
         }
         // each product over the four independent accumulators in turn (no
         // back-to-back MFMAs on one accumulator); the low parts of D first for X
         // lines, those of U for Y lines (a fixed order of the sums per direction)
-        auto product = [&](const V8 (&x)[2], const V8 (&y)[2]) __attribute__((always_inline)) {
+        auto product = [&](const V8 (&x)[4], const V8 &y) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = MfmaOps<E>::mfma(x[i], y[j], acc[i][j]);
+            for (int i = 0; i < 4; ++i) acc[i] = MfmaOps<E>::mfma(x[i], y, acc[i]);
         };
-        product(ah, bh);
-        if (dir == 0) {
-            product(ah, bl);
-            product(al, bh);
+        product(ah, d.b[s][0]);
+        if constexpr (DIR == 0) {
+            product(ah, d.b[s][1]);
+            product(al, d.b[s][0]);
         } else {
-            product(al, bh);
-            product(ah, bl);
+            product(al, d.b[s][0]);
+            product(ah, d.b[s][1]);
         }
     }
 }
 
-template <typename E>
-__device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt, const float *ftab,
-                                          unsigned char *gemm_lds) {
+// The workgroup's LDS writes become visible; loads in flight are not waited for.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <typename E, int DIR>
+__device__ __forceinline__ void gemm_tile(const StageArgs &a, GTile gt, const float *ftab, unsigned char *gemm_lds) {
     E *ulds = reinterpret_cast<E *>(gemm_lds);
-    E *dlds = ulds + kGemmLdsU;
-    const TileDesc &td = gt.t;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lg = wave >> 1, og = wave & 1;
-    const int e = gemm_scale_exp(a, td.scene, td.vel);
+    const Seg td = &gt->t;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int e = gemm_scale_exp(a, td->scene, td->vel);
     const float sc = ldexpf(1.f, e);
-    const float *src = source(a, td.vel);
-    const Rsrc dr = bytes_rsrc(a.dmat, gt.d_img * 2, (int)(gt.d_len * 2));
-    const bool dot = gt.dot_off >= 0;
-    const Rsrc dotr = bytes_rsrc(ftab, dot ? (long long)gt.dot_off * 4 : 0, dot ? gt.K * 4 : 0);
-    const int nch = gt.k_pad / kGK;
-    bool line_ok[kGSlots];
+    const Rsrc dr = bytes_rsrc(a.dmat, gt->d_img * 2, (int)(gt->d_len * 2));
+    const bool dot = gt->dot_off >= 0;
+    const int nch = gt->k_pad / kGK;
+    GemmLines in;
+    in.src = source(a, td->vel);
+    in.td = td;
+    in.K = gt->K;
+    in.r = block_rsrc(in.src, td->m_dom, td->m_size);
 #pragma unroll
-    for (int q = 0; q < kGSlots; ++q) line_ok[q] = stage_line(tid, q) < td.count;
-    const LineAddr L[kGSlots] = {LineAddr(td, td.line0 + stage_line(tid, 0), gt.K),
-                                 LineAddr(td, td.line0 + stage_line(tid, 1), gt.K)};
-    // waves whose lines or outputs lie outside the tile skip their MFMAs
-    const bool active = 64 * lg < td.count && 64 * og < gt.n_g - gt.n0;
-    f32x16 acc[2][2];
+    for (int q = 0; q < kGSlots; ++q) {
+        in.ok[q] = stage_line(tid, q) < td->count;
+        in.voff[q] = in.ok[q] ? (td->m_a + (td->line0 + stage_line(tid, q)) * td->m_ls + stage_kq(tid)) * 4 : kOOB;
+    }
+    const Rsrc dotr = bytes_rsrc(ftab, dot ? (long long)gt->dot_off * 4 : 0, dot ? in.K * 4 : 0);
+    // waves whose outputs lie outside the tile skip their MFMAs
+    const bool active = 32 * wave < gt->n_g - gt->n0;
+    f32x16 acc[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+        for (int q = 0; q < 16; ++q) acc[i][q] = 0.f;
     float gv[kGSlots] = {0.f, 0.f};
-    // One register set: the loads of chunk c+1 are issued right after the
-    // barrier that makes chunk c visible, and are in flight while the MFMAs of
-    // chunk c run; then chunk c+1 is converted into the other LDS buffer.
-    UChunk u;
-    gemm_load_u(src, td, L, line_ok, 0, dotr, dot, u);
-    gemm_dma_d(dr, dlds, 0);
-    gemm_stage<E>(ulds, 0, u, sc, dot, gv);
-    __syncthreads();
-    // Chunks whose every k lies in the main piece, [cm0, cm1), load through
-    // MainU (no per-chunk piece logic); the halo chunks around them through
-    // the generic loader.  c: the chunk whose MFMAs run next; chunk c + 1 loads.
-    const int cm0 = (td.wlen + kGK - 1) / kGK, cm1 = max(cm0, (td.wlen + td.n_main) / kGK);
+    // While chunk c is multiplied, the lines of chunk c + 2 and D of chunk c + 1 are
+    // on their way to registers, and the lines of chunk c + 1, requested an iteration
+    // before, are then converted into the other LDS buffer.
+    UChunk u0, u1;
+    DChunk<E> da, db;
+    const int dv = (wave * 64 + lane) * 16;
+    in.load(0, u0);
+    da.load(dr, dv, 0);
+    if (nch > 1) in.load(1, u1);
+    gemm_stage<E>(ulds, 0, u0, sc);
+    if (dot) gemm_dot(u0, dotr, 0, gv);
+    lds_barrier();
     int c = 0;
-    auto step = [&](auto load_next) {
-        const int buf = c & 1;
-        load_next((c + 1) * kGK);
-        // D of chunk c + 1 into the other buffer (read last before the previous barrier)
-        gemm_dma_d(dr, dlds + (buf ^ 1) * kGemmDChunk, c + 1);
-        if (active) gemm_chunk<E>(ulds, dlds, buf, lg, og, td.dir, acc);
-        gemm_stage<E>(ulds, buf ^ 1, u, sc, dot, gv);
-        __syncthreads();  // also waits for the D copy
+    // chunk c + 2 is of main values: no branch between its loads and their use
+    auto step_main = [&](auto mult, auto parity, const DChunk<E> &d, DChunk<E> &next) __attribute__((always_inline)) {
+        constexpr int buf = decltype(parity)::value;
+        UChunk &cur = buf ? u0 : u1, &after = buf ? u1 : u0;
+        if constexpr (decltype(mult)::value) next.load(dr, dv, c + 1);
+        in.load_main(c + 2, after);
+        if constexpr (decltype(mult)::value) {
+            gemm_chunk<E, DIR>(ulds + buf * 2 * kGPart, d, acc);
+        }
+        gemm_stage<E>(ulds, buf ^ 1, cur, sc);
+        if (dot) gemm_dot(cur, dotr, c + 1, gv);
+        lds_barrier();
         ++c;
     };
-    auto generic = [&](int k0) { gemm_load_u(src, td, L, line_ok, k0, dotr, dot, u); };
-    while (c + 1 < min(cm0, nch)) step(generic);
-    {
-        const MainU m = main_u(src, td, line_ok);
-        // the same step with the LDS buffer parity known at compile time
-        // (LDS addresses as immediate offsets): two chunks per iteration
-        auto step_p = [&](auto parity) {
-            constexpr int buf = decltype(parity)::value;
-            gemm_load_u_main(m, (c + 1) * kGK, dotr, dot, u);
-            gemm_dma_d(dr, dlds + (buf ^ 1) * kGemmDChunk, c + 1);
-            if (active) gemm_chunk<E>(ulds, dlds, buf, lg, og, td.dir, acc);
-            gemm_stage<E>(ulds, buf ^ 1, u, sc, dot, gv);
-            __syncthreads();
-            ++c;
-        };
-        using P0 = std::integral_constant<int, 0>;
-        using P1 = std::integral_constant<int, 1>;
-        if ((c & 1) && c + 1 < cm1) step_p(P1{});
-        while (c + 2 < cm1) {
-            step_p(P0{});
-            step_p(P1{});
+    auto step_end = [&](auto parity, const DChunk<E> &d, DChunk<E> &next) __attribute__((always_inline)) {
+        constexpr int buf = decltype(parity)::value;
+        const bool more = c + 1 < nch;
+        UChunk &cur = buf ? u0 : u1, &after = buf ? u1 : u0;
+        if (more) next.load(dr, dv, c + 1);
+        if (c + 2 < nch) in.load(c + 2, after);
+        if (active) gemm_chunk<E, DIR>(ulds + buf * 2 * kGPart, d, acc);
+        if (more) {
+            gemm_stage<E>(ulds, buf ^ 1, cur, sc);
+            if (dot) gemm_dot(cur, dotr, c + 1, gv);
+            lds_barrier();
         }
-        if (c + 1 < cm1) step_p(P0{});
+        ++c;
+    };
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    // main chunks: [1, cm1) (a halo is at most 32 long)
+    const int cm1 = (td->wlen + td->n_main) / kGK;
+    if (active) {
+#pragma unroll 1
+        while (c + 3 < cm1) {
+            step_main(P1{}, P0{}, da, db);
+            step_main(P1{}, P1{}, db, da);
+        }
+    } else {
+#pragma unroll 1
+        while (c + 3 < cm1) {
+            step_main(P0{}, P0{}, da, db);
+            step_main(P0{}, P1{}, db, da);
+        }
     }
-    while (c + 1 < nch) step(generic);
-    if (active) gemm_chunk<E>(ulds, dlds, c & 1, lg, og, td.dir, acc);
-    __syncthreads();
+#pragma unroll 1
+    while (true) {
+        step_end(P0{}, da, db);
+        if (c >= nch) break;
+        step_end(P1{}, db, da);
+        if (c >= nch) break;
+    }
     // epilogue: L = C / (2^e 2^d_exp); out = t_n - s*coef*L (Solver::update_field_values)
-    const float sc_upd = a.s * td.coef, inv = ldexpf(1.f, -(e + gt.d_exp));
-    const bool use_pml = a.last && td.is_pml;
-    const Rsrc rt = block_rsrc(a.tn, td.m_dom, td.m_size);
-    const Rsrc rp = block_rsrc(a.pml, td.m_dom, td.m_size);
-    const Rsrc ro = block_rsrc(a.out, td.m_dom, td.m_size);
+    const float sc_upd = a.s * td->coef, inv = ldexpf(1.f, -(e + gt->d_exp));
+    const bool use_pml = a.last && td->is_pml;
+    const Rsrc rt = block_rsrc(a.tn, td->m_dom, td->m_size);
+    const Rsrc rp = block_rsrc(a.pml, td->m_dom, td->m_size);
+    const Rsrc ro = block_rsrc(a.out, td->m_dom, td->m_size);
     float mx = 0.f;
     if (active) {
-        // value q of block (i, j): row 32 i + 8 (q >> 2) + 4 (lane >> 5) + (q & 3), column 32 j + (lane & 31)
-        // of the wave's 64 x 64; all t_n loads are issued before the first is used
-        const int lrow0 = 64 * lg + 4 * (lane >> 5), nrow0 = gt.n0 + 64 * og + (lane & 31);
-        auto offset = [&](int i, int j, int q, bool &ok) {
-            const int line = lrow0 + 32 * i + 8 * (q >> 2) + (q & 3), n = nrow0 + 32 * j;
-            ok = line < td.count && n < gt.n_g;
-            return ok ? (td.o_f + (td.line0 + line) * td.o_ls + n) * 4 : kOOB;
+        // value q of block i: line 32 i + 8 (q >> 2) + 4 (lane >> 5) + (q & 3), output 32 wave + (lane & 31)
+        // of the tile; all t_n loads are issued before the first is used.  A per-lane
+        // offset and, per value, a uniform one (the buffer instruction's scalar offset;
+        // no address arithmetic on the vector unit) — lines past the tile's last by
+        // their own condition
+        const int line0 = 4 * (lane >> 5), n = gt->n0 + 32 * wave + (lane & 31);
+        const int base = n < gt->n_g ? (td->o_f + (td->line0 + line0) * td->o_ls + n) * 4 : kOOB;
+        auto line = [](int i, int q) { return 32 * i + 8 * (q >> 2) + (q & 3); };
+        // (what a block of 16 values is addressed with, anew for each pass over them)
+        struct Rows {
+            int left, ls4;  // lines from this lane's first on; bytes from line to line
         };
-        float tnv[2][2][16];
-        if (64 * lg + 64 <= td.count && 64 * og + 64 <= gt.n_g - gt.n0) {
-            // the wave's whole 64 x 64 block lies inside the tile: a per-lane
-            // offset and, per value, a uniform one (the buffer instruction's
-            // scalar offset; no address arithmetic on the vector unit)
-            const int base = (td.o_f + (td.line0 + lrow0) * td.o_ls + nrow0) * 4;
-            const int sl = td.o_ls * 4;
-            auto uoff = [&](int i, int j, int q) { return (32 * i + 8 * (q >> 2) + (q & 3)) * sl + 128 * j; };
+        auto rows = [&]() __attribute__((always_inline)) {
+            Rows r{td->count - line0, again(td->o_ls) * 4};
+            asm volatile("" : "+v"(r.left));
+            return r;
+        };
+        auto offset = [&](const Rows &r, int i, int q) __attribute__((always_inline)) {
+            return line(i, q) < r.left ? base : kOOB;
+        };
+        float y[4][16];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 4; ++i) {
+            const Rows r = rows();
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+            for (int q = 0; q < 16; ++q) y[i][q] = bload(rt, offset(r, i, q), line(i, q) * r.ls4);
+        }
 #pragma unroll
-                    for (int q = 0; q < 16; ++q)
-                        tnv[i][j][q] = __builtin_bit_cast(
-                            float, __builtin_amdgcn_raw_buffer_load_b32(rt, base, uoff(i, j, q), 0));
+        for (int i = 0; i < 4; ++i) {
+            const Rows r = rows();
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int q = 0; q < 16; ++q) {
+                y[i][q] = __builtin_fmaf(-sc_upd, acc[i][q] * inv, y[i][q]);
+                const int o = offset(r, i, q);
+                bstore(ro, o, line(i, q) * r.ls4, y[i][q]);
+                mx = fmaxf(mx, o == kOOB ? 0.f : fabsf(y[i][q]));
+            }
+        }
+        if (a.last) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+            for (int i = 0; i < 4; ++i) {
+                const Rows r = rows();
+                if (use_pml) {
+                    float pm[16];
 #pragma unroll
-                    for (int q = 0; q < 16; ++q) {
-                        const int so = uoff(i, j, q);
-                        const float nv = __builtin_fmaf(-sc_upd, acc[i][j][q] * inv, tnv[i][j][q]);
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, nv), ro, base, so, 0);
-                        if (a.last) {
-                            const float pm = use_pml ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                                                  rp, base, so, 0))
-                                                     : 1.f;
-                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, nv * pm), rt, base, so, 0);
-                        }
-                        mx = fmaxf(mx, fabsf(nv));
-                    }
-        } else {
+                    for (int q = 0; q < 16; ++q) pm[q] = bload(rp, offset(r, i, q), line(i, q) * r.ls4);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+                    for (int q = 0; q < 16; ++q) y[i][q] *= pm[q];
+                }
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) {
-                        bool ok;
-                        tnv[i][j][q] = bload(rt, offset(i, j, q, ok));
-                    }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) {
-                        bool ok;
-                        const int off = offset(i, j, q, ok);
-                        const float nv = __builtin_fmaf(-sc_upd, acc[i][j][q] * inv, tnv[i][j][q]);
-                        bstore(ro, off, 0, nv);
-                        if (a.last) bstore(rt, off, 0, nv * (use_pml ? bload(rp, off) : 1.f));
-                        if (ok) mx = fmaxf(mx, fabsf(nv));
-                    }
+                for (int q = 0; q < 16; ++q) bstore(rt, offset(r, i, q), line(i, q) * r.ls4, y[i][q]);
+            }
         }
     }
     if (dot) {
         // output n_out - 1 of every line: the FP32 dot products (no scaling)
-        const int n = gt.n_g;
+        const int n = gt->n_g;
         auto write_dot = [&](int line, float Ldot) {
-            if (line < 0 || line >= td.count) return;
-            const int off = (td.o_f + (td.line0 + line) * td.o_ls + n) * 4;
+            if (line < 0 || line >= td->count) return;
+            const int off = (td->o_f + (td->line0 + line) * td->o_ls + n) * 4;
             const float tnv = bload(rt, off), pm = use_pml ? bload(rp, off) : 1.f;
             const float nv = __builtin_fmaf(-sc_upd, Ldot, tnv);
             bstore(ro, off, 0, nv);
@@ -1238,22 +1239,23 @@ __device__ __forceinline__ void gemm_tile(const StageArgs &a, const GemmTile &gt
 #pragma unroll
         for (int q = 0; q < kGSlots; ++q) {
             float g = gv[q];
-            g += __shfl_xor(g, td.dir == 0 ? 1 : 2);
-            g += __shfl_xor(g, td.dir == 0 ? 2 : 1);
+            g += __shfl_xor(g, DIR == 0 ? 1 : 2);
+            g += __shfl_xor(g, DIR == 0 ? 2 : 1);
             write_dot((tid & 3) == 0 ? stage_line(tid, q) : -1, g);
         }
     }
-    track_max(a, gt.t.slot, mx);
+    track_max(a, td->slot, mx);
 }
 
 template <typename E>
-__global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2))) stage_gemm_kernel(StageArgs a, const GemmTile *__restrict__ tiles,
-                                                                  const float *__restrict__ ftab) {
+__global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2)))
+stage_gemm_kernel(StageArgs a, const GemmTile *__restrict__ tiles, const float *__restrict__ ftab) {
     extern __shared__ __attribute__((aligned(16))) unsigned char gemm_lds[];
     // XCD-contiguous runs of tiles always (the tiles of one matrix and of one
     // line block share an XCD's L2), whatever order the FFT-form tiles use
-    const GemmTile gt = tiles[tile_index(blockIdx.x, gridDim.x, 1)];
-    gemm_tile<E>(a, gt, ftab, gemm_lds);
+    const GTile gt = (GTile)tiles + tile_index(blockIdx.x, gridDim.x, 1);
+    if (gt->t.dir == 0) gemm_tile<E, 0>(a, gt, ftab, gemm_lds);
+    else gemm_tile<E, 1>(a, gt, ftab, gemm_lds);
 }
 
 // Largest |p0| and |vx|, |vy| of every scene in the state a first stage reads
@@ -1684,13 +1686,9 @@ int pstd_ctx_create(int device, pstd_ctx **out) {
     if (hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess) ctx->side = nullptr;
     if (hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess) ctx->ev_fork = nullptr;
     if (hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess) ctx->ev_join = nullptr;
-    // more than 64 KiB of LDS per workgroup: 512-thread stage blocks, the GEMM kernel
+    // more than 64 KiB of LDS per workgroup: 512-thread stage blocks
     const hipFuncAttribute attr = hipFuncAttributeMaxDynamicSharedMemorySize;
-    bool lds_ok = hipFuncSetAttribute((const void *)stage_kernel(512), attr, stage_lds(512)) == hipSuccess;
-    lds_ok = lds_ok &&
-             hipFuncSetAttribute((const void *)stage_gemm_kernel<_Float16>, attr, kGemmLdsBytes) == hipSuccess &&
-             hipFuncSetAttribute((const void *)stage_gemm_kernel<__bf16>, attr, kGemmLdsBytes) == hipSuccess;
-    if (!lds_ok) {
+    if (hipFuncSetAttribute((const void *)stage_kernel(512), attr, stage_lds(512)) != hipSuccess) {
         ctx->err = "cannot reserve LDS for the long-line kernels";
     }
     unsigned *sp = nullptr;
@@ -2024,7 +2022,7 @@ static int add_gemm_tiles(pstd_ctx *ctx, const pstd_plan_desc *plan, const pstd_
         for (int i = 0; i < n_g; ++i)
             for (int k = 0; k < K; ++k) dm = std::max(dm, std::fabs(D[(size_t)i * K + k]));
         const int d_exp = dm > 0 ? 14 - std::ilogb(dm) : 0;
-        // LDS images: for every 128-output block b and chunk c, [hi, lo][128 rows][kGP]
+        // for every 128-output block, its chunks (gemm_d_at)
         const long long hi = (long long)dmat.size();
         dmat.resize(dmat.size() + (size_t)(n_rows / kGN) * nch * kGemmDChunk, 0);
         for (int i = 0; i < n_g; ++i)
@@ -2032,9 +2030,9 @@ static int add_gemm_tiles(pstd_ctx *ctx, const pstd_plan_desc *plan, const pstd_
                 const double v = std::ldexp(D[(size_t)i * K + k], d_exp);
                 const uint16_t h = bf16 ? to_bf16_bits(v) : to_f16_bits(v);
                 const double hv = bf16 ? from_bf16_bits(h) : from_f16_bits(h);
-                const size_t at = hi + ((size_t)(i / kGN) * nch + k / kGK) * kGemmDChunk + (size_t)(i % kGN) * kGP + k % kGK;
-                dmat[at] = h;
-                dmat[at + (size_t)kGN * kGP] = bf16 ? to_bf16_bits(v - hv) : to_f16_bits(v - hv);
+                const size_t tile = hi + (size_t)(i / kGN) * nch * kGemmDChunk;
+                dmat[tile + gemm_d_at(i % kGN, k, 0)] = h;
+                dmat[tile + gemm_d_at(i % kGN, k, 1)] = bf16 ? to_bf16_bits(v - hv) : to_f16_bits(v - hv);
             }
         int dot_off = -1;
         if (dot_row) {
