@@ -75,7 +75,8 @@ __device__ __forceinline__ void dft(float2 *a) {
     else dft8(a);
 }
 
-// Values per thread; pass schedule: radix of pass p for length F <= 4096.  An
+// Values per thread (1024 and 2048 points: or 8, fft_run's V); pass schedule: radix of
+// pass p for length F <= 4096.  An
 // 8192-point pair is two 4096-point sequences (split_first), each with 8 values
 // per thread: T = 512, 16 values in all.
 __host__ __device__ constexpr int fft_values(int F) { return F <= 512 ? 8 : 16; }
@@ -206,11 +207,11 @@ __device__ __forceinline__ void fft_passes(float2 *v, int t, float2 *lds, const 
     }
 }
 
-template <int F>
+template <int F, int V>
 __device__ __forceinline__ void fft_run(float2 *v, int t, float2 *lds, const Table &tab, int tw) {
     const float2 w0[kTwPass] = {};
     if constexpr (F == 8192) fft_passes<4096, 512, 2, 0>(v, t, lds, tab, tw, w0);
-    else fft_passes<F, F / fft_values(F), 1, 0>(v, t, lds, tab, tw, w0);
+    else fft_passes<F, F / V, 1, 0>(v, t, lds, tab, tw, w0);
 }
 
 // 8192 points as two sequences of 4096: with W = exp(-2 pi i / 8192), the even bins

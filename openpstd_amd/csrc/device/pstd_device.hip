@@ -134,6 +134,7 @@ struct StageArgs {
     float *wmax;
     const unsigned *umax;
     const void *dmat;  // derivative matrices (2-byte elements)
+    int f8;            // longest lines with 8 values per thread (pstd_ctx::values)
 };
 
 // ------------------------------------------------------------- device code
@@ -450,8 +451,8 @@ __device__ __forceinline__ void derivative_tile(const StageArgs &a, Seg td, floa
         asm volatile("" : "+v"(ti));  // LDS addresses per pass, not kept for all lengths across the loop
 #define PSTD_FFT_CASE(FV)                                                                            \
     case FV:                                                                                         \
-        if constexpr (fft_values(FV) == V && FV <= V * NT && (FV == 128) == SHORT && (FV == 8192) == SPLIT) \
-            fft_run<FV>(v, ti, buf, tab, tw);                                                         \
+        if constexpr ((fft_values(FV) == V || (FV <= 2048 && V == 8)) && FV <= V * NT && (FV == 128) == SHORT && (FV == 8192) == SPLIT) \
+            fft_run<FV, V>(v, ti, buf, tab, tw);                                                        \
         break;
         switch (F) {
             PSTD_FFT_CASE(128)
@@ -559,7 +560,7 @@ stage_fft_kernel(const TileDesc *tiles, int ntiles, int remap, StageArgs a) {
     switch (td->kind) {
         case 0:
             if (td->F == 128) derivative_tile<8, NT, true, false>(a, td, lds_dyn);
-            else if (fft_values(td->F) == 8) derivative_tile<8, NT, false, false>(a, td, lds_dyn);
+            else if (td->F <= a.f8) derivative_tile<8, NT, false, false>(a, td, lds_dyn);
             else if (NT == 512 && td->F == 8192) derivative_tile<16, NT, false, NT == 512>(a, td, lds_dyn);
             else derivative_tile<16, NT, false, false>(a, td, lds_dyn);
             break;
@@ -1327,6 +1328,16 @@ static int strided_factor(int F) {
     return std::max(1, 16 / std::max(2, 2 * 256 / (F / fft_values(F))));
 }
 
+// 1024- and 2048-point lines take 16 values per thread (one and two wavefronts per
+// pair) or 8 (two and four): half the chain of arithmetic, t_n and the filter loaded
+// with the lines, for a barrier per exchange and twice the twiddle loads.  A scene
+// of few wavefronts (counted with 16; the chip holds 4096, 1024 at a time) is bound
+// by that chain.  Measured with 16 / 8, us per stage: 623 x 182 (700 wavefronts) 11.0
+// / 9.1, rooms of 333, 141, 477 x 217 11.8 / 10.5, 500^2 12.8 / 11.8, 1268 x 303 20.0 /
+// 17.1, 850^2 (1900) 18.9 / 19.9, two of 480^2 (2300) 17.7 / 16.6, 600 x 1073 (2600) 20.8 /
+// 21.8, 1200 x 700 24 / 25.5, 1024^2 29.8 / 30.9, six of 480^2 35.2 / 36.3.
+constexpr long long kFewWaves = 2500;
+
 struct pstd_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -1352,7 +1363,9 @@ struct pstd_ctx {
     int small_fmax = 0;  // largest F of the F <= 2048 class (128 threads need F <= 1024)
     int fmax = 0;        // largest F
     // block size of the stage launch: the threads of one line pair
-    int stage_threads() const { return std::max(small_nt, fmax / fft_values(fmax)); }
+    int stage_threads() const { return std::max(small_nt, fmax / values(fmax)); }
+    int f8 = 512;  // longest lines with 8 values per thread (kFewWaves)
+    int values(int F) const { return F <= f8 ? 8 : 16; }
     std::vector<GemmTile> tiles_gemm;
     int n_scenes = 1;
     std::vector<MaxRange> max_ranges;  // state read by a first stage after host writes (GEMM form)
@@ -1393,6 +1406,7 @@ struct pstd_ctx {
     int sample_cap = 0;
     int steps_done = 0;
     bool p0_explicit = true;
+    bool p0_turn = false;  // explicit p0 written since its transpose was
     int xcd_remap = 1;
     int lean = 1;  // stage kernel flavour as set (0 early, 1 late, 2 mid): one kernel serves them all
     float tuned_stage_ms = 0;
@@ -1474,12 +1488,12 @@ struct pstd_ctx {
 namespace {
 
 // Device plan cache entries: the tables of plan_tables.h rounded once to float.
-void build_filter(int F, int L, int field, double dx, std::vector<float2> &out) {
+void build_filter(int F, int L, int field, double dx, int values, std::vector<float2> &out) {
     const std::vector<std::complex<double>> h = pstdamd::derivative_filter(F, L, field, dx);
     out.resize(F);
     // thread t's values t + m T in pairs of m, [m / 2][t][m % 2]; length 8192: the even
     // and the odd bin of t + 512 m, [m][t][bin % 2]
-    const int T = F / fft_values(F);
+    const int T = F / values;
     for (int k = 0; k < F; ++k) {
         const int m = k / T, t = k % T;
         out[F == 8192 ? k : ((m / 2) * T + t) * 2 + m % 2] = make_float2((float)h[k].real(), (float)h[k].imag());
@@ -1538,7 +1552,14 @@ void timed_launch(pstd_ctx *ctx, hipStream_t st, int cls, Fn launch) {
 
 // One RK stage.  sample_slot >= 0 (first stage only): the launch also records
 // the receivers of the previous step into that sample slot.
+int launch_p0(pstd_ctx *ctx, int d, bool from_stage);
+
 int launch_stage(pstd_ctx *ctx, int k, int sample_slot) {
+    if (k == 0 && ctx->p0_turn) {
+        const int rc = launch_p0(ctx, -1, false);
+        if (rc) return rc;
+        ctx->p0_turn = false;
+    }
     StageArgs a{};
     a.ctab = ctx->ctab;
     a.ftab = ctx->ftab;
@@ -1554,6 +1575,7 @@ int launch_stage(pstd_ctx *ctx, int k, int sample_slot) {
     a.out = ctx->S(outi);
     a.pml = ctx->pml;
     a.s = ctx->dt * ctx->alpha[k];
+    a.f8 = ctx->f8;
     a.last = k == 5;
     const int ng = (int)ctx->tiles_gemm.size();
     if (ng) {
@@ -1768,14 +1790,14 @@ static int upload_tiles(pstd_ctx *ctx) {
     // fits is better off with its kinds of tiles mixed over the CUs
     long long waves = 0;
     for (const TileDesc &g : ctx->fft_segs)
-        if (g.kind == 0) waves += (long long)g.count / 2 * (g.F / fft_values(g.F)) / 64;
+        if (g.kind == 0) waves += (long long)g.count / 2 * (g.F / ctx->values(g.F)) / 64;
     std::vector<int> order(ctx->fft_segs.size());
     for (size_t k = 0; k < order.size(); ++k) order[k] = (int)k;
     auto length = [&](int k) { return ctx->fft_segs[k].kind == 0 ? ctx->fft_segs[k].F : 0; };
     if (waves > 4096) std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return length(x) > length(y); });
     for (int k : order) {
         const TileDesc &g = ctx->fft_segs[k];
-        const int per = g.kind == 0 ? 2 * nt / (g.F / fft_values(g.F)) : kPassChunk;
+        const int per = g.kind == 0 ? 2 * nt / (g.F / ctx->values(g.F)) : kPassChunk;
         for (int l = 0; l < g.count; l += per) {
             tiles.push_back(g);
             tiles.back().line0 = g.line0 + l;
@@ -2304,6 +2326,15 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             bp = 0;
         }
     };
+    long long waves = 0;
+    for (int si = 0; si < plan->n_segments; ++si) {
+        const pstd_plan_segment &s = plan->segments[si];
+        if (s.domain < 0 || s.domain >= plan->n_domains || s.wlen <= 0) continue;  // (refused below)
+        const DomainDev &dm = ctx->doms[s.domain];
+        const int F = next_pow2((s.direction == 0 ? dm.nx : dm.ny) + 2 * s.wlen);
+        waves += (long long)(s.line_end - s.line_begin) / 2 * (F / fft_values(F)) / 64;
+    }
+    ctx->f8 = waves <= kFewWaves ? 2048 : 512;
     long long strided_bytes = 0, pass_cells = 0;  // p0 on the fly, or by the pass
     for (const DomainDev &d : ctx->doms) pass_cells += (long long)d.nx * d.ny;
     std::vector<std::vector<char>> covered(plan->n_domains, std::vector<char>(4, 0));
@@ -2400,7 +2431,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         auto it = filt_cache.find(fk);
         if (it == filt_cache.end()) {
             std::vector<float2> h;
-            build_filter(g.F, s.table_len, s.field, dx, h);
+            build_filter(g.F, s.table_len, s.field, dx, ctx->values(g.F), h);
             it = filt_cache.emplace(fk, (int)ctab.size()).first;
             ctab.insert(ctab.end(), h.begin(), h.end());
         }
@@ -2713,8 +2744,7 @@ int pstd_ctx_set_field(pstd_ctx *ctx, int domain, int field, const float *host, 
     }
     if (field == PSTD_FIELD_P0) {
         HIP_TRY(hipMemcpyAsync(ctx->P0I() + field_off(d, PSTD_FIELD_PX), host, bytes, hipMemcpyHostToDevice, ctx->stream));
-        int rc = launch_p0(ctx, domain, false);
-        if (rc) return rc;
+        ctx->p0_turn = true;  // for all domains at once, by the next first stage
     } else if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
         // column-major on the device; S0 holds nothing between time steps
         float *rows = ctx->S(0) + field_off(d, field);

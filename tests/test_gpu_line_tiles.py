@@ -67,3 +67,24 @@ def test_p0_on_the_fly_is_bitwise_the_pass(nx, ny, copies):
     for f in ("p0", "px0", "py0", "vx0", "vy0"):
         for d in range(k.domain_count()):
             assert np.array_equal(batch.field(copies - 1, d, f), dev.field(d, f)), (f, d)
+
+
+@pytest.mark.parametrize("nx, ny, n", [(600, 700, 3), (1100, 300, 3), (90, 1300, 4), (447, 959, 4)])
+def test_values_per_thread_are_bitwise_neutral(nx, ny, n):
+    """1024- and 2048-point lines take 8 values per thread in a scene of few
+    wavefronts and 16 in a batch of many: the same bits."""
+    conf = P.PSTDConfiguration()
+    W.base_settings(conf, 5)
+    conf.Domains = [W.domain(0, 0, nx, ny, 0.9)]
+    conf.Speakers = [(W._world_pos(nx / 3), W._world_pos(ny / 2), 0.0)]
+    k = P.PSTDKernel(GPU=True)
+    k.initialize_kernel(conf)
+    one = k.prepare()
+    batch = P.BatchSolver([conf] * n)
+    one.advance(5)
+    batch.advance(5)
+    for d in range(k.domain_count()):
+        for f in ("p0", "px0", "py0", "vx0", "vy0"):
+            want = one.field(d, f)
+            for i in range(n):
+                assert np.array_equal(batch.field(i, d, f), want), (i, d, f)
