@@ -1846,8 +1846,9 @@ static int upload_tiles(pstd_ctx *ctx) {
 }
 
 // Launch-shape autotuner.  Times every (block size, tile order) candidate on the
-// freshly uploaded (all-zero) state and keeps the fastest.  Zero fields stay exactly zero under the update, and the arenas are
-// cleared again afterwards, so tuning leaves no trace in the results.
+// freshly uploaded (all-zero) state and keeps the fastest.  Zero fields stay
+// exactly zero under the update, and the arenas are cleared again afterwards, so
+// tuning leaves no trace in the results.
 // The autotuner's choices, per (device, plan signature): a later context with a
 // plan of the same launch geometry on the same device takes the choice and
 // runs no trials.
@@ -1892,6 +1893,14 @@ uint64_t plan_signature(const pstd_ctx *ctx) {
         mix(g.k_pad);
     }
     return h;
+}
+
+// The block size an earlier plan of the same signature was tuned to, before the
+// tile list is cut for it.
+static void take_tuned_threads(pstd_ctx *ctx) {
+    std::lock_guard<std::mutex> lock(g_tune_mu);
+    auto it = g_tune.find({ctx->device, plan_signature(ctx)});
+    if (it != g_tune.end()) ctx->small_nt = it->second.small_nt;
 }
 
 static int autotune(pstd_ctx *ctx) {
@@ -2515,10 +2524,14 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             if (f == 0 || f == 2) {
                 std::memcpy(pml.data() + offs[f], src[f], sizeof(float) * sizes[f]);
             } else {  // vy, py: column-major
+                // (16 columns at a time: their cache lines serve all 16)
                 const int rows = f == 1 ? p.ny + 1 : p.ny;
                 float *dst = pml.data() + offs[f];
-                for (int x = 0; x < p.nx; ++x)
-                    for (int y = 0; y < rows; ++y) dst[(size_t)x * rows + y] = src[f][(size_t)y * p.nx + x];
+                for (int x0 = 0; x0 < p.nx; x0 += 16)
+                    for (int y0 = 0; y0 < rows; y0 += 16)
+                        for (int x = x0; x < std::min(x0 + 16, p.nx); ++x)
+                            for (int y = y0; y < std::min(y0 + 16, rows); ++y)
+                                dst[(size_t)x * rows + y] = src[f][(size_t)y * p.nx + x];
             }
         }
     }
@@ -2596,6 +2609,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
                                hipMemcpyHostToDevice, ctx->stream));
     }
     {
+        take_tuned_threads(ctx);
         const int rc = upload_tiles(ctx);
         if (rc) return rc;
     }
