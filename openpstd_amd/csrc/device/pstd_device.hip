@@ -540,7 +540,8 @@ __device__ __forceinline__ int tile_index(int b, int n, int remap) {
 // decides how long the lines may be (8192-point ones take a 512-thread block),
 // how many adjacent lines a tile has and how finely a small scene spreads over
 // the CUs.  Bound by the VALU and the L1 together (16 sources of 512 x 1024 twice:
-// VALU 63 % and L1 address units 67 % busy, 270 us of the 350 us stage; one launch
+// VALU 63 % and L1 address units 67 % busy, 275 us of the 346 us stage, 200 of them
+// also without the transforms, which is what its memory traffic takes; one launch
 // of 8-value tiles, 568 us per stage, had each column access touch 8-16 bytes of a
 // cache line).
 constexpr size_t stage_lds(int nt) { return (size_t)(16 * nt / 256) * lds_pitch(256) * sizeof(float2); }
@@ -1318,10 +1319,10 @@ constexpr int kDefaultGraphSteps = 20;
 // a launch (5 us); on the fly, a tile of n adjacent lines reads 4 n bytes of every
 // 64-byte sector the other layout's field has in it.  The pass is taken where the
 // fly moves this many bytes per stage more (about 5 us at 4 TB/s).  Measured, us
-// per stage on the fly / with the pass: 333 000 cells 12.8 / 19.7, one 900^2 domain
-// 24.3 / 27.1, 1024^2 32.9 / 32.9, 1200^2 37.5 / 36.5, 1500^2 49.5 / 43.9, 4096^2
-// 406 / 352, 16 sources of 512 x 1024 twice 368 / 362; twelve scenes of lines up to
-// 600 (at least 8 lines per tile) 111 / 117.
+// per stage on the fly / with the pass: L-shape 7.7 / 14.2, 333 000 cells 11.8 / 19.2,
+// one 900^2 domain 22.1 / 26.0, 1024^2 30.3 / 32.8, 1200^2 37.0 / 36.3, 1900^2 59.5 /
+// 55.3, 2501 x 1237 69.1 / 55.7, 4096^2 465 / 394, 16 sources of 512 x 1024 twice 344 /
+// 346; twelve scenes of lines up to 600 (at least 8 lines per tile) 93.5 / 106.
 constexpr long long kP0PassBytes = 20000000;
 // 64-byte sectors read per 64 bytes used by a tile's strided reads (256 threads)
 static int strided_factor(int F) {
@@ -1787,7 +1788,9 @@ static int upload_tiles(pstd_ctx *ctx) {
     std::vector<TileDesc> tiles;
     // the longest tiles first, so that none of them starts last — where there are
     // more wavefronts than the chip holds at once (4 x 1024 SIMDs); a scene that
-    // fits is better off with its kinds of tiles mixed over the CUs
+    // fits may be better off with its kinds of tiles mixed over the CUs (us per stage
+    // mixed / sorted: three rooms of 333 000 cells 11.7 / 12.5, L-shape 7.7 / 7.7, 1200^2
+    // 37.2 / 36.0, 1900^2 59.5 / 55.0, 4096^2 399 / 393, twelve scenes 91.0 / 93.6)
     long long waves = 0;
     for (const TileDesc &g : ctx->fft_segs)
         if (g.kind == 0) waves += (long long)g.count / 2 * (g.F / ctx->values(g.F)) / 64;
