@@ -1332,12 +1332,14 @@ static int strided_factor(int F) {
 // 1024- and 2048-point lines take 16 values per thread (one and two wavefronts per
 // pair) or 8 (two and four): half the chain of arithmetic, t_n and the filter loaded
 // with the lines, for a barrier per exchange and twice the twiddle loads.  A scene
-// of few wavefronts (counted with 16; the chip holds 4096, 1024 at a time) is bound
-// by that chain.  Measured with 16 / 8, us per stage: 623 x 182 (700 wavefronts) 11.0
-// / 9.1, rooms of 333, 141, 477 x 217 11.8 / 10.5, 500^2 12.8 / 11.8, 1268 x 303 20.0 /
-// 17.1, 850^2 (1900) 18.9 / 19.9, two of 480^2 (2300) 17.7 / 16.6, 600 x 1073 (2600) 20.8 /
-// 21.8, 1200 x 700 24 / 25.5, 1024^2 29.8 / 30.9, six of 480^2 35.2 / 36.3.
-constexpr long long kFewWaves = 2500;
+// of few wavefronts (counted with 16; the chip holds 4096) is bound by that chain.
+// Measured with 16 / 8, us per stage, wavefronts in brackets: 623 x 182 (1132) 11.0 /
+// 9.2, 500^2 (1792) 13.8 / 12.6, 1500 x 150 (2214) 15.4 / 12.2, 700^2 (2392) 16.9 / 15.4,
+// rooms of 333, 141, 477 x 217 (2508) 11.7 / 11.0, 1198 x 206 (2702) 14.8 / 14.1, 850^2
+// (2844) 18.9 / 20.0, 900^2 (2992) 19.5 / 20.6, 1268 x 303 (3048) 15.9 / 15.7, two of 480^2
+// (3472) 17.7 / 16.6, 600 x 1073 (3504) 20.9 / 21.5, 1024^2 (5616) 29.8 / 30.9, six of 480^2
+// (10416) 35.2 / 36.3.
+constexpr long long kFewWaves = 2750;
 
 struct pstd_ctx {
     int device = 0;
@@ -1786,18 +1788,18 @@ static int enqueue_steps(pstd_ctx *ctx, int chunk, int base = 0) {
 static int upload_tiles(pstd_ctx *ctx) {
     const int nt = ctx->stage_threads();
     std::vector<TileDesc> tiles;
-    // the longest tiles first, so that none of them starts last — where there are
-    // more wavefronts than the chip holds at once (4 x 1024 SIMDs); a scene that
-    // fits may be better off with its kinds of tiles mixed over the CUs (us per stage
-    // mixed / sorted: three rooms of 333 000 cells 11.7 / 12.5, L-shape 7.7 / 7.7, 1200^2
-    // 37.2 / 36.0, 1900^2 59.5 / 55.0, 4096^2 399 / 393, twelve scenes 91.0 / 93.6)
+    // the longest tiles first, so that none of them starts last, but in the smallest
+    // scenes, whose kinds of tiles stay mixed over the CUs.  Measured mixed / sorted, us
+    // per stage: L-shape 8.1 / 8.2, rooms of 333, 141, 477 x 217 11.7 / 12.3 (11.0 / 11.0
+    // with 8 values per thread), 1500 x 150 18.1 / 15.4, 900^2 22.1 / 19.5, 1268 x 303 20.1 /
+    // 15.9, 1200^2 37.2 / 36.0, 1900^2 59.5 / 55.0, 4096^2 399 / 393, twelve scenes 91.0 / 93.6
     long long waves = 0;
     for (const TileDesc &g : ctx->fft_segs)
         if (g.kind == 0) waves += (long long)g.count / 2 * (g.F / ctx->values(g.F)) / 64;
     std::vector<int> order(ctx->fft_segs.size());
     for (size_t k = 0; k < order.size(); ++k) order[k] = (int)k;
     auto length = [&](int k) { return ctx->fft_segs[k].kind == 0 ? ctx->fft_segs[k].F : 0; };
-    if (waves > 4096) std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return length(x) > length(y); });
+    if (waves > 2048) std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return length(x) > length(y); });
     for (int k : order) {
         const TileDesc &g = ctx->fft_segs[k];
         const int per = g.kind == 0 ? 2 * nt / (g.F / ctx->values(g.F)) : kPassChunk;
