@@ -211,6 +211,10 @@ int pstd_ctx_get_form(const pstd_ctx *ctx);
  * (kernel/Solver.cpp:62-93); a batch advances each scene exactly as that loop
  * does. */
 int pstd_ctx_upload_plans(pstd_ctx *ctx, const pstd_plan_desc *plans, int n_plans);
+/* Threads: calls on one context may come from several threads; they take turns, in
+ * the order of their arrival, and each sees the state after a whole number of time
+ * steps.  Calls on different contexts do not wait for each other.  A context is
+ * destroyed once no call on it is running. */
 /* Host <-> device copies of one field of one domain (FieldValues::current). */
 int pstd_ctx_set_field(pstd_ctx *ctx, int domain, int field, const float *host, size_t count);
 int pstd_ctx_get_field(pstd_ctx *ctx, int domain, int field, float *host, size_t count);

@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <cmath>
 #include <complex>
+#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -1341,7 +1342,36 @@ static int strided_factor(int F) {
 // (10416) 35.2 / 36.3.
 constexpr long long kFewWaves = 2750;
 
+// Calls on one context take turns, in the order of their arrival: a thread that
+// advances in a loop does not keep one that reads frames from its turn (a plain
+// mutex is taken again before a thread woken up by its release can run).
+class TurnLock {
+public:
+    void lock() {
+        std::unique_lock<std::mutex> l(mu);
+        const uint64_t mine = next++;
+        cv.wait(l, [&] { return serving == mine; });
+    }
+    void unlock() {
+        {
+            std::lock_guard<std::mutex> l(mu);
+            ++serving;
+        }
+        cv.notify_all();
+    }
+
+private:
+    std::mutex mu;
+    std::condition_variable cv;
+    uint64_t next = 0, serving = 0;
+};
+
 struct pstd_ctx {
+    // Held by every call that issues work or changes the context, until the work
+    // that the call waits for is done: reads share the pinned memory and turn vy and
+    // py through S0, which is free between time steps only, and a captured step
+    // graph must hold nothing else.
+    TurnLock turn;
     int device = 0;
     hipStream_t stream = nullptr;
     // with `overlap`, GEMM-form stages run their FFT-form tiles on `side`,
@@ -2683,11 +2713,13 @@ static int upload_form(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
 
 int pstd_ctx_upload_plan(pstd_ctx *ctx, const pstd_plan_desc *plan) {
     if (!ctx || !plan) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     return upload_form(ctx, plan, nullptr);
 }
 
 int pstd_ctx_upload_plans(pstd_ctx *ctx, const pstd_plan_desc *plans, int n_plans) {
     if (!ctx || !plans || n_plans <= 0) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     if (n_plans == 1) return upload_form(ctx, plans, nullptr);
     // independent scenes: one plan with the domain lists concatenated; scenes
     // share the time step, the RK coefficients and the grid (one launch per
@@ -2745,7 +2777,9 @@ int pstd_ctx_upload_plans(pstd_ctx *ctx, const pstd_plan_desc *plans, int n_plan
 }
 
 int pstd_ctx_set_field(pstd_ctx *ctx, int domain, int field, const float *host, size_t count) {
-    if (!ctx || !ctx->planned || !host) return PSTD_ERR_INVALID;
+    if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    if (!ctx->planned || !host) return PSTD_ERR_INVALID;
     if (domain < 0 || domain >= (int)ctx->doms.size() || field < 0 || field > 4) return PSTD_ERR_INVALID;
     const pstd_plan_domain &p = ctx->plan_domains[domain];
     if (count != (size_t)field_size(p, field)) {
@@ -2794,7 +2828,9 @@ static bool short_result(pstd_ctx *ctx, size_t bytes) {
 }
 
 int pstd_ctx_get_field(pstd_ctx *ctx, int domain, int field, float *host, size_t count) {
-    if (!ctx || !ctx->planned || !host) return PSTD_ERR_INVALID;
+    if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    if (!ctx->planned || !host) return PSTD_ERR_INVALID;
     if (domain < 0 || domain >= (int)ctx->doms.size() || field < 0 || field > 4) return PSTD_ERR_INVALID;
     const pstd_plan_domain &p = ctx->plan_domains[domain];
     if (count != (size_t)field_size(p, field)) {
@@ -2871,8 +2907,7 @@ static int build_graph(pstd_ctx *ctx) {
 }
 
 static int advance_impl(pstd_ctx *ctx, int steps, float *samples) {
-    if (!ctx || !ctx->planned) return PSTD_ERR_INVALID;
-    if (steps < 0) return PSTD_ERR_INVALID;
+    if (!ctx->planned || steps < 0) return PSTD_ERR_INVALID;
     HIP_TRY(hipSetDevice(ctx->device));
     if (ctx->max_stale) {
         // the next first stage recomputes the maxima from the state (explicit p0)
@@ -2924,16 +2959,23 @@ static int advance_impl(pstd_ctx *ctx, int steps, float *samples) {
 }
 
 int pstd_ctx_advance(pstd_ctx *ctx, int steps, float *samples) {
+    if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     int rc = advance_impl(ctx, steps, samples);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return PSTD_OK;
 }
 
-int pstd_ctx_advance_async(pstd_ctx *ctx, int steps) { return advance_impl(ctx, steps, nullptr); }
+int pstd_ctx_advance_async(pstd_ctx *ctx, int steps) {
+    if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    return advance_impl(ctx, steps, nullptr);
+}
 
 int pstd_ctx_synchronize(pstd_ctx *ctx) {
     if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return PSTD_OK;
@@ -2943,6 +2985,7 @@ int pstd_ctx_steps_done(const pstd_ctx *ctx) { return ctx ? ctx->steps_done : -1
 
 int pstd_ctx_set_stage_overlap(pstd_ctx *ctx, int on) {
     if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     if (on && !(ctx->side && ctx->ev_fork && ctx->ev_join)) {
         ctx->err = "no side stream for overlapped stages";
         return PSTD_ERR_DEVICE;
@@ -2955,7 +2998,9 @@ int pstd_ctx_set_stage_overlap(pstd_ctx *ctx, int on) {
 }
 
 int pstd_ctx_capture_graph(pstd_ctx *ctx) {
-    if (!ctx || !ctx->planned) return PSTD_ERR_INVALID;
+    if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    if (!ctx->planned) return PSTD_ERR_INVALID;
     if (ctx->graph_steps <= 0 || ctx->graph_exec) return PSTD_OK;
     if (ctx->p0_explicit) {
         ctx->err = "the step graph is captured once p0 comes from the stage outputs (after a time step)";
@@ -2968,6 +3013,7 @@ int pstd_ctx_capture_graph(pstd_ctx *ctx) {
 
 int pstd_ctx_set_graph_steps(pstd_ctx *ctx, int steps) {
     if (!ctx || steps < 0) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     if (ctx->planned && steps > ctx->sample_cap) {
         ctx->err = "graph longer than the sample buffer (" + std::to_string(ctx->sample_cap) + " steps)";
         return PSTD_ERR_INVALID;
@@ -2983,6 +3029,7 @@ int pstd_ctx_set_form(pstd_ctx *ctx, int form) {
     if (!ctx || (form != PSTD_FORM_FFT && form != PSTD_FORM_GEMM_F16 && form != PSTD_FORM_GEMM_BF16 &&
                  form != PSTD_FORM_AUTO))
         return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     if (ctx->planned) {
         ctx->err = "the derivative form is chosen before the plan is uploaded";
         return PSTD_ERR_INVALID;
@@ -2996,6 +3043,7 @@ int pstd_ctx_get_form(const pstd_ctx *ctx) { return ctx ? ctx->form : PSTD_ERR_I
 
 int pstd_ctx_set_kernel_flavour(pstd_ctx *ctx, int flavour) {
     if (!ctx || flavour < 0 || flavour > 2) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->drop_graph();
@@ -3019,7 +3067,9 @@ int pstd_ctx_get_autotune(const pstd_ctx *ctx, int32_t *trial_steps, int32_t *fr
 }
 
 int pstd_ctx_set_tile_threads(pstd_ctx *ctx, int threads) {
-    if (!ctx || !ctx->planned || (threads != 128 && threads != 256 && threads != 512)) return PSTD_ERR_INVALID;
+    if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    if (!ctx->planned || (threads != 128 && threads != 256 && threads != 512)) return PSTD_ERR_INVALID;
     if (threads == 128 && ctx->small_fmax > 1024) {
         ctx->err = "128-thread tiles need every line of the F <= 2048 class to have F <= 1024";
         return PSTD_ERR_INVALID;
@@ -3044,6 +3094,7 @@ int pstd_ctx_get_tile_threads(const pstd_ctx *ctx) {
 
 int pstd_ctx_set_tile_order(pstd_ctx *ctx, int xcd_contiguous) {
     if (!ctx) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->drop_graph();
@@ -3052,7 +3103,9 @@ int pstd_ctx_set_tile_order(pstd_ctx *ctx, int xcd_contiguous) {
 }
 
 int pstd_ctx_profile_stages(pstd_ctx *ctx, int steps, double *mean_stage_ms, int *launches) {
-    if (!ctx || !ctx->planned || steps <= 0 || !mean_stage_ms) return PSTD_ERR_INVALID;
+    if (!ctx || steps <= 0 || !mean_stage_ms) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    if (!ctx->planned) return PSTD_ERR_INVALID;
     HIP_TRY(hipSetDevice(ctx->device));
     hipEvent_t ev[2];
     HIP_TRY(hipEventCreate(&ev[0]));
@@ -3073,7 +3126,9 @@ int pstd_ctx_profile_stages(pstd_ctx *ctx, int steps, double *mean_stage_ms, int
 }
 
 int pstd_ctx_advance_static(pstd_ctx *ctx, int steps) {
-    if (!ctx || !ctx->planned || steps < 0) return PSTD_ERR_INVALID;
+    if (!ctx || steps < 0) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    if (!ctx->planned) return PSTD_ERR_INVALID;
     const bool gemm = !ctx->tiles_gemm.empty();
     if (gemm && ctx->n_scenes > kStaticScenes) {
         ctx->err = "allocation-free advance: " + std::to_string(ctx->n_scenes) + " scenes, at most " +
@@ -3109,7 +3164,9 @@ int pstd_ctx_advance_static(pstd_ctx *ctx, int steps) {
 }
 
 int pstd_ctx_profile_kernels(pstd_ctx *ctx, int steps, double *ms, int *launches) {
-    if (!ctx || !ctx->planned || steps <= 0 || !ms || !launches) return PSTD_ERR_INVALID;
+    if (!ctx || steps <= 0 || !ms || !launches) return PSTD_ERR_INVALID;
+    std::lock_guard<TurnLock> turn(ctx->turn);
+    if (!ctx->planned) return PSTD_ERR_INVALID;
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     hipEvent_t ev[2];
