@@ -737,13 +737,32 @@ __global__ void __launch_bounds__(256) p0_pass_kernel(const float *__restrict__ 
     }
 }
 
-// dst (cols x rows) = transpose of src (rows x cols): host fields are row-major,
-// vy and py are stored column-major.
-__global__ void __launch_bounds__(256) transpose_kernel(const float *__restrict__ src, float *__restrict__ dst, int rows,
-                                                        int cols) {
+// Fields between the host's layout and the device's: host fields are row-major, vy
+// and py are stored column-major.  dst (cols x rows) = transpose of src (rows x
+// cols), for up to N fields in one launch (a launch costs what turning a field of a
+// small scene does several times over).
+struct TurnField {
+    const float *src;
+    float *dst;
+    int rows, cols;
+    unsigned first;  // the field's first workgroup
+};
+template <int N>
+struct TurnFields {
+    TurnField f[N];
+    int n;
+};
+template <int N>
+__global__ void __launch_bounds__(256) turn_kernel(TurnFields<N> fields) {
     __shared__ float turn[kP0Side][kP0Side + 1];
+    int k = 0;
+    while (k + 1 < fields.n && blockIdx.x >= fields.f[k + 1].first) ++k;
+    const float *src = fields.f[k].src;
+    float *dst = fields.f[k].dst;
+    const int rows = fields.f[k].rows, cols = fields.f[k].cols, across = (cols + kP0Side - 1) / kP0Side;
+    const int b = blockIdx.x - fields.f[k].first;
     const int lane = threadIdx.x & 63, row0 = threadIdx.x >> 6;
-    const int x0 = blockIdx.x * kP0Side, y0 = blockIdx.y * kP0Side;
+    const int x0 = b % across * kP0Side, y0 = b / across * kP0Side;
 #pragma unroll
     for (int i = 0; i < kP0Side / 4; ++i) {
         const int r = y0 + row0 + 4 * i;
@@ -1440,6 +1459,10 @@ struct pstd_ctx {
     int steps_done = 0;
     bool p0_explicit = true;
     bool p0_turn = false;  // explicit p0 written since its transpose was
+    // vy (even) and py (odd) of every domain written by the host and not turned yet:
+    // row-major in S0 (turn_written)
+    std::vector<char> written;
+    bool any_written = false;
     int xcd_remap = 1;
     int lean = 1;  // stage kernel flavour as set (0 early, 1 late, 2 mid): one kernel serves them all
     float tuned_stage_ms = 0;
@@ -1703,12 +1726,57 @@ int materialise_p0(pstd_ctx *ctx) {
     return PSTD_OK;
 }
 
+// Workgroups of turn_kernel for a rows x cols field.
+unsigned turn_blocks(int rows, int cols) {
+    return (unsigned)((rows + kP0Side - 1) / kP0Side) * (unsigned)((cols + kP0Side - 1) / kP0Side);
+}
+
 // Row-major rows x cols field <-> column-major: the host's and the device's
 // layout of vy and py.
-int launch_transpose(pstd_ctx *ctx, const float *src, float *dst, int rows, int cols) {
-    hipLaunchKernelGGL(transpose_kernel, dim3((cols + kP0Side - 1) / kP0Side, (rows + kP0Side - 1) / kP0Side), dim3(256),
-                       0, ctx->stream, src, dst, rows, cols);
+int launch_turn(pstd_ctx *ctx, const float *src, float *dst, int rows, int cols) {
+    hipLaunchKernelGGL(turn_kernel<1>, dim3(turn_blocks(rows, cols)), dim3(256), 0, ctx->stream,
+                       TurnFields<1>{{{src, dst, rows, cols, 0}}, 1});
     HIP_TRY(hipGetLastError());
+    return PSTD_OK;
+}
+
+// The same for many fields.
+constexpr int kTurnFields = 64;  // 2 KiB of kernel arguments
+int launch_turns(pstd_ctx *ctx, const std::vector<TurnField> &fields) {
+    for (size_t at = 0; at < fields.size(); at += kTurnFields) {
+        TurnFields<kTurnFields> t;
+        t.n = (int)std::min<size_t>(kTurnFields, fields.size() - at);
+        unsigned blocks = 0;
+        for (int k = 0; k < t.n; ++k) {
+            t.f[k] = fields[at + k];
+            t.f[k].first = blocks;
+            blocks += turn_blocks(t.f[k].rows, t.f[k].cols);
+        }
+        hipLaunchKernelGGL(turn_kernel<kTurnFields>, dim3(blocks), dim3(256), 0, ctx->stream, t);
+        HIP_TRY(hipGetLastError());
+    }
+    return PSTD_OK;
+}
+
+// The vy and py that the host wrote since the last time step, from S0 to TN.  A
+// program writes the fields of all domains before it advances: they are turned
+// together, in one launch per 64 fields (a launch and a wait per field took 12 us of
+// the 26 us that writing a py of an 18-domain scene took, and made a run() of two
+// steps of it 0.92 of the speed it has without).
+int turn_written(pstd_ctx *ctx) {
+    if (!ctx->any_written) return PSTD_OK;
+    std::vector<TurnField> fields;
+    for (size_t d = 0; d < ctx->doms.size(); ++d)
+        for (int f : {PSTD_FIELD_VY, PSTD_FIELD_PY}) {
+            if (!ctx->written[2 * d + (f == PSTD_FIELD_PY)]) continue;
+            const pstd_plan_domain &p = ctx->plan_domains[d];
+            const long long off = field_off(ctx->doms[d], f);
+            fields.push_back({ctx->S(0) + off, ctx->TN() + off, field_size(p, f) / p.nx, p.nx, 0});
+        }
+    const int rc = launch_turns(ctx, fields);
+    if (rc) return rc;
+    std::fill(ctx->written.begin(), ctx->written.end(), 0);
+    ctx->any_written = false;
     return PSTD_OK;
 }
 
@@ -2309,6 +2377,8 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     ctx->gemm_flops = 0;
     ctx->gemm_cells = 0;
     ctx->plan_domains.assign(plan->domains, plan->domains + plan->n_domains);
+    ctx->written.assign(2 * (size_t)std::max(0, plan->n_domains), 0);
+    ctx->any_written = false;
     // arena layout: one block per domain (vx, vy, px, py), 256 B aligned
     long long off = kLead;  // zeros before the first block
     auto align = [](long long v) { return (v + 63) & ~63LL; };
@@ -2799,11 +2869,11 @@ int pstd_ctx_set_field(pstd_ctx *ctx, int domain, int field, const float *host, 
         HIP_TRY(hipMemcpyAsync(ctx->P0I() + field_off(d, PSTD_FIELD_PX), host, bytes, hipMemcpyHostToDevice, ctx->stream));
         ctx->p0_turn = true;  // for all domains at once, by the next first stage
     } else if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
-        // column-major on the device; S0 holds nothing between time steps
-        float *rows = ctx->S(0) + field_off(d, field);
-        HIP_TRY(hipMemcpyAsync(rows, host, bytes, hipMemcpyHostToDevice, ctx->stream));
-        int rc = launch_transpose(ctx, rows, ctx->TN() + field_off(d, field), (int)(count / d.nx), d.nx);
-        if (rc) return rc;
+        // column-major on the device: turned from S0, which holds nothing else between
+        // time steps, before the next step or read of such a field
+        HIP_TRY(hipMemcpyAsync(ctx->S(0) + field_off(d, field), host, bytes, hipMemcpyHostToDevice, ctx->stream));
+        ctx->written[2 * domain + (field == PSTD_FIELD_PY)] = 1;
+        ctx->any_written = true;
     } else {
         HIP_TRY(hipMemcpyAsync(ctx->TN() + field_off(d, field), host, bytes, hipMemcpyHostToDevice, ctx->stream));
     }
@@ -2840,6 +2910,10 @@ int pstd_ctx_get_field(pstd_ctx *ctx, int domain, int field, float *host, size_t
     HIP_TRY(hipSetDevice(ctx->device));
     const DomainDev &d = ctx->doms[domain];
     const float *src = ctx->TN() + field_off(d, field);
+    if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
+        const int rc = turn_written(ctx);
+        if (rc) return rc;
+    }
     if (short_result(ctx, count * sizeof(float))) {
         if (field == PSTD_FIELD_P0 && !ctx->p0_explicit && !ctx->p0_pass) {
             hipLaunchKernelGGL(p0_rows_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, ctx->stream,
@@ -2847,7 +2921,7 @@ int pstd_ctx_get_field(pstd_ctx *ctx, int domain, int field, float *host, size_t
                                (float *)ctx->pin, d.nx, d.ny);
             HIP_TRY(hipGetLastError());
         } else if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
-            int rc = launch_transpose(ctx, src, (float *)ctx->pin, d.nx, (int)(count / d.nx));
+            int rc = launch_turn(ctx, src, (float *)ctx->pin, d.nx, (int)(count / d.nx));
             if (rc) return rc;
         } else {
             if (field == PSTD_FIELD_P0) src = ctx->P0I() + field_off(d, PSTD_FIELD_PX);
@@ -2867,7 +2941,7 @@ int pstd_ctx_get_field(pstd_ctx *ctx, int domain, int field, float *host, size_t
     } else if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
         // row-major for the host; S0 holds nothing between time steps
         float *rows = ctx->S(0) + field_off(d, field);
-        int rc = launch_transpose(ctx, src, rows, d.nx, (int)(count / d.nx));
+        int rc = launch_turn(ctx, src, rows, d.nx, (int)(count / d.nx));
         if (rc) return rc;
         src = rows;
     }
@@ -2909,6 +2983,10 @@ static int build_graph(pstd_ctx *ctx) {
 static int advance_impl(pstd_ctx *ctx, int steps, float *samples) {
     if (!ctx->planned || steps < 0) return PSTD_ERR_INVALID;
     HIP_TRY(hipSetDevice(ctx->device));
+    {
+        const int rc = turn_written(ctx);
+        if (rc) return rc;
+    }
     if (ctx->max_stale) {
         // the next first stage recomputes the maxima from the state (explicit p0)
         const int rc = materialise_p0(ctx);
@@ -3145,6 +3223,10 @@ int pstd_ctx_advance_static(pstd_ctx *ctx, int steps) {
         // the shared array starts from the maxima of the current state (explicit
         // p0, then the first stage's reduction), as after host writes
         int rc = materialise_p0(ctx);
+        if (rc) return rc;
+    }
+    {
+        const int rc = turn_written(ctx);
         if (rc) return rc;
     }
     unsigned *own = ctx->umax;
