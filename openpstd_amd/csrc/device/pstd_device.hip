@@ -776,12 +776,17 @@ __global__ void __launch_bounds__(256) turn_kernel(TurnFields<N> fields) {
     }
 }
 
-// p0 = px + py of one domain, row-major, for the caller of a short read (`p0` is
-// pinned host memory).
-__global__ void __launch_bounds__(256) p0_rows_kernel(const float *__restrict__ px, const float *__restrict__ py,
-                                                      float *__restrict__ p0, int nx, int ny) {
+// A column-major field of one domain, row-major (py and vy), or p0 = px + py of it
+// (px: row-major), for the caller of a short read: `out` is pinned host memory.  An
+// element per thread: the read waits for one access to memory and one to the host,
+// where turn_kernel's pieces do 16 after each other (a py of 100 x 50 cells in 13.4
+// us against 15.7, of 255 x 250 in 22.0 against 25.1).
+__global__ void __launch_bounds__(256) rows_kernel(const float *__restrict__ px, const float *__restrict__ py,
+                                                   float *__restrict__ out, int nx, int rows) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < nx * ny) p0[i] = px[i] + py[i % nx * ny + i / nx];
+    if (i >= nx * rows) return;
+    const float y = py[i % nx * rows + i / nx];
+    out[i] = px ? px[i] + y : y;
 }
 
 // ------------------------------------------------------------- GEMM form
@@ -2884,10 +2889,14 @@ int pstd_ctx_set_field(pstd_ctx *ctx, int domain, int field, const float *host, 
 // Results of at most kPinBytes reach the caller's (pageable) memory through pinned
 // memory of the context: a copy to pinned memory needs no staging by the runtime,
 // and a kernel that has to run first writes there itself (100 x 50 room: one
-// step's samples cost 21 -> 5 us, p0 36 -> 17.5, vy0 29 -> 19).  Longer results go
-// through the runtime's staging: the first touch of the caller's pages bounds them
-// (4 MiB 320 us; eight threads copying 256-KiB pieces from pinned memory took 420).
-constexpr size_t kPinBytes = 256 << 10;
+// step's samples 5 us instead of 21, p0 13.5 instead of 36, vy0 13.4 instead of 29).
+// A runtime copy that follows a kernel waits for it on the host, 16 us: through
+// pinned memory / by the runtime, p0 of 257 x 256 cells takes 23 / 139 us, py 22 / 36;
+// of 400 x 301 32 / 48 and 31 / 46; of 500 x 501 53 / 72 and 53 / 68; of 700 x 700 (1.9
+// MiB) 125 / 126 and 115 / 123, but its px 114 / 106; of 1000 x 1001 254 / 238.  Longer
+// results go through the runtime's staging (eight threads copying 256-KiB pieces
+// from pinned memory took 420 us for 4 MiB, against 320 into untouched pages).
+constexpr size_t kPinBytes = 1 << 20;
 static bool short_result(pstd_ctx *ctx, size_t bytes) {
     if (bytes > kPinBytes) return false;
     if (!ctx->pin && hipHostMalloc((void **)&ctx->pin, kPinBytes, hipHostMallocDefault) != hipSuccess) {
@@ -2916,13 +2925,14 @@ int pstd_ctx_get_field(pstd_ctx *ctx, int domain, int field, float *host, size_t
     }
     if (short_result(ctx, count * sizeof(float))) {
         if (field == PSTD_FIELD_P0 && !ctx->p0_explicit && !ctx->p0_pass) {
-            hipLaunchKernelGGL(p0_rows_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, ctx->stream,
+            hipLaunchKernelGGL(rows_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, ctx->stream,
                                ctx->S(1) + field_off(d, PSTD_FIELD_PX), ctx->S(1) + field_off(d, PSTD_FIELD_PY),
                                (float *)ctx->pin, d.nx, d.ny);
             HIP_TRY(hipGetLastError());
         } else if (field == PSTD_FIELD_VY || field == PSTD_FIELD_PY) {
-            int rc = launch_turn(ctx, src, (float *)ctx->pin, d.nx, (int)(count / d.nx));
-            if (rc) return rc;
+            hipLaunchKernelGGL(rows_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, ctx->stream,
+                               (const float *)nullptr, src, (float *)ctx->pin, d.nx, (int)(count / d.nx));
+            HIP_TRY(hipGetLastError());
         } else {
             if (field == PSTD_FIELD_P0) src = ctx->P0I() + field_off(d, PSTD_FIELD_PX);
             HIP_TRY(hipMemcpyAsync(ctx->pin, src, count * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
