@@ -1366,6 +1366,55 @@ static int strided_factor(int F) {
 // (10416) 35.2 / 36.3.
 constexpr long long kFewWaves = 2750;
 
+// Results of at most kPinBytes reach the caller's (pageable) memory through pinned
+// memory of the context: a copy to pinned memory needs no staging by the runtime,
+// and a kernel that has to run first writes there itself (100 x 50 room: one
+// step's samples 5 us instead of 21, p0 13.5 instead of 36, vy0 13.4 instead of 29).
+// A runtime copy that follows a kernel waits for it on the host, 16 us: through
+// pinned memory / by the runtime, p0 of 257 x 256 cells takes 23 / 139 us, py 22 / 36;
+// of 400 x 301 32 / 48 and 31 / 46; of 500 x 501 53 / 72 and 53 / 68; of 700 x 700 (1.9
+// MiB) 125 / 126 and 115 / 123, but its px 114 / 106; of 1000 x 1001 254 / 238.  Longer
+// results go through the runtime's staging (eight threads copying 256-KiB pieces
+// from pinned memory took 420 us for 4 MiB, against 320 into untouched pages).
+constexpr size_t kPinBytes = 1 << 20;
+
+// A context takes its pinned memory at the first short result and gives it back when
+// it is destroyed.  A program that makes a solver per run (PSTDKernel::run) paid 70 to
+// 120 us for it each time (run() of 121 steps of the L-shape 7400 -> 7285 us, of two
+// steps of 18 domains 1680 -> 1610): up to kPinKept buffers wait for the next
+// context, of any device (portable), the others are freed.
+constexpr size_t kPinKept = 4;
+static std::mutex g_pinned_mu;
+static std::vector<char *> g_pinned;
+
+static char *take_pinned() {
+    {
+        std::lock_guard<std::mutex> lock(g_pinned_mu);
+        if (!g_pinned.empty()) {
+            char *p = g_pinned.back();
+            g_pinned.pop_back();
+            return p;
+        }
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, kPinBytes, hipHostMallocPortable) == hipSuccess) return (char *)p;
+    (void)hipGetLastError();  // the runtime's staging then
+    return nullptr;
+}
+
+// (no work that uses it is in flight)
+static void give_pinned(char *p) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lock(g_pinned_mu);
+        if (g_pinned.size() < kPinKept) {
+            g_pinned.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
 // Calls on one context take turns, in the order of their arrival: a thread that
 // advances in a loop does not keep one that reads frames from its turn (a plain
 // mutex is taken again before a thread woken up by its release can run).
@@ -1491,7 +1540,7 @@ struct pstd_ctx {
     bool tune_cached = false;
 
     // Pinned memory that short results pass through on their way to the caller
-    // (short_result), allocated by the first of them.
+    // (short_result), taken by the first of them.
     char *pin = nullptr;
 
     void drop_graph() {
@@ -1851,7 +1900,7 @@ void pstd_ctx_destroy(pstd_ctx *ctx) {
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
-    if (ctx->pin) (void)hipHostFree(ctx->pin);
+    give_pinned(ctx->pin);
     delete ctx;
 }
 
@@ -2886,23 +2935,9 @@ int pstd_ctx_set_field(pstd_ctx *ctx, int domain, int field, const float *host, 
     return PSTD_OK;
 }
 
-// Results of at most kPinBytes reach the caller's (pageable) memory through pinned
-// memory of the context: a copy to pinned memory needs no staging by the runtime,
-// and a kernel that has to run first writes there itself (100 x 50 room: one
-// step's samples 5 us instead of 21, p0 13.5 instead of 36, vy0 13.4 instead of 29).
-// A runtime copy that follows a kernel waits for it on the host, 16 us: through
-// pinned memory / by the runtime, p0 of 257 x 256 cells takes 23 / 139 us, py 22 / 36;
-// of 400 x 301 32 / 48 and 31 / 46; of 500 x 501 53 / 72 and 53 / 68; of 700 x 700 (1.9
-// MiB) 125 / 126 and 115 / 123, but its px 114 / 106; of 1000 x 1001 254 / 238.  Longer
-// results go through the runtime's staging (eight threads copying 256-KiB pieces
-// from pinned memory took 420 us for 4 MiB, against 320 into untouched pages).
-constexpr size_t kPinBytes = 1 << 20;
 static bool short_result(pstd_ctx *ctx, size_t bytes) {
     if (bytes > kPinBytes) return false;
-    if (!ctx->pin && hipHostMalloc((void **)&ctx->pin, kPinBytes, hipHostMallocDefault) != hipSuccess) {
-        ctx->pin = nullptr;
-        (void)hipGetLastError();  // the runtime's staging then
-    }
+    if (!ctx->pin) ctx->pin = take_pinned();
     return ctx->pin != nullptr;
 }
 
