@@ -2665,8 +2665,11 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     }
     if (ctab.empty()) ctab.push_back(make_float2(0, 0));
     if (ftab.empty()) ftab.push_back(0);
-    // PML factor arena (1 where no PML)
+    // PML factor arena (1 where no PML), vy and py row-major as they come: the device
+    // turns them
     std::vector<float> pml(ctx->arena_floats, 1.f);
+    std::vector<TurnField> pml_turned;  // vy and py of the PML domains (src, dst: below)
+    std::vector<long long> pml_off;
     for (int i = 0; i < plan->n_domains; ++i) {
         const pstd_plan_domain &p = plan->domains[i];
         if (!p.is_pml) continue;
@@ -2680,17 +2683,10 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
                 ctx->err = "PML domain without factor arrays";
                 return PSTD_ERR_INVALID;
             }
-            if (f == 0 || f == 2) {
-                std::memcpy(pml.data() + offs[f], src[f], sizeof(float) * sizes[f]);
-            } else {  // vy, py: column-major
-                // (16 columns at a time: their cache lines serve all 16)
-                const int rows = f == 1 ? p.ny + 1 : p.ny;
-                float *dst = pml.data() + offs[f];
-                for (int x0 = 0; x0 < p.nx; x0 += 16)
-                    for (int y0 = 0; y0 < rows; y0 += 16)
-                        for (int x = x0; x < std::min(x0 + 16, p.nx); ++x)
-                            for (int y = y0; y < std::min(y0 + 16, rows); ++y)
-                                dst[(size_t)x * rows + y] = src[f][(size_t)y * p.nx + x];
+            std::memcpy(pml.data() + offs[f], src[f], sizeof(float) * sizes[f]);
+            if (f == 1 || f == 3) {
+                pml_turned.push_back({nullptr, nullptr, sizes[f] / p.nx, p.nx, 0});
+                pml_off.push_back(offs[f]);
             }
         }
     }
@@ -2734,9 +2730,20 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     // allocate + upload
     const size_t af = ctx->arena_floats;
     HIP_TRY(hipMalloc(&ctx->arena, 4 * af * sizeof(float)));
-    HIP_TRY(hipMemsetAsync(ctx->arena, 0, 4 * af * sizeof(float), ctx->stream));
     HIP_TRY(hipMalloc(&ctx->pml, af * sizeof(float)));
-    HIP_TRY(hipMemcpyAsync(ctx->pml, pml.data(), af * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    // the PML factors by way of S0, whose vy and py are turned over them (on the host
+    // that took 30 to 100 us of the set-up of a small scene); then the arenas are zeroed
+    HIP_TRY(hipMemcpyAsync(ctx->S(0), pml.data(), af * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    HIP_TRY(hipMemcpyAsync(ctx->pml, ctx->S(0), af * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
+    for (size_t k = 0; k < pml_turned.size(); ++k) {
+        pml_turned[k].src = ctx->S(0) + pml_off[k];
+        pml_turned[k].dst = ctx->pml + pml_off[k];
+    }
+    {
+        const int rc = launch_turns(ctx, pml_turned);
+        if (rc) return rc;
+    }
+    HIP_TRY(hipMemsetAsync(ctx->arena, 0, 4 * af * sizeof(float), ctx->stream));
     HIP_TRY(hipMalloc(&ctx->ctab, ctab.size() * sizeof(float2)));
     HIP_TRY(hipMemcpyAsync(ctx->ctab, ctab.data(), ctab.size() * sizeof(float2), hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(hipMalloc(&ctx->ftab, ftab.size() * sizeof(float)));
