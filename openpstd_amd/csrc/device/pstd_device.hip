@@ -2494,20 +2494,20 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             bp = 0;
         }
     };
-    long long waves = 0;
-    for (int si = 0; si < plan->n_segments; ++si) {
-        const pstd_plan_segment &s = plan->segments[si];
-        if (s.domain < 0 || s.domain >= plan->n_domains || s.wlen <= 0) continue;  // (refused below)
-        const DomainDev &dm = ctx->doms[s.domain];
-        const int F = next_pow2((s.direction == 0 ? dm.nx : dm.ny) + 2 * s.wlen);
-        waves += (long long)(s.line_end - s.line_begin) / 2 * (F / fft_values(F)) / 64;
-    }
-    ctx->f8 = waves <= kFewWaves ? 2048 : 512;
     long long strided_bytes = 0, pass_cells = 0;  // p0 on the fly, or by the pass
     for (const DomainDev &d : ctx->doms) pass_cells += (long long)d.nx * d.ny;
     std::vector<std::vector<char>> covered(plan->n_domains, std::vector<char>(4, 0));
     std::vector<uint16_t> dmat;
     std::map<std::string, std::tuple<long long, int, int>> dcache;  // matrix key -> (hi offset, d_exp, dot row)
+    // the segments as tiles' records (without tables yet), each checked before anything
+    // is computed from it
+    struct Line {
+        const pstd_plan_segment *s;
+        TileDesc g;
+        bool gemm;
+    };
+    std::vector<Line> checked;
+    long long waves = 0;
     for (int si = 0; si < plan->n_segments; ++si) {
         const pstd_plan_segment &s = plan->segments[si];
         if (s.domain < 0 || s.domain >= plan->n_domains || s.side1 >= plan->n_domains || s.side2 >= plan->n_domains ||
@@ -2526,6 +2526,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             ctx->err = "segment line range outside its domain";
             return PSTD_ERR_INVALID;
         }
+        const int nlines_seg = s.line_end - s.line_begin;
         TileDesc g{};
         g.kind = 0;
         g.dir = s.direction;
@@ -2584,6 +2585,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
                 g.s2_size = dn.size;
             }
         }
+        waves += (long long)nlines_seg / 2 * (g.F / fft_values(g.F)) / 64;
         if (s.interp_only) {
             if (s.direction != 0 || s.field != 0) {
                 ctx->err = "interpolation-only segment " + std::to_string(si) + " is not an X pressure segment";
@@ -2595,6 +2597,20 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         g.o_f = s.direction == 0 ? (s.field == 0 ? dm.f_vx : dm.f_px) : (s.field == 0 ? dm.f_vy : dm.f_py);
         g.o_ls = s.field == 0 ? n + 1 : n;
         covered[s.domain][s.direction == 0 ? (s.field == 0 ? 2 : 0) : (s.field == 0 ? 3 : 1)] = 1;
+        g.scene = scene_of(s.domain);
+        if (s.field == 0) strided_bytes += 4LL * (s.line_end - s.line_begin) * n * strided_factor(g.F);
+        g.line0 = s.line_begin;
+        g.count = s.line_end - s.line_begin;
+        // GEMM form: segments that fill the 128 x 256 tiles at least to 3/4
+        // become GEMM tiles; thin ones (PML strips) stay FFT tiles
+        const bool gemm = (ctx->form == PSTD_FORM_GEMM_F16 || ctx->form == PSTD_FORM_GEMM_BF16) &&
+                          gemm_fills(g.count, s.field == 0 ? g.n_out - 1 : g.n_out);
+        checked.push_back({&s, g, gemm});
+    }
+    ctx->f8 = waves <= kFewWaves ? 2048 : 512;
+    for (Line &l : checked) {
+        const pstd_plan_segment &s = *l.s;
+        TileDesc &g = l.g;
         auto fk = std::make_tuple(g.F, s.table_len, s.field);
         auto it = filt_cache.find(fk);
         if (it == filt_cache.end()) {
@@ -2620,19 +2636,11 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             ftab.insert(ftab.end(), w.begin(), w.end());
         }
         g.win_off = wt->second;
-        g.scene = scene_of(s.domain);
-        if (s.field == 0) strided_bytes += 4LL * (s.line_end - s.line_begin) * n * strided_factor(g.F);
-        // GEMM form: segments that fill the 128 x 256 tiles at least to 3/4
-        // become GEMM tiles; thin ones (PML strips) stay FFT tiles
-        const int nlines_seg = s.line_end - s.line_begin;
-        if ((ctx->form == PSTD_FORM_GEMM_F16 || ctx->form == PSTD_FORM_GEMM_BF16) &&
-            gemm_fills(nlines_seg, s.field == 0 ? g.n_out - 1 : g.n_out)) {
+        if (l.gemm) {
             int rc = add_gemm_tiles(ctx, plan, s, g, dmat, ftab, dcache);
             if (rc) return rc;
             continue;
         }
-        g.line0 = s.line_begin;
-        g.count = s.line_end - s.line_begin;
         ctx->fmax = std::max(ctx->fmax, g.F);
         if (g.F <= 2048) ctx->small_fmax = std::max(ctx->small_fmax, g.F);
         ctx->fft_segs.push_back(g);
