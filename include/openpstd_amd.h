@@ -298,13 +298,17 @@ int pstd_ctx_set_stage_overlap(pstd_ctx *ctx, int on);
  * pstd_ctx_get_tuning reports the choice and its timed GPU ms per stage,
  * pstd_ctx_get_tile_threads the block size, pstd_ctx_get_autotune the time
  * steps the trials ran on this context (launches of the stage kernels that are
- * not part of the caller's steps) and whether the choice came from the cache. */
+ * not part of the caller's steps) and whether the choice came from the cache.
+ * pstd_ctx_get_stage_paths reports what the plan's sizes chose at upload: whether
+ * p0 is formed by a pass after every stage (1) or by the tiles that read it (0),
+ * and the longest FFT length whose lines take 8 values per thread (512 or 2048). */
 int pstd_ctx_set_tile_order(pstd_ctx *ctx, int xcd_contiguous);
 int pstd_ctx_set_kernel_flavour(pstd_ctx *ctx, int flavour);
 int pstd_ctx_set_tile_threads(pstd_ctx *ctx, int threads);
 int pstd_ctx_get_tile_threads(const pstd_ctx *ctx);
 int pstd_ctx_get_tuning(const pstd_ctx *ctx, int32_t *flavour, int32_t *xcd_contiguous, double *stage_ms);
 int pstd_ctx_get_autotune(const pstd_ctx *ctx, int32_t *trial_steps, int32_t *from_cache);
+int pstd_ctx_get_stage_paths(const pstd_ctx *ctx, int32_t *p0_pass, int32_t *eight_value_points);
 /* Work of the GEMM-form segments in one RK stage: algorithmic MFMA flops
  * (3 split products x 2 x K x outputs x lines) and line outputs. */
 int pstd_ctx_gemm_work(const pstd_ctx *ctx, double *flops_per_stage, long long *outputs_per_stage);

@@ -3204,6 +3204,13 @@ int pstd_ctx_get_autotune(const pstd_ctx *ctx, int32_t *trial_steps, int32_t *fr
     return PSTD_OK;
 }
 
+int pstd_ctx_get_stage_paths(const pstd_ctx *ctx, int32_t *p0_pass, int32_t *eight_value_points) {
+    if (!ctx || !ctx->planned) return PSTD_ERR_INVALID;
+    if (p0_pass) *p0_pass = ctx->p0_pass ? 1 : 0;
+    if (eight_value_points) *eight_value_points = ctx->f8;
+    return PSTD_OK;
+}
+
 int pstd_ctx_set_tile_threads(pstd_ctx *ctx, int threads) {
     if (!ctx) return PSTD_ERR_INVALID;
     std::lock_guard<TurnLock> turn(ctx->turn);

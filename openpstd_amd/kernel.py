@@ -279,7 +279,9 @@ class _Context:
     def tuning(self):
         """The autotuner's choice: {"lean" (flavour 0 early, 1 late, 2 mid), "xcd_order", "tile_threads",
         "stage_ms", "trial_steps" (time steps its trials ran on this solver), "cached" (the choice came from
-        the per-(device, plan signature) cache, without trials)}."""
+        the per-(device, plan signature) cache, without trials)}, and what the plan's sizes chose:
+        "p0_pass" (p0 formed by a pass after every stage, or by the tiles that read it), "eight_value_points"
+        (longest FFT length whose lines take 8 values per thread)."""
         lean, xcd = C.c_int32(), C.c_int32()
         ms = C.c_double()
         _check(lib().pstd_ctx_get_tuning(self.ctx, C.byref(lean), C.byref(xcd), C.byref(ms)), self._err)
@@ -287,8 +289,11 @@ class _Context:
         _check(min(nt, 0), self._err)
         trials, cached = C.c_int32(), C.c_int32()
         _check(lib().pstd_ctx_get_autotune(self.ctx, C.byref(trials), C.byref(cached)), self._err)
+        p0_pass, points = C.c_int32(), C.c_int32()
+        _check(lib().pstd_ctx_get_stage_paths(self.ctx, C.byref(p0_pass), C.byref(points)), self._err)
         return {"lean": lean.value, "xcd_order": xcd.value, "tile_threads": nt, "stage_ms": ms.value,
-                "trial_steps": trials.value, "cached": bool(cached.value)}
+                "trial_steps": trials.value, "cached": bool(cached.value), "p0_pass": bool(p0_pass.value),
+                "eight_value_points": points.value}
 
     def _get(self, i, name, shape):
         out = np.zeros(shape, dtype=np.float32)
