@@ -1363,7 +1363,9 @@ static int strided_factor(int F) {
 // rooms of 333, 141, 477 x 217 (2508) 11.7 / 11.0, 1198 x 206 (2702) 14.8 / 14.1, 850^2
 // (2844) 18.9 / 20.0, 900^2 (2992) 19.5 / 20.6, 1268 x 303 (3048) 15.9 / 15.7, two of 480^2
 // (3472) 17.7 / 16.6, 600 x 1073 (3504) 20.9 / 21.5, 1024^2 (5616) 29.8 / 30.9, six of 480^2
-// (10416) 35.2 / 36.3.
+// (10416) 35.2 / 36.3; the line tiles beside the matrix form of 1024^2 (1520) 63.4 / 60.4 with
+// that form's launch.  No count separates the gains from the losses between 2700 and 3500:
+// the line lies below the first loss, and what it gives away there is at most 6 %.
 constexpr long long kFewWaves = 2750;
 
 // Results of at most kPinBytes reach the caller's (pageable) memory through pinned
@@ -2019,8 +2021,9 @@ std::map<std::pair<int, uint64_t>, TuneChoice> g_tune;
 std::map<std::pair<int, uint64_t>, int> g_form;
 
 // FNV-1a over what the launches' timing depends on: the form, the scene count,
-// every tile's line class, line count and direction, and the arena size.  Two
-// plans that hash alike launch the same grids of the same kernels.
+// the paths that the plan's sizes chose, every tile's line class, line count and
+// direction, and the arena size.  Two plans that hash alike launch the same grids of
+// the same kernels.
 uint64_t plan_signature(const pstd_ctx *ctx) {
     uint64_t h = 1469598103934665603ull;
     auto mix = [&h](long long v) {
@@ -2031,6 +2034,8 @@ uint64_t plan_signature(const pstd_ctx *ctx) {
     };
     mix(ctx->form);
     mix(ctx->n_scenes);
+    mix(ctx->p0_pass);
+    mix(ctx->f8);
     mix((long long)ctx->arena_floats);
     mix((long long)ctx->fft_segs.size());
     for (const TileDesc &t : ctx->fft_segs) {
@@ -2526,7 +2531,6 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             ctx->err = "segment line range outside its domain";
             return PSTD_ERR_INVALID;
         }
-        const int nlines_seg = s.line_end - s.line_begin;
         TileDesc g{};
         g.kind = 0;
         g.dir = s.direction;
@@ -2585,7 +2589,6 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
                 g.s2_size = dn.size;
             }
         }
-        waves += (long long)nlines_seg / 2 * (g.F / fft_values(g.F)) / 64;
         if (s.interp_only) {
             if (s.direction != 0 || s.field != 0) {
                 ctx->err = "interpolation-only segment " + std::to_string(si) + " is not an X pressure segment";
@@ -2605,6 +2608,8 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         // become GEMM tiles; thin ones (PML strips) stay FFT tiles
         const bool gemm = (ctx->form == PSTD_FORM_GEMM_F16 || ctx->form == PSTD_FORM_GEMM_BF16) &&
                           gemm_fills(g.count, s.field == 0 ? g.n_out - 1 : g.n_out);
+        // of the lines this plan's stage launch runs
+        if (!gemm) waves += (long long)g.count / 2 * (g.F / fft_values(g.F)) / 64;
         checked.push_back({&s, g, gemm});
     }
     ctx->f8 = waves <= kFewWaves ? 2048 : 512;

@@ -102,3 +102,50 @@ def test_8192_point_lines_in_either_order_and_in_a_batch(across):
         for d in range(k.domain_count()):
             assert np.array_equal(a.field(d, f), b.field(d, f)), (f, d)
     assert_same_fields(k, a, batch, 2)
+
+
+def fft_wavefronts(k):
+    """Wavefronts of the line tiles of one stage with 16 values per thread from 1024
+    points on, counted from the plan's segments (all of them in the FFT form)."""
+    total = 0
+    for s in k.segments():
+        d = k.domain_info(s["domain"])
+        n = (d["nx"] if s["direction"] == 0 else d["ny"]) + (1 if s["field"] else 0) + 2 * s["wlen"]
+        f = 1 << (n - 1).bit_length()
+        if not s["interp_only"]:
+            total += (s["line_end"] - s["line_begin"]) // 2 * (f // (8 if f <= 512 else 16)) // 64
+    return total
+
+
+# rigid walls above and below: spectral receivers read lines there that no stage runs,
+# which took (1060, 600) and (1300, 530) past the limit
+@pytest.mark.parametrize("nx, ny", [(1060, 600), (1300, 530), (1060, 650), (700, 500)])
+def test_lines_of_receivers_only_choose_no_values_per_thread(nx, ny):
+    points, series = [], []
+    for spectral in (False, True):
+        conf = scene(nx, ny, 2, spectral)
+        conf.Domains = [W.domain(0, 0, nx, ny, {"T": 0.0, "B": 0.0, "L": 1.0, "R": 1.0})]
+        k, dev = device(conf)
+        assert any(s["interp_only"] for s in k.segments()) == spectral
+        points.append(dev.tuning()["eight_value_points"])
+        assert points[-1] == (2048 if fft_wavefronts(k) <= 2750 else 512)
+        dev.advance(2)
+        series.append([dev.field(d, f) for d in range(k.domain_count()) for f in FIELDS])
+    assert points[0] == points[1]
+    for a, b in zip(*series):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("form", ["gemm_f16", "gemm_bf16"])
+def test_lines_of_the_matrix_form_choose_no_values_per_thread(form):
+    """A 1024 x 1024 scene in the matrix form: the line tiles are its absorbing layers',
+    few wavefronts; the same bits as in a batch, whose layers are many."""
+    conf = scene(1024, 1024, 2)
+    k = P.PSTDKernel(GPU=True)
+    k.initialize_kernel(conf)
+    k.set_form(form)
+    dev = k.prepare()
+    batch = P.BatchSolver([conf] * 4, form=form)
+    assert dev.tuning()["eight_value_points"] == 2048 and batch.tuning()["eight_value_points"] == 512
+    assert np.array_equal(batch.scene_samples(batch.advance(2), 3), dev.advance(2))
+    assert_same_fields(k, dev, batch, 3)
