@@ -262,10 +262,8 @@ def main():
                          "eagerly)")
     ap.add_argument("--tile-order", default="auto", choices=["auto", "xcd", "plain"],
                     help="workgroup-to-tile order (default: the autotuner's choice)")
-    ap.add_argument("--flavour", default="auto", choices=["auto", "early", "late", "mid"],
-                    help="FFT stage-kernel flavour (default: the autotuner's choice)")
     ap.add_argument("--tile-threads", default="auto", choices=["auto", "128", "256", "512"],
-                    help="block size for lines of FFT length <= 2048 (default: the autotuner's choice)")
+                    help="block size of the stage kernel where its lines leave it (default: the autotuner's choice)")
     ap.add_argument("--receivers", default="physical", choices=["physical", "spectral"],
                     help="receiver reading: the receiver's cell, or spectral interpolation at its location")
     ap.add_argument("--overlap", action="store_true",
@@ -303,8 +301,6 @@ def main():
         dev.set_stage_overlap(True)
     if args.tile_order != "auto":
         dev.set_tile_order(args.tile_order == "xcd")
-    if args.flavour != "auto":
-        dev.set_kernel_flavour(args.flavour)
     if args.tile_threads != "auto":
         dev.set_tile_threads(int(args.tile_threads))
     tuning = dev.tuning()
@@ -378,10 +374,8 @@ def main():
         "config": {"workload": desc, "scenes": len(confs), "cells_per_stage": cells, "user_cells": user,
                    "domains": len(infos), "rk_stages_per_step": 6, "form": form,
                    "form_requested": args.form,
-                   "launch_shape": {"flavour": ["early", "late", "mid"][tuning["lean"]],
-                                    "xcd_order": tuning["xcd_order"], "tile_threads": tuning["tile_threads"],
-                                    "autotuned": args.tile_order == "auto" and args.flavour == "auto"
-                                    and args.tile_threads == "auto",
+                   "launch_shape": {"xcd_order": tuning["xcd_order"], "tile_threads": tuning["tile_threads"],
+                                    "autotuned": args.tile_order == "auto" and args.tile_threads == "auto",
                                     "autotune_trial_steps": tuning["trial_steps"],
                                     "autotune_cached": tuning["cached"],
                                     "graph_steps": 20 if args.graph_steps is None else args.graph_steps},

@@ -25,7 +25,7 @@ HEADERS = ["device/fft_line.h", "host/kernel_api.h", "host/scene_model.h", "host
 
 # Packed FP32 instructions are kept out of the device code.  No implicit FMA
 # contraction: the device code writes its fused multiply-adds explicitly, so
-# every kernel flavour and launch shape rounds the same way (bitwise-equal
+# every kernel variant and launch shape rounds the same way (bitwise-equal
 # results whichever the autotuner picks).  The first eight words of kernel
 # arguments arrive in scalar registers (the stage kernel's finds its tile's record
 # with them, without a load of its arguments first).

@@ -1520,7 +1520,9 @@ struct pstd_ctx {
     std::vector<char> written;
     bool any_written = false;
     int xcd_remap = 1;
-    int lean = 1;  // stage kernel flavour as set (0 early, 1 late, 2 mid): one kernel serves them all
+    // stage kernel flavour as set (0 early, 1 late, 2 mid) and reported back: one kernel
+    // serves them all
+    int lean = 1;
     float tuned_stage_ms = 0;
     // the GEMM form's maxima in `umax` no longer describe the state (an
     // allocation-free advance used the shared array): recompute before the next step
@@ -2012,7 +2014,7 @@ static int upload_tiles(pstd_ctx *ctx) {
 // plan of the same launch geometry on the same device takes the choice and
 // runs no trials.
 struct TuneChoice {
-    int lean, xcd_remap, small_nt;
+    int xcd_remap, small_nt;
     float stage_ms;
 };
 std::mutex g_tune_mu;
@@ -2073,7 +2075,6 @@ static int autotune(pstd_ctx *ctx) {
         std::lock_guard<std::mutex> lock(g_tune_mu);
         auto it = g_tune.find(key);
         if (it != g_tune.end()) {
-            ctx->lean = it->second.lean;
             ctx->xcd_remap = it->second.xcd_remap;
             ctx->tuned_stage_ms = it->second.stage_ms;
             ctx->tune_cached = true;
@@ -2151,7 +2152,7 @@ static int autotune(pstd_ctx *ctx) {
     ctx->tuned_stage_ms = best / (6.0 * n);
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
-        g_tune[key] = {ctx->lean, ctx->xcd_remap, ctx->small_nt, ctx->tuned_stage_ms};
+        g_tune[key] = {ctx->xcd_remap, ctx->small_nt, ctx->tuned_stage_ms};
     }
     HIP_TRY(hipMemsetAsync(ctx->arena, 0, 4 * (size_t)ctx->arena_floats * sizeof(float), ctx->stream));
     if (ctx->umax) HIP_TRY(hipMemsetAsync(ctx->umax, 0, 2 * (size_t)ctx->n_scenes * sizeof(unsigned), ctx->stream));
@@ -3187,9 +3188,6 @@ int pstd_ctx_get_form(const pstd_ctx *ctx) { return ctx ? ctx->form : PSTD_ERR_I
 int pstd_ctx_set_kernel_flavour(pstd_ctx *ctx, int flavour) {
     if (!ctx || flavour < 0 || flavour > 2) return PSTD_ERR_INVALID;
     std::lock_guard<TurnLock> turn(ctx->turn);
-    HIP_TRY(hipSetDevice(ctx->device));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    ctx->drop_graph();
     ctx->lean = flavour;
     return PSTD_OK;
 }

@@ -277,8 +277,8 @@ class _Context:
         return {T.PSTD_FORM_FFT: "fft", T.PSTD_FORM_GEMM_F16: "gemm_f16", T.PSTD_FORM_GEMM_BF16: "gemm_bf16"}[f]
 
     def tuning(self):
-        """The autotuner's choice: {"lean" (flavour 0 early, 1 late, 2 mid), "xcd_order", "tile_threads",
-        "stage_ms", "trial_steps" (time steps its trials ran on this solver), "cached" (the choice came from
+        """The autotuner's choice: {"lean" (the flavour set on this solver: 0 early, 1 late, 2 mid; chooses
+        nothing), "xcd_order", "tile_threads", "stage_ms", "trial_steps" (time steps its trials ran on this solver), "cached" (the choice came from
         the per-(device, plan signature) cache, without trials)}, and what the plan's sizes chose:
         "p0_pass" (p0 formed by a pass after every stage, or by the tiles that read it), "eight_value_points"
         (longest FFT length whose lines take 8 values per thread)."""

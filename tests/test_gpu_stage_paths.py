@@ -4,15 +4,19 @@ in a batch.  Each test asserts from the context which path its solvers take.  Le
 that the other tests leave out are compared with the FP64 oracle; the tolerance of
 fields after two steps is 2e-6 rel-L2, as in test_gpu_parity.py (FP32 roundings of one
 derivative are a few 1e-7 of its largest value, twelve stages add up at random)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import openpstd_amd as P
 from openpstd_amd import abi_types as T
 from openpstd_amd import workloads as W
+from openpstd_amd._lib import lib
 from oracle import binding as ob
 
 from test_gpu_parity import THREADS, compare_fields, device
+from test_gpu_plan_checks import Domain, Plan
 
 pytestmark = pytest.mark.gpu
 FIELDS = ("p0", "px0", "py0", "vx0", "vy0")
@@ -149,3 +153,28 @@ def test_lines_of_the_matrix_form_choose_no_values_per_thread(form):
     assert dev.tuning()["eight_value_points"] == 2048 and batch.tuning()["eight_value_points"] == 512
     assert np.array_equal(batch.scene_samples(batch.advance(2), 3), dev.advance(2))
     assert_same_fields(k, dev, batch, 3)
+
+
+def test_flavour_is_the_contexts_own():
+    """A flavour chooses nothing and is reported back; one context's does not reach others
+    through the launch shapes kept per plan (a plan that is tuned here for the first
+    time: no other test has a domain of its size)."""
+    ctx = [C.c_void_p(), C.c_void_p()]
+    for c in ctx:
+        assert lib().pstd_ctx_create(0, C.byref(c)) == T.PSTD_OK
+    try:
+        dom = (Domain * 1)(Domain(nx=123, ny=71, rho=1.2))
+        seg = (T.pstd_plan_segment * 1)()
+        for name, v in dict(domain=0, line_end=71, side1=-1, side2=-1, wlen=32, table_len=256, c_main1=1.0,
+                            c_main2=1.0).items():
+            setattr(seg[0], name, v)
+        plan = Plan(n_domains=1, domains=dom, n_segments=1, segments=seg, dx=0.2, dt=1e-4, c1=340.0, patch_error=70.0)
+        assert lib().pstd_ctx_set_kernel_flavour(ctx[0], 0) == T.PSTD_OK
+        for c, want in zip(ctx, (0, 1)):
+            assert lib().pstd_ctx_upload_plan(c, C.byref(plan)) == T.PSTD_OK
+            got = C.c_int32(-1)
+            assert lib().pstd_ctx_get_tuning(c, C.byref(got), None, None) == T.PSTD_OK
+            assert got.value == want
+    finally:
+        for c in ctx:
+            lib().pstd_ctx_destroy(c)
