@@ -2420,6 +2420,10 @@ static int build_spectral_receivers(pstd_ctx *ctx, const pstd_plan_desc *plan) {
 }
 
 static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vector<int> *dom_scene = nullptr) {
+    if (plan->n_domains < 0) {
+        ctx->err = "negative number of domains";
+        return PSTD_ERR_INVALID;
+    }
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->release();
@@ -2437,7 +2441,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
     ctx->gemm_flops = 0;
     ctx->gemm_cells = 0;
     ctx->plan_domains.assign(plan->domains, plan->domains + plan->n_domains);
-    ctx->written.assign(2 * (size_t)std::max(0, plan->n_domains), 0);
+    ctx->written.assign(2 * (size_t)plan->n_domains, 0);
     ctx->any_written = false;
     // arena layout: one block per domain (vx, vy, px, py), 256 B aligned
     long long off = kLead;  // zeros before the first block
@@ -2448,8 +2452,9 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             ctx->err = "domain with empty extent";
             return PSTD_ERR_INVALID;
         }
-        const long long cells = (long long)p.nx * p.ny, block = 4 * cells + p.nx + p.ny + 4 * 64;
-        if (block > kMaxDomainFloats) {
+        // (four times the cells of the largest extents do not fit 64 bits)
+        const long long cells = (long long)p.nx * p.ny;
+        if (cells > kMaxDomainFloats / 4 || 4 * cells + p.nx + p.ny + 4 * 64 > kMaxDomainFloats) {
             ctx->err = "domain of " + std::to_string(cells) + " cells exceeds one buffer block";
             return PSTD_ERR_UNSUPPORTED;
         }
@@ -2567,7 +2572,7 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
         // neighbour bounds: lines and halo columns must exist in the neighbour
         for (int side = 0; side < 2; ++side) {
             int nb = side == 0 ? s.side1 : s.side2;
-            int o = side == 0 ? s.side1_offset : s.side2_offset;
+            const long long o = side == 0 ? s.side1_offset : s.side2_offset;  // a line + any 32-bit offset
             if (nb < 0) continue;
             const DomainDev &dn = ctx->doms[nb];
             int nlen = (s.direction == 0 ? dn.nx : dn.ny) + (s.field == 1 ? 1 : 0);
@@ -2578,13 +2583,13 @@ static int upload_impl(pstd_ctx *ctx, const pstd_plan_desc *plan, const std::vec
             }
             if (side == 0) {
                 src_addr(dn, s.direction, s.field, g.s1_a, g.s1_b, g.s1_ls, g.s1_bp);
-                g.s1_line = o;
+                g.s1_line = (int)o;
                 g.s1_len = nlen;
                 g.s1_dom = dn.base;
                 g.s1_size = dn.size;
             } else {
                 src_addr(dn, s.direction, s.field, g.s2_a, g.s2_b, g.s2_ls, g.s2_bp);
-                g.s2_line = o;
+                g.s2_line = (int)o;
                 g.s2_len = nlen;
                 g.s2_dom = dn.base;
                 g.s2_size = dn.size;
