@@ -232,7 +232,7 @@ int pstd_ctx_advance_async(pstd_ctx *ctx, int steps);
  * allocating routine: the launches are issued one by one (no graph is
  * instantiated), and the GEMM form's scratch -- the per-scene maxima that
  * choose the split scaling -- lives in a file-scope device array of
- * 3 x 2 x 1024 words per device instead of the context's buffer; more than
+ * 2 x 1024 words per device instead of the context's buffer; more than
  * 1024 scenes in a GEMM-form context is PSTD_ERR_INVALID.  Every call starts
  * that array from zero and from the maxima of the current state, so results
  * equal pstd_ctx_advance_async's from the same state (bitwise when that call
@@ -251,10 +251,11 @@ int pstd_ctx_profile_stages(pstd_ctx *ctx, int steps, double *mean_stage_ms, int
 /* Advances `steps` time steps like pstd_ctx_advance_async, issuing every
  * launch eagerly with a HIP event pair on the solver stream around each
  * launch of a kernel class, and waits.  ms[c] / launches[c] receive the summed
- * GPU time and launch count of class c: 0 the FFT-form kernel of lines up to
- * 2048 points (with the passthrough and receiver tiles), 1 the 4096-point
- * kernel, 2 the 8192-point kernel, 3 the GEMM-form kernel; ms[4] the whole
- * run, launches[4] its 6*steps RK stages.  For measurement (no counterpart in
+ * GPU time and launch count of class c: the FFT-form launch of a stage (all its
+ * lines, the passthrough and receiver tiles) counts for its longest lines, class
+ * 0 up to 2048 points, 1 4096, 2 8192 points; 3 the GEMM-form kernel; ms[4] the
+ * whole run with the launches of no class (the pass that forms p0, receivers),
+ * launches[4] its 6*steps RK stages.  For measurement (no counterpart in
  * the reference). */
 int pstd_ctx_profile_kernels(pstd_ctx *ctx, int steps, double ms[5], int launches[5]);
 /* Replays whole blocks of `steps` time steps as one captured hipGraph (0 = the
@@ -274,8 +275,8 @@ int pstd_ctx_capture_graph(pstd_ctx *ctx);
  * segments, PML strips, passthrough and receiver tiles) run on a second
  * stream of the context, concurrently with the GEMM kernel, forked after and
  * joined before the neighbouring stages.  Default 0: issued in order on one
- * stream (the GEMM kernel occupies every CU's LDS, so concurrency gains
- * nothing measurable).  Results are identical either way.  No counterpart in
+ * stream (the two kernels' wavefronts do not fit the registers of a SIMD
+ * together: overlapped stages measure 0 to 7 % longer).  Results are identical either way.  No counterpart in
  * the reference. */
 int pstd_ctx_set_stage_overlap(pstd_ctx *ctx, int on);
 /* Launch shape of the stage kernel (no counterpart in the reference, whose

@@ -10,12 +10,13 @@
 // conjugate of the forward transform of the conjugate (the same roundings), so
 // one piece of code runs twice (it is straight-line and long).
 //
-// V = 16 from F = 1024 on: a 1024-point pair fits one wavefront (no workgroup
-// barrier in its tile), the butterflies of a thread share their twiddles in the
-// passes of span <= T, and address, halo and update work is shared by twice the
-// values.  V = 8 up to 512 points: the scenes with short lines are bound by one
-// wavefront's instruction stream, which is half as long.  V changes no result:
-// which values a butterfly combines depends on F alone.  One LDS buffer per pair
+// V = 16 from F = 1024 on, in launches of many wavefronts: a 1024-point pair fits one
+// wavefront (no workgroup barrier in its tile), the butterflies of a thread share
+// their twiddles in the passes of span <= T, and address, halo and update work is
+// shared by twice the values.  V = 8 up to 512 points, and for 1024 and 2048 points in
+// launches of few wavefronts (the caller's choice): these are bound by one
+// wavefront's instruction stream, which is half as long.  V changes no result: which
+// values a butterfly combines depends on F alone.  One LDS buffer per pair
 // (17/16 F complex values): 16 wavefronts fit a CU.
 #pragma once
 

@@ -820,11 +820,11 @@ __global__ void __launch_bounds__(256) rows_kernel(const float *__restrict__ px,
 // stored column-major).
 // Measured (launch alone, D through the LDS -> D straight to registers and the
 // lines two chunks ahead): 1024^2 in BF16 53.6 -> 47.3 us, 16 scenes of 512 x 1024
-// twice in FP16 536 -> 492 us (335 GFLOP of products: 680 TFLOP/s, and 3.2 TB/s of
-// memory traffic).  Neither bounds it alone: without its MFMAs it takes three
-// quarters of the time, without its stores and t_n four fifths.  Three workgroups
-// per CU (168 registers, one chunk ahead) do the 16 scenes in 502 us and the one
-// scene, which has one workgroup per CU, in 62.
+// twice in FP16 536 -> 492 us (335 GFLOP of products: 680 TFLOP/s); 256 such sources in
+// 6.22 ms (863 TFLOP/s, and 4.6 TB/s beyond the L2).  Neither bounds it alone: without
+// its MFMAs it takes three quarters of the time, without its stores and t_n four
+// fifths.  Three workgroups per CU (168 registers, one chunk ahead) do the 16 scenes in
+// 502 us and the one scene, which has one workgroup per CU, in 62.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1346,8 +1346,9 @@ constexpr int kDefaultGraphSteps = 20;
 // fly moves this many bytes per stage more (about 5 us at 4 TB/s).  Measured, us
 // per stage on the fly / with the pass: L-shape 7.7 / 14.2, 333 000 cells 11.8 / 19.2,
 // one 900^2 domain 22.1 / 26.0, 1024^2 30.3 / 32.8, 1200^2 37.0 / 36.3, 1900^2 59.5 /
-// 55.3, 2501 x 1237 69.1 / 55.7, 4096^2 465 / 394, 16 sources of 512 x 1024 twice 344 /
-// 346; twelve scenes of lines up to 600 (at least 8 lines per tile) 93.5 / 106.
+// 55.3, 2501 x 1237 69.1 / 55.7, 4096^2 465 / 394; twelve scenes of lines up to 600 (at
+// least 8 lines per tile) 93.5 / 106.  Far above the line the two can be level: 16
+// sources of 512 x 1024 twice, 133 MB more by this count, take 344 / 346.
 constexpr long long kP0PassBytes = 20000000;
 // 64-byte sectors read per 64 bytes used by a tile's strided reads (256 threads)
 static int strided_factor(int F) {
@@ -1451,9 +1452,12 @@ struct pstd_ctx {
     hipStream_t stream = nullptr;
     // with `overlap`, GEMM-form stages run their FFT-form tiles on `side`,
     // concurrently with the GEMM kernel on `stream` (fork and join through the
-    // two events; both streams at the default priority).  Off by default: the
-    // GEMM kernel fills every CU's LDS, so the two only trade places (measured
-    // +1 % on 64 scenes, 0 on 256 sources, -4 % on one 4096^2 domain)
+    // two events; both streams at the default priority).  Off by default: two
+    // wavefronts of the GEMM kernel leave 112 of a SIMD's 512 registers, one of an
+    // FFT-form tile takes 128, so the two kernels only trade places, and the events
+    // cost.  In order / overlapped, us per stage in the FP16 form: 1024^2 60.4 / 64.6
+    // (one workgroup per CU, where both would fit), 4096^2 1566 / 1638, 16 sources of
+    // 512 x 1024 twice 532 / 536, 64 scenes 1822 / 1849
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     bool overlap = false;
@@ -1945,7 +1949,9 @@ static int upload_tiles(pstd_ctx *ctx) {
     const int nt = ctx->stage_threads();
     std::vector<TileDesc> tiles;
     // the longest tiles first, so that none of them starts last, but in the smallest
-    // scenes, whose kinds of tiles stay mixed over the CUs.  Measured mixed / sorted, us
+    // scenes, whose kinds of tiles stay mixed over the CUs.  (A batch of many lengths would
+    // gain 3 % mixed, but the wavefront count is on the side of the single scenes that gain
+    // 8 to 21 % sorted.)  Measured mixed / sorted, us
     // per stage: L-shape 8.1 / 8.2, rooms of 333, 141, 477 x 217 11.7 / 12.3 (11.0 / 11.0
     // with 8 values per thread), 1500 x 150 18.1 / 15.4, 900^2 22.1 / 19.5, 1268 x 303 20.1 /
     // 15.9, 1200^2 37.2 / 36.0, 1900^2 59.5 / 55.0, 4096^2 399 / 393, twelve scenes 91.0 / 93.6
